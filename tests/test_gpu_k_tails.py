@@ -1,0 +1,85 @@
+"""Rows of k that end inside a step of the matrix-core tile kernels (128 bytes): what their direct global-to-LDS loads
+fetch past the end are zeros, also where the memory behind a row holds NaN.  Both operand orders of the 16-bit product,
+the stream kernel, K in uneven slices, float8 operands, the int8 op's many-row form."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from _util import ODT, bits, gen, unbits
+from test_gpu_fp8mm import FLOAT8, run_case
+from test_gpu_gemm16 import close, col_major
+
+pytestmark = pytest.mark.gpu
+DTYPES = [torch.bfloat16, torch.float16]
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("variant", [0, 3, 4, 5])
+@pytest.mark.parametrize("m,k,n", [(264, 1, 136), (136, 63, 264), (264, 65, 520), (1032, 129, 264), (72, 407, 72)])
+def test_k_major_operands_any_k(dtype, variant, m, k, n):
+    """x.t() @ y over any number of rows (the weight gradient of a batch of any size)."""
+    import _dev
+    a = bits((torch.randn(m, k, generator=gen(21)) * 0.5).to(dtype))
+    b = bits((torch.randn(k, n, generator=gen(22)) * 0.5).to(dtype))
+    want, mag = oracle.gemm16(a, b, ODT[dtype], want_mag=True)
+    close(_dev.gemm16(col_major(a), b, ODT[dtype], variant=variant), want, mag, dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("variant", [0, 3, 4, 5, 6])
+@pytest.mark.parametrize("k", [72, 120, 136, 200, 1032])
+def test_rows_of_k_in_wider_rows(dtype, variant, k):
+    """One operand or both in rows of k whose memory goes on with NaN."""
+    import _dev
+    m, n = 300, 520
+    a = bits((torch.randn(m, k, generator=gen(23)) * 0.5).to(dtype))
+    w = bits((torch.randn(n, k, generator=gen(24)) * 0.5).to(dtype))
+    want, mag = oracle.gemm16(a, w.T, ODT[dtype], want_mag=True)
+    wide = lambda x: np.concatenate([x, np.full((x.shape[0], 64), 0x7FC1 if dtype == torch.bfloat16 else 0x7E01, np.uint16)], 1)[:, :k]  # noqa: E731
+    close(_dev.gemm16(wide(a), wide(w).T, ODT[dtype], variant=variant), want, mag, dtype)
+    if variant != 6:
+        close(_dev.gemm16(wide(a), np.ascontiguousarray(w.T), ODT[dtype], variant=variant), want, mag, dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+def test_stream_kernel_is_the_tile_kernel(dtype):
+    """More tiles than workgroups, k of two steps and a bit: streams that cross tiles at a partial step; same bits."""
+    import _dev
+    a = bits((torch.randn(4352, 136, generator=gen(25)) * 0.5).to(dtype))
+    w = bits((torch.randn(4360, 136, generator=gen(26)) * 0.5).to(dtype))
+    assert np.array_equal(_dev.gemm16(a, w.T, ODT[dtype], variant=6), _dev.gemm16(a, w.T, ODT[dtype], variant=3))
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+@pytest.mark.parametrize("k,variant", [(1096, 10 | 3 << 8), (1000, 10 | 16 << 8), (3592, 0)])
+def test_uneven_slices(dtype, layout, k, variant):
+    import _dev
+    m, n = 200, 264
+    a = bits((torch.randn(m, k, generator=gen(27)) * 0.5).to(dtype))
+    w = bits((torch.randn(n, k, generator=gen(28)) * 0.5).to(dtype))
+    want, mag = oracle.gemm16(a, w.T, ODT[dtype], want_mag=True)
+    close(_dev.gemm16(a, w.T if layout == "nt" else np.ascontiguousarray(w.T), ODT[dtype], variant=variant), want, mag, dtype)
+
+
+@pytest.mark.parametrize("k", [144, 176, 1040, 2112])
+@pytest.mark.parametrize("variant,out", [(0, torch.bfloat16), (8, torch.bfloat16), (5, torch.float8_e4m3fn), (11, torch.bfloat16),
+                                         (11, torch.float8_e5m2), (6, torch.float32), (9, torch.float16), (14 | 3 << 8, torch.bfloat16)])
+def test_float8(k, variant, out):
+    if variant >> 8 and k < 1024:
+        pytest.skip("shorter than three slices of 128 bytes")
+    run_case(300, k, 264, FLOAT8[0], FLOAT8[1], out, True, torch.float32, None if out.itemsize > 1 else 2.0, variant=variant, seed=k)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("m,k,n", [(1500, 208, 6000), (400, 80, 8264)])
+def test_int8_many_rows(dtype, m, k, n):
+    import _dev
+    a = torch.randn(m, k, generator=gen(29)).to(dtype)
+    b = torch.randint(-128, 128, (n, k), dtype=torch.int8, generator=gen(30))
+    s = (torch.rand(n, generator=gen(31)) * 0.02).to(dtype)
+    got = unbits(_dev.qmm8(bits(a), ODT[dtype], b.numpy(), bits(s)), dtype).double().numpy()
+    _, c64, mag = oracle.qmm8(bits(a), ODT[dtype], b.numpy(), bits(s), want_f64=True)
+    # eps * |want| + 2^-20 * mag; below 2^-14, float16's smallest normal number, its values lie eps * 2^-14 apart
+    assert (np.abs(got - c64) <= torch.finfo(dtype).eps * np.maximum(np.abs(c64), 2.0**-14) + 2.0**-20 * mag).all()

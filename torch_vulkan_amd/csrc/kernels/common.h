@@ -42,6 +42,15 @@ __device__ __forceinline__ void stg_stream(uint64_t addr, X v) {
   __builtin_nontemporal_store(v, reinterpret_cast<VKT_GLOBAL X*>(addr));
 }
 
+// One LDS-direct load of 16 bytes per lane: global address `base` + `offset` + OFF, LDS address `lds_at` + OFF + 16 * lane.
+// (M0 is written in every statement that uses it and by nothing else in the kernels that use it: no other instruction the compiler
+// emits here reads it, and a clobber of a reserved register is not something the compiler honours anyway.)
+template <int OFF>
+__device__ __forceinline__ void load_to_lds(uint32_t offset, uint64_t base, uint32_t lds_at) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3" ::"v"(offset), "s"(base), "s"(lds_at), "i"(OFF)
+               : "memory");
+}
+
 __device__ __forceinline__ float bits_f32(uint32_t u) { return __builtin_bit_cast(float, u); }
 inline float bits_f32_host(uint32_t u) { return __builtin_bit_cast(float, u); }
 __device__ __forceinline__ uint32_t f32_bits(float f) { return __builtin_bit_cast(uint32_t, f); }

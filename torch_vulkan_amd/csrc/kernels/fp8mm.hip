@@ -71,6 +71,7 @@ __device__ __forceinline__ float output_inv(const F8Params& p) {
 // the bias, the output scale and the cast.
 struct F8Problem : F8Params {
   static constexpr bool kTransA = false, kTransB = false;  // float8 operands are rows of k
+  static constexpr bool kSliced = false;
   uint32_t batches = 1;
   uint64_t a_batch = 0, b_batch = 0;
   struct Whole {
@@ -332,8 +333,8 @@ template <int FA, int FB>
 int launch_sliced(const F8Params& p0, uint32_t slices, const Machine& mc, hipStream_t stream, std::string* err) {
   F8Problem p;
   static_cast<F8Params&>(p) = p0;
-  if (slices < 2 || p0.k % (BK * slices) || uint64_t(slices) * p0.m * p0.n * 4 > mc.workspace_bytes) {
-    *err = "fp8mm: " + std::to_string(slices) + " slices of K do not divide its steps of 128 bytes, or their partial sums do not fit the workspace";
+  if (slices < 2 || slices > (p0.k + BK - 1) / BK || uint64_t(slices) * p0.m * p0.n * 4 > mc.workspace_bytes) {
+    *err = "fp8mm: " + std::to_string(slices) + " slices of K are fewer than 2 or more than its steps of 128 bytes, or their partial sums do not fit the workspace";
     return -1;
   }
   if (p0.out_dtype == VKT_F32 || p0.out_dtype == VKT_F16) return launch_tile_slices<FA, FB, true, kMathFp8Wide>(p, slices, mc, stream, err, "fp8mm");
@@ -364,8 +365,7 @@ int launch_formats(const F8Params& p, uint32_t variant, const Machine& mc, hipSt
   // variant 0: planned.  Explicit variants run the MFMA kernel whatever the output dtype
   // (tests, tuning): 1: 128x128 tiles (4 waves of 64x64, 16x16x128 MFMA); 2: 256x256 (4 waves of
   // 128x128, 16x16x128); 3: 256x128; 4: 256x256 with the 32x32x64 MFMA (measured ~10 % faster
-  // than 16x16x128 at equal work); 5: as 4 with global-to-LDS direct loads when k is a
-  // multiple of 128 (else 4); 8: as 5 with 8 waves of 64x128 instead of 4 of 128x128 (two waves per SIMD cover each
+  // than 16x16x128 at equal work); 5: as 4 with global-to-LDS direct loads; 8: as 5 with 8 waves of 64x128 instead of 4 of 128x128 (two waves per SIMD cover each
   // other's waits: 8192^3 2.34-2.42 -> 2.56-2.59 PFLOP/s; what they get where the stream kernel does not serve).  11: the stream kernel of
   // mma_stream.h where it serves the problem (large bfloat16 and float8 outputs get it), else 8.  255: the one-thread-per-output kernel.
   // 6 / 7: the exact path (float8 widened to bfloat16 in registers, 32x32x16 bfloat16 MFMA) on
@@ -422,28 +422,20 @@ int launch_formats(const F8Params& p, uint32_t variant, const Machine& mc, hipSt
     variant = (p.out_dtype == VKT_F32 || p.out_dtype == VKT_F16) ? (big && tiles256 >= cus ? 6 : 7) : (big && 4 * tiles256 > cus ? 11 : 1);
   if ((variant & 0xff) == 14) return launch_sliced<FA, FB>(p, (variant >> 8) & 31u, mc, stream, err);
   switch (variant) {
-    case 6:
-      if (p.k % BK == 0) return launch_tile<2, 2, 8, 8, FA, FB, true, true, true>(p, compute_units, stream, err);
-      return launch_tile<2, 2, 8, 4, FA, FB, true, false, true>(p, compute_units, stream, err);  // (256x256 without the direct loads runs out of registers)
+    case 6: return launch_tile<2, 2, 8, 8, FA, FB, true, true, true>(p, compute_units, stream, err);
     case 7: return launch_tile<2, 2, 4, 4, FA, FB, true, false, true>(p, compute_units, stream, err);
     case 1: return launch_tile<2, 2, 4, 4, FA, FB>(p, compute_units, stream, err);
     case 2: return launch_tile<2, 2, 8, 8, FA, FB>(p, compute_units, stream, err);
     case 3: return launch_tile<2, 2, 8, 4, FA, FB>(p, compute_units, stream, err);
     case 4: return launch_tile<2, 2, 8, 8, FA, FB, true>(p, compute_units, stream, err);
-    case 9:  // as 6 with 8 waves of 64x128
-      if (p.k % BK == 0) return launch_tile<4, 2, 4, 8, FA, FB, true, true, true>(p, compute_units, stream, err);
-      return launch_tile<2, 2, 8, 4, FA, FB, true, false, true>(p, compute_units, stream, err);
+    case 9: return launch_tile<4, 2, 4, 8, FA, FB, true, true, true>(p, compute_units, stream, err);  // as 6 with 8 waves of 64x128
     case 11: {  // the stream kernel (mma_stream.h), else 8
       const int rc = launch_stream<FA, FB>(p, compute_units, stream, err);
       if (rc != -2) return rc;
     }
       [[fallthrough]];
-    case 8:  // 256x256 tiles over 8 waves of 64x128 (two waves per SIMD), direct loads
-      if (p.k % BK == 0) return launch_tile<4, 2, 4, 8, FA, FB, true, true>(p, compute_units, stream, err);
-      return launch_tile<2, 2, 8, 8, FA, FB, true>(p, compute_units, stream, err);
-    case 5:
-      if (p.k % BK == 0) return launch_tile<2, 2, 8, 8, FA, FB, true, true>(p, compute_units, stream, err);
-      return launch_tile<2, 2, 8, 8, FA, FB, true>(p, compute_units, stream, err);
+    case 8: return launch_tile<4, 2, 4, 8, FA, FB, true, true>(p, compute_units, stream, err);  // 256x256 tiles over 8 waves of 64x128 (two waves per SIMD), direct loads
+    case 5: return launch_tile<2, 2, 8, 8, FA, FB, true, true>(p, compute_units, stream, err);
   }
   *err = "fp8mm: unknown variant " + std::to_string(variant);
   return -1;

@@ -8,8 +8,10 @@
 //     tiles, direct global-to-LDS loads, persistent grid) with V_MFMA_F32_32X32X16_{BF16,F16}
 //     and an alpha / beta epilogue.  A contiguous along k and B along k (x @ W.t(), the Linear
 //     layout) takes k a multiple of 8; an operand contiguous along m or n (x @ W, x.t() @ y:
-//     what backward passes produce) is read through the transposing LDS load and takes k a
-//     multiple of 64 and m (n) of 8;
+//     what backward passes produce) is read through the transposing LDS load and takes m (n) a
+//     multiple of 8, and both of them (x.t() @ y over any number of rows) every k: the lanes of
+//     the last step's loads that lie past k fetch zeros (1610 rows into 3648 x 6400: 0.10 ms;
+//     17 ms on the strided kernel, which such a k went to before);
 //   - everything else (strided views, odd sizes): one thread per output over the strides as
 //     given.  Correct for any strides, and slow.
 #include "kernels.h"
@@ -26,7 +28,7 @@ __device__ __forceinline__ float slot_float(uint64_t slot) { return bits_f32(uin
 template <class T, bool TRA = false, bool TRB = false>
 struct GemmProblem {
   static constexpr bool kTransA = TRA, kTransB = TRB;
-  static constexpr bool kRegisterEpilogue = false;
+  static constexpr bool kRegisterEpilogue = false, kSliced = false;
   // operands as the tile kernel takes them (bytes)
   uint64_t a, b;
   uint32_t m, n, k, lda, ldb, batches;
@@ -255,8 +257,8 @@ int launch_tiles(const GemmParams& p, uint32_t use_cin, uint32_t batch, uint32_t
       const bool asked = (variant & 0xff) == 10;
       const uint64_t budget = mc.workspace_bytes < VKT_STATIC_SCRATCH_BYTES ? mc.workspace_bytes : VKT_STATIC_SCRATCH_BYTES;
       const uint32_t slices = asked ? (variant >> 8) & 31u : (p.m > 64 ? tile_slices(p.m, p.n, g.k, uint32_t(mc.compute_units), budget) : 1);
-      if (asked && (slices < 2 || g.k % (BK * slices) || uint64_t(slices) * p.m * p.n * 4 > mc.workspace_bytes)) {
-        *err = "gemmcm: " + std::to_string(slices) + " slices of K do not divide its steps of 64 values, or their partial sums do not fit the workspace";
+      if (asked && (slices < 2 || slices > (g.k + BK - 1) / BK || uint64_t(slices) * p.m * p.n * 4 > mc.workspace_bytes)) {
+        *err = "gemmcm: " + std::to_string(slices) + " slices of K are fewer than 2 or more than its steps of 64 values, or their partial sums do not fit the workspace";
         return -1;
       }
       if (asked || (slices >= 2 && uint64_t((p.m + 127) / 128) * ((p.n + 127) / 128) * 2 <= uint64_t(mc.compute_units)))
@@ -295,10 +297,9 @@ int launch_tiles(const GemmParams& p, uint32_t use_cin, uint32_t batch, uint32_t
       }
     }
   }
-  const bool direct_ok = g.k % BK == 0;
   // variant 0: planned; 1: 128x128 tiles; 2: 256x128; 3: 256x256 with direct loads; 4: 128x128 with direct loads;
   // 5: 256x256 with direct loads over 8 waves; 6: the stream kernel (mma_stream.h; else 3)
-  // (direct loads: k a multiple of 64; k-major operands run on the direct forms only)
+  // (k-major operands run on the direct forms only)
   if (variant == 0) {
     // 256 x 256 tiles where they give every compute unit one, else 128 x 128
     // (from five eighths of a tile per unit on: 1024 x 4096 x 14336 is 224 tiles on 256 units, 121 us on the stream
@@ -306,23 +307,23 @@ int launch_tiles(const GemmParams& p, uint32_t use_cin, uint32_t batch, uint32_t
     const bool large = uint64_t((p.m + 255) / 256) * ((p.n + 255) / 256) * batch * 8 >= uint64_t(mc.compute_units) * 5;
     // (both operands k-major: 8 waves, whose transposing LDS reads cover each other: 8192^3 0.94 -> 1.11-1.13 PFLOP/s;
     //  with k-contiguous operands the 8-wave form reads 1.5x the LDS bytes and is 3-5 % slower)
-    variant = large ? (direct_ok ? (TRA && TRB ? 5 : 3) : 2) : (TRA || TRB ? 4 : 1);
+    variant = large ? (TRA && TRB ? 5 : 3) : (TRA || TRB ? 4 : 1);
     // both operands contiguous along k (x @ w.T): the stream kernel where it serves (8192^3: 0.94-1.00 -> 0.89 ms)
     if (!TRA && !TRB && variant == 3) variant = 6;
   }
-  const bool stream_ok = direct_ok && g.k >= 2 * BK && p.n % 8 == 0 && p.c_sm % 8 == 0 && p.c_sb % 8 == 0 && p.c % 16 == 0 &&
+  const bool stream_ok = g.k > BK && p.n % 8 == 0 && p.c_sm % 8 == 0 && p.c_sb % 8 == 0 && p.c % 16 == 0 &&
                          mma_stream_strides_ok(g.lda, g.ldb);
   if (variant == 6 && !stream_ok) variant = 3;
   if constexpr (!TRA && !TRB) {
-    // 6: the stream kernel (mma_stream.h) where it serves the problem: k a multiple of 64 values and at least 128, n a multiple of 8, C in 16-byte aligned rows
+    // 6: the stream kernel (mma_stream.h) where it serves the problem: more than 64 values of k, n a multiple of 8, C in 16-byte aligned rows
     if (variant == 6) return launch_mma_stream<0, 0, MATH>(g, mc.compute_units, stream, err, "gemmcm");
     if (variant == 1) return launch_mma_tile<2, 2, 4, 4, 0, 0, true, false, MATH>(g, mc.compute_units, stream, err, "gemmcm");
     if (variant == 2) return launch_mma_tile<2, 2, 8, 4, 0, 0, true, false, MATH>(g, mc.compute_units, stream, err, "gemmcm");
   }
-  if (variant == 3 && direct_ok) return launch_mma_tile<2, 2, 8, 8, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "gemmcm");
-  if (variant == 4 && direct_ok) return launch_mma_tile<2, 2, 4, 4, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "gemmcm");
+  if (variant == 3) return launch_mma_tile<2, 2, 8, 8, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "gemmcm");
+  if (variant == 4) return launch_mma_tile<2, 2, 4, 4, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "gemmcm");
   // 5: 256x256 over 8 waves of 64x128 (two waves per SIMD), direct loads
-  if (variant == 5 && direct_ok) return launch_mma_tile<4, 2, 4, 8, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "gemmcm");
+  if (variant == 5) return launch_mma_tile<4, 2, 4, 8, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "gemmcm");
   *err = "gemmcm: unknown variant " + std::to_string(variant) + " for this k and layout";
   return -1;
 }
@@ -338,7 +339,7 @@ int launch_gemm16_t(const GemmParams& p, uint32_t use_cin, uint32_t batch, uint3
   const bool a_k = rows_ok(p.a_sk, p.a_sm, p.a_sb, p.a, p.k), b_k = rows_ok(p.b_sk, p.b_sn, p.b_sb, p.b, p.k);
   const bool a_m = !a_k && p.m % 8 == 0 && rows_ok(p.a_sm, p.a_sk, p.a_sb, p.a, p.m);
   const bool b_n = !b_k && p.n % 8 == 0 && rows_ok(p.b_sn, p.b_sk, p.b_sb, p.b, p.n);
-  const bool k_ok = p.k != 0 && (a_m || b_n ? p.k % 64 == 0 : p.k % 8 == 0);
+  const bool k_ok = p.k != 0 && (a_k || b_k ? p.k % 8 == 0 : true);  // (rows of k end on 16 bytes; k-major operands: any number of rows)
   const bool tiles_ok = (a_k || a_m) && (b_k || b_n) && k_ok && p.c_sn == 1 && p.c_sm > 0 && p.c_sb >= 0 && variant != 255;
   if (!tiles_ok) {
     if ((p.m + 3) / 4 > 65535 || batch > 65535) {
@@ -362,7 +363,7 @@ int launch_gemm16_t(const GemmParams& p, uint32_t use_cin, uint32_t batch, uint3
 template <class T>
 struct Q8GemmProblem {
   static constexpr bool kTransA = false, kTransB = false;
-  static constexpr bool kRegisterEpilogue = false;
+  static constexpr bool kRegisterEpilogue = false, kSliced = false;
   uint64_t a, b;
   uint32_t m, n, k, lda, ldb, batches;
   uint64_t a_batch, b_batch;
@@ -461,14 +462,10 @@ int launch_q8_gemm_t(const Q8Params& p, const Machine& mc, hipStream_t stream, s
   g.a = p.a, g.b = mc.scratch, g.m = p.m, g.n = p.n, g.k = p.k * 2, g.lda = uint32_t(p.a_sm) * 2, g.ldb = p.k * 2;
   g.batches = 1, g.a_batch = 0, g.b_batch = 0, g.c = p.c, g.scales = p.scales;
   const bool large = uint64_t((p.m + 255) / 256) * ((p.n + 255) / 256) * 8 >= uint64_t(mc.compute_units) * 5;  // (as for the 16-bit product)
-  if (g.k % BK == 0) {
-    if (large && g.k >= 2 * BK && p.n % 8 == 0 && p.c % 16 == 0 && p.scales % 16 == 0 && mma_stream_strides_ok(g.lda, g.ldb))
-      return launch_mma_stream<0, 0, MATH>(g, mc.compute_units, stream, err, "qmm8");
-    if (large) return launch_mma_tile<2, 2, 8, 8, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "qmm8");
-    return launch_mma_tile<2, 2, 4, 4, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "qmm8");
-  }
-  if (large) return launch_mma_tile<2, 2, 8, 4, 0, 0, true, false, MATH>(g, mc.compute_units, stream, err, "qmm8");
-  return launch_mma_tile<2, 2, 4, 4, 0, 0, true, false, MATH>(g, mc.compute_units, stream, err, "qmm8");
+  if (large && g.k > BK && p.n % 8 == 0 && p.c % 16 == 0 && p.scales % 16 == 0 && mma_stream_strides_ok(g.lda, g.ldb))
+    return launch_mma_stream<0, 0, MATH>(g, mc.compute_units, stream, err, "qmm8");
+  if (large) return launch_mma_tile<2, 2, 8, 8, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "qmm8");
+  return launch_mma_tile<2, 2, 4, 4, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "qmm8");
 }
 
 }  // namespace

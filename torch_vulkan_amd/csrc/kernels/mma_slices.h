@@ -5,13 +5,14 @@
 // The tile kernel already runs batches of products; slice s of K is batch s of a product whose operands begin
 // s * (k / slices) bytes into their rows (both operands are rows of k) and whose "outputs" are float32 partial sums in
 // the workspace, [slice][m][n]: SliceProblem is that product (weights stored [k, n]: a slice begins k / slices rows
-// down).  A second launch adds the slices up in slice order (the result does not depend on timing) and runs the real
+// down; the last slice ends where k does).  A second launch adds the slices up in slice order (the result does not depend on timing) and runs the real
 // problem's epilogue on 4 consecutive columns of a row, the unit every problem's store<DT>() takes.
 #pragma once
 #include <string>
 #include <type_traits>
 
 #include "kernels.h"
+#include "limits.h"
 #include "mma_tile.h"
 
 namespace vkt {
@@ -20,9 +21,11 @@ namespace {
 template <bool TRB>
 struct SliceProblem {
   static constexpr bool kTransA = false, kTransB = TRB;  // (TRB: the second operand stored [k, n], 16-bit values)
-  static constexpr bool kRegisterEpilogue = false;
+  static constexpr bool kRegisterEpilogue = false, kSliced = true;
   uint64_t a, b;
-  uint32_t m, n, k, lda, ldb, batches;  // (k: bytes of one slice; batches: the slices)
+  uint32_t m, n, k, lda, ldb, batches;  // (k: bytes of one slice, a multiple of the step; batches: the slices)
+  uint32_t k_all;
+  __device__ __forceinline__ uint32_t k_of(uint32_t slice) const { return k_all - slice * k < k ? k_all - slice * k : k; }
   uint64_t a_batch, b_batch;            // (a slice's offset: k bytes into the rows; for [k, n] weights k / 2 rows)
   uint64_t partial;                     // float32 [batches][m][n]
   struct Whole {
@@ -80,16 +83,17 @@ __global__ __launch_bounds__(256) void mma_slices_finish(Problem p, uint32_t sli
   p.for_output_type(col + 3 < p.n, whole, [&](auto dt) { p.template store<decltype(dt)::value>(0, row, col, sum, cs, whole); });
 }
 
-// How many slices of K serve a product of m rows whose operands are rows of k bytes: a power of two that divides the
-// steps of 128 bytes, leaves a slice 1024 bytes and more, brings the 128 x 128 tiles up to two workgroups per compute
-// unit at most, and whose partial sums fit `budget` bytes.  1: the product is not split.
+// How many slices of K serve a product of m rows whose operands are rows of k bytes: a power of two that
+// leaves a slice 1024 bytes and more, brings the 128 x 128 tiles up to two workgroups per compute
+// unit at most, and whose partial sums fit `budget` bytes.  1: the product is not split.  (The slices need not divide
+// the steps: fp8, 111 x 4672 x 11904 and its way back 114 -> 70 us for the two, which went unsplit, or to the few-row
+// kernels, while they had to.)
 inline uint32_t tile_slices(uint32_t m, uint32_t n, uint32_t k_bytes, uint32_t cus, uint64_t budget) {
-  if (k_bytes % BK) return 1;
-  const uint32_t steps = k_bytes / BK;
+  const uint32_t steps = (k_bytes + BK - 1) / BK;
   const uint64_t tiles = uint64_t((m + 127) / 128) * ((n + 127) / 128);
   uint32_t s = 1;
-  while (s < 16 && steps % (2 * s) == 0 && steps / (2 * s) >= 8 && tiles * (2 * s) <= 2ull * cus && uint64_t(2 * s) * m * n * 4 <= budget) s *= 2;
-  return s;
+  while (s < 16 && steps / (2 * s) >= 8 && tiles * (2 * s) <= 2ull * cus && uint64_t(2 * s) * m * n * 4 <= budget) s *= 2;
+  return k_slices(steps, s).slices;  // (no empty slice)
 }
 
 // Launches the 128 x 128 tile kernel of the given arithmetic over `slices` slices of K and the second launch.
@@ -99,7 +103,9 @@ int launch_tile_slices(const Problem& p, uint32_t slices, const Machine& mc, hip
   constexpr bool TRB = Problem::kTransB;  // (k-major operands run on the tile kernel's direct-load form)
   static_assert(!Problem::kTransA, "slices of K: the first operand in rows of k");
   SliceProblem<TRB> sp;
-  sp.a = p.a, sp.b = p.b, sp.m = p.m, sp.n = p.n, sp.k = p.k / slices, sp.lda = p.lda, sp.ldb = p.ldb, sp.batches = slices;
+  const KSlices cut = k_slices((p.k + BK - 1) / BK, slices);
+  slices = cut.slices;
+  sp.a = p.a, sp.b = p.b, sp.m = p.m, sp.n = p.n, sp.k = cut.chunks_per_slice * BK, sp.k_all = p.k, sp.lda = p.lda, sp.ldb = p.ldb, sp.batches = slices;
   sp.a_batch = sp.k, sp.b_batch = TRB ? uint64_t(sp.k / 2) * p.ldb : uint64_t(sp.k), sp.partial = mc.workspace;
   const int rc = launch_mma_tile<2, 2, 4, 4, FA, FB, MF32, TRB, MATH>(sp, mc.compute_units, stream, err, name);
   if (rc != 0) return rc;

@@ -32,7 +32,7 @@
 //   pack4(values[4], whole, out[2])                    converted: two words of 16-bit outputs, or one of 8-bit
 //   narrow(whole)                                      whether outputs are 8-bit
 //   store8(batch, m, n, U4) / store8_narrow(batch, m, n, U2)     8 consecutive outputs of a row
-// k a multiple of 128 bytes and at least 256, n a multiple of 8, 16-byte aligned operand rows.
+// k more than 128 bytes and a multiple of 16 (TAIL: not of 128), n a multiple of 8, 16-byte aligned operand rows.
 #pragma once
 
 #include "limits.h"
@@ -41,16 +41,13 @@
 namespace vkt {
 namespace {
 
-// One LDS-direct load of 16 bytes per lane: global address `base` + `offset` + OFF, LDS address `lds_at` + OFF + 16 * lane.
-// (M0 is written in every statement that uses it and by nothing else in this kernel: no other instruction the compiler
-// emits here reads it, and a clobber of a reserved register is not something the compiler honours anyway.)
+// load_to_lds (common.h) with a 64-bit address per lane.
 template <int OFF>
-__device__ __forceinline__ void load_to_lds(uint32_t offset, uint64_t base, uint32_t lds_at) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3" ::"v"(offset), "s"(base), "s"(lds_at), "i"(OFF)
-               : "memory");
+__device__ __forceinline__ void load_to_lds_at(uint64_t address, uint32_t lds_at) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off offset:%2" ::"v"(address), "s"(lds_at), "i"(OFF) : "memory");
 }
 
-template <int FA, int FB, int MATH, class P>
+template <int FA, int FB, int MATH, bool TAIL, class P>
 __global__ __launch_bounds__(512) void mma_stream(P p, uint32_t tiles_m, uint32_t tiles_n) {
   static_assert(!P::kTransA && !P::kTransB, "operands contiguous along k");
   constexpr int WM = 4;  // waves along m: 8 waves of 64 x 128
@@ -64,7 +61,7 @@ __global__ __launch_bounds__(512) void mma_stream(P p, uint32_t tiles_m, uint32_
 
   const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t wm = wave >> 1, wn = wave & 1u, l32 = lane & 31u, h = lane >> 5;
-  const uint32_t steps = p.k / BK;
+  const uint32_t steps = (p.k + BK - 1) / BK;
 
   // this workgroup's tiles: slot first, first + stride, ... of its XCD's band (the order of mma_tile)
   const uint32_t per_batch = tiles_m * tiles_n, total = per_batch * p.batches, per = (total + 7) / 8;
@@ -113,6 +110,23 @@ __global__ __launch_bounds__(512) void mma_stream(P p, uint32_t tiles_m, uint32_
     const uint64_t base = (second ? load_b : load_a) + uint64_t(load_s) * BK;
     const uint32_t at = lds0 + stage * STAGE + (second ? B_AT : 0u) + wave * (ROWS * BK) + uint32_t(i >> 2) * 4096;
     const uint32_t offset = second ? off_b[i < PER ? i : 0] : off_a[i < PER ? i : 0];
+    if constexpr (TAIL) {
+      // the last step of a tile: lanes whose chunk lies past k fetch zeros instead (kZeroChunk)
+      if (load_s + 1 == steps) {
+        uint32_t ln;
+        asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
+        const uint32_t c = (ln & 7u) ^ ((4 * i + (ln >> 4)) & 7u);  // (rows 32 wave + 8 i + ln / 8)
+        uint64_t address = base + offset;
+        if (load_s * BK + c * 16 >= p.k) address = reinterpret_cast<uint64_t>(&kZeroChunk[0]) - 1024 * (i & 3);
+        switch (i & 3) {
+          case 0: load_to_lds_at<0>(address, at); break;
+          case 1: load_to_lds_at<1024>(address, at); break;
+          case 2: load_to_lds_at<2048>(address, at); break;
+          default: load_to_lds_at<3072>(address, at); break;
+        }
+        return;
+      }
+    }
     switch (i & 3) {
       case 0: load_to_lds<0>(offset, base, at); break;
       case 1: load_to_lds<1024>(offset, base, at); break;
@@ -345,13 +359,13 @@ __global__ __launch_bounds__(512) void mma_stream(P p, uint32_t tiles_m, uint32_
 // Whether mma_stream serves problem p (the caller has checked the operands' alignment).
 template <class P>
 bool mma_stream_serves(const P& p) {
-  return p.k % BK == 0 && p.k >= 2 * BK && p.n % 8 == 0 && p.n >= 8 && p.m >= 1 && mma_stream_strides_ok(p.lda, p.ldb);
+  return p.k % 16 == 0 && p.k > BK && p.n % 8 == 0 && p.n >= 8 && p.m >= 1 && mma_stream_strides_ok(p.lda, p.ldb);
 }
 
-template <int FA, int FB, int MATH, class P>
-int launch_mma_stream(const P& p, int compute_units, hipStream_t stream, std::string* err, const char* who) {
+template <int FA, int FB, int MATH, bool TAIL, class P>
+int launch_mma_stream_one(const P& p, int compute_units, hipStream_t stream, std::string* err, const char* who) {
   constexpr uint32_t lds_bytes = 2 * (256 + 256) * BK;
-  auto kernel = mma_stream<FA, FB, MATH, P>;
+  auto kernel = mma_stream<FA, FB, MATH, TAIL, P>;
   static bool configured = false;  // guarded by the runtime's stream mutex
   if (!configured) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess) {
@@ -363,7 +377,7 @@ int launch_mma_stream(const P& p, int compute_units, hipStream_t stream, std::st
   }
   const uint32_t tiles_m = (p.m + 255) / 256, tiles_n = (p.n + 255) / 256;
   const uint64_t total = uint64_t(tiles_m) * tiles_n * p.batches;
-  if (total * (p.k / BK) >= (1ull << 31)) {
+  if (total * ((p.k + BK - 1) / BK) >= (1ull << 31)) {
     *err = std::string(who) + ": too many tiles";
     return -1;
   }
@@ -371,6 +385,12 @@ int launch_mma_stream(const P& p, int compute_units, hipStream_t stream, std::st
   const uint64_t grid = (total + 7) / 8 * 8 < resident ? (total + 7) / 8 * 8 : resident;
   hipLaunchKernelGGL(kernel, dim3(uint32_t(grid)), dim3(512), lds_bytes, stream, p, tiles_m, tiles_n);
   return 0;
+}
+
+template <int FA, int FB, int MATH, class P>
+int launch_mma_stream(const P& p, int compute_units, hipStream_t stream, std::string* err, const char* who) {
+  return p.k % BK == 0 ? launch_mma_stream_one<FA, FB, MATH, false>(p, compute_units, stream, err, who)
+                       : launch_mma_stream_one<FA, FB, MATH, true>(p, compute_units, stream, err, who);
 }
 
 }  // namespace

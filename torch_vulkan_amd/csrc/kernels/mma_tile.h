@@ -14,7 +14,8 @@
 //     row_scale(m, whole), column_terms(n, whole, scale[4], bias[4])   what an output needs: acc * row_scale * scale[c] + bias[c]
 //   kTransA, kTransB                     16-bit operands only: the operand is stored k-major, i.e.
 //                                        as [k, m] (or [k, n]) rows lda (ldb) bytes apart, contiguous
-//                                        along m (n); m (n) a multiple of 8, k of 64 values
+//                                        along m (n); m (n) a multiple of 8, k any number where both are
+//   kSliced                              batch b's k is p.k_of(b) bytes instead of p.k (slices of K over batches)
 // A k-major operand keeps its global layout in LDS ([64 k][BM or BN values], 16-byte chunks
 // swizzled by the row's low bits) and the matrix-core fragments come out of it through the
 // transposing LDS read (ds_read_b64_tr_b16: 16 lanes read a 4 (k) x 16 block of 2-byte
@@ -37,6 +38,10 @@ using V4I = int __attribute__((ext_vector_type(4)));
 using V4F = float __attribute__((ext_vector_type(4)));
 
 constexpr int BK = 128;  // bytes (= fp8 values) of K per step, one MFMA deep
+
+// What the lanes of an LDS-direct load fetch whose 16 bytes lie past the end of k: an LDS-direct load writes what it
+// fetched, so there is no register to put a zero into on the way.
+__device__ const __attribute__((aligned(16))) uint32_t kZeroChunk[4] = {0, 0, 0, 0};
 
 template <int FA, int FB>
 __device__ __forceinline__ V4F mfma_f8(const V8I& first, const V8I& second, const V4F& acc) {
@@ -118,6 +123,8 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
   const uint32_t wb = (blockIdx.x & 7u) * per + slot;
   if (wb >= total) break;  // whole workgroups only, and between barriers
   const uint32_t batch = wb / per_batch, w = wb % per_batch;
+  uint32_t k_bytes = p.k;
+  if constexpr (P::kSliced) k_bytes = p.k_of(batch);
   const uint64_t a_base = p.a + uint64_t(batch) * p.a_batch, b_base = p.b + uint64_t(batch) * p.b_batch;
   constexpr uint32_t PANEL = 8;
   const uint32_t panel = w / (PANEL * tiles_n), in_panel = w % (PANEL * tiles_n);
@@ -195,7 +202,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
   constexpr int NSIDE = DIRECT ? NC : 2 * NC, NMFMA = MF32 ? TM * TN / 2 : TM * TN;  // side operations / MFMAs per step
   V4I reg[NC];
   const V4I zero = {0, 0, 0, 0};
-  const uint32_t steps = (p.k + BK - 1) / BK;
+  const uint32_t steps = (k_bytes + BK - 1) / BK;
   // chunk c: A chunks first, then B chunks
   // A full step's chunk is loaded as is: nothing may touch the register until the LDS write,
   // or the wave would wait for the load where it was issued.  Only the last step of a k that
@@ -207,11 +214,11 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
   auto load_chunk_tail = [&](int c, uint32_t k0) {
     const uint64_t src = c < A_CHUNKS ? a_src[c < A_CHUNKS ? c : 0] : b_src[c < A_CHUNKS ? 0 : c - A_CHUNKS];
     const uint32_t kc = c < A_CHUNKS ? a_k[c < A_CHUNKS ? c : 0] : b_k[c < A_CHUNKS ? 0 : c - A_CHUNKS];
-    const bool inside = k0 + kc < p.k;
+    const bool inside = k0 + kc < k_bytes;
     const V4I v = ldg<V4I>(src + (inside ? k0 : 0));  // (k >= 16: chunk 0 of the row exists)
     reg[c] = inside ? v : zero;
   };
-  const uint32_t full_steps = p.k / BK;  // steps whose 128 bytes all lie inside k
+  const uint32_t full_steps = k_bytes / BK;  // steps whose 128 bytes all lie inside k
   auto load_step = [&](int c, uint32_t step) {
     if (step < full_steps) load_chunk(c, step * BK);
     else load_chunk_tail(c, step * BK);
@@ -230,23 +237,33 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
   // writes begin, every load is at least half a step old).  STEADY: both steps exist and are
   // full, so the code is straight-line (a branch here would make the compiler wait for
   // every load where it is issued).
-  // DIRECT (k a multiple of 128): global_load_lds_dwordx4 moves a chunk from global memory
+  // DIRECT: global_load_lds_dwordx4 moves a chunk from global memory
   // straight into LDS (a wave's 64 lanes fill 1 KiB at a wave-uniform base, in lane order):
   // no staging registers, no LDS write instructions.  The chunks of step s+1 go into the
   // stage that step s-1 read, while step s computes.
-  auto direct_chunk = [&](int c, uint32_t step) {
-    const uint64_t src = c < A_CHUNKS ? a_src[c < A_CHUNKS ? c : 0] : b_src[c < A_CHUNKS ? 0 : c - A_CHUNKS];
+  // partial: the last step of a k that is not a multiple of 128 bytes.  The lanes whose chunk (a k-contiguous operand)
+  // or whose row of k (a k-major one) lies past the end fetch zeros.  Only that step pays for the comparison.
+  auto direct_chunk = [&](int c, uint32_t step, auto partial) {
+    uint64_t src = c < A_CHUNKS ? a_src[c < A_CHUNKS ? c : 0] : b_src[c < A_CHUNKS ? 0 : c - A_CHUNKS];
     const uint32_t tile_base = c < A_CHUNKS ? uint32_t(c) * NT * 16 : BM * BK + uint32_t(c - A_CHUNKS) * NT * 16;
     uint8_t* dst = lds + (step & 1u) * STAGE + tile_base + uint32_t(wave) * 1024;
     // a step is 128 bytes along a k-contiguous row, or 64 rows of a k-major operand
     const uint64_t advance = c < A_CHUNKS ? (TRA ? uint64_t(BK / 2) * p.lda : uint64_t(BK)) : (TRB ? uint64_t(BK / 2) * p.ldb : uint64_t(BK));
-    __builtin_amdgcn_global_load_lds(reinterpret_cast<const VKT_GLOBAL void*>(src + uint64_t(step) * advance),
+    src += uint64_t(step) * advance;
+    if constexpr (decltype(partial)::value) {
+      const bool first = c < A_CHUNKS;
+      const uint32_t id = tid + NT * (first ? c : c - A_CHUNKS), row = id >> 3;
+      const uint32_t at = (first ? TRA : TRB) ? id / ((first ? BM : BN) / 8) * 2 : ((id & 7u) ^ ((row >> 1) & 7u)) * 16;  // (k-major: rows of k of 2 bytes each)
+      if (step * BK + at >= k_bytes) src = reinterpret_cast<uint64_t>(&kZeroChunk[0]);
+    }
+    __builtin_amdgcn_global_load_lds(reinterpret_cast<const VKT_GLOBAL void*>(src),
                                      (__attribute__((address_space(3))) void*)(dst), 16, 0, 0);
   };
   auto side = [&](int op, uint32_t s, auto steady) {
     constexpr bool kSteady = decltype(steady)::value;
     if constexpr (DIRECT) {
-      if (kSteady || s + 1 < steps) direct_chunk(op, s + 1);
+      if (kSteady || s + 1 < full_steps) direct_chunk(op, s + 1, std::false_type{});
+      else if (s + 1 < steps) direct_chunk(op, s + 1, std::true_type{});
     } else if (op < NC) {
       if (kSteady || s + 1 < steps) store_chunk(op, (s + 1) & 1u);
     } else {
@@ -386,10 +403,13 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
   uint32_t s = 0;
   if constexpr (DIRECT) {
 #pragma unroll
-    for (int c = 0; c < NC; ++c) direct_chunk(c, 0);
+    for (int c = 0; c < NC; ++c) {
+      if (full_steps != 0) direct_chunk(c, 0, std::false_type{});
+      else direct_chunk(c, 0, std::true_type{});
+    }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    for (; s + 1 < steps; ++s) step(s, std::true_type{});
+    for (; s + 1 < full_steps; ++s) step(s, std::true_type{});
     for (; s < steps; ++s) step(s, std::false_type{});
   } else {
     // prologue: step 0 into LDS, step 1 into the registers
