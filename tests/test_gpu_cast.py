@@ -77,6 +77,20 @@ def test_producer_rowwise(f8, src, m, k, pad):
         assert np.array_equal(s[2:].view(np.uint32), ts.view(np.uint32)) and np.array_equal(q[2:], tq)
 
 
+@pytest.mark.parametrize("m,k,pad", [(255, 4112, 0), (256, 4112, 0), (9, 16384, 0), (300, 16400, 0), (16, 28672, 16), (1, 65536, 0),
+                                     (2, 65552, 0)])
+def test_producer_row_forms(m, k, pad):
+    """Either side of the lines between the forms of the row kernel: rows fewer than the compute units, 16384 and 65536 values."""
+    import _dev
+    x = (torch.randn(m, k, generator=gen(55 + k)) * 2).bfloat16()
+    x[0, k - 1], x[m - 1, 0] = 300.0, -500.0  # the largest value at an end of the row
+    q, s = _dev.fp8_quant(bits(x), oracle.BF16, oracle.E4M3, pad=pad)
+    wq, ws = oracle.fp8_quant(bits(x), oracle.BF16, oracle.E4M3)
+    assert np.array_equal(s.view(np.uint32), ws.view(np.uint32)) and np.array_equal(q, wq)
+    q, _ = _dev.fp8_quant(bits(x), oracle.BF16, oracle.E4M3, scale=0.0123, pad=pad)
+    assert np.array_equal(q, oracle.fp8_quant(bits(x), oracle.BF16, oracle.E4M3, scale=0.0123)[0])
+
+
 @pytest.mark.parametrize("f8", FLOAT8, ids=str)
 def test_producer_given_scale(f8):
     import _dev

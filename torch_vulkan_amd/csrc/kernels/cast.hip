@@ -102,14 +102,16 @@ __global__ __launch_bounds__(256) void cast_strided(MovePlan p) {
   }
 }
 
-// Workgroup-wide maximum of per-thread values (256 threads).
+// Workgroup-wide maximum of per-thread values, called once per launch.
+template <int THREADS>
 __device__ __forceinline__ float block_max(float v) {
-  __shared__ float part[4];
+  __shared__ float part[THREADS / 64];
   v = wave_max(v);
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
   __syncthreads();
-  const float r = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
-  __syncthreads();  // (part is reused by the next call)
+  float r = part[0];
+#pragma unroll
+  for (int i = 1; i < THREADS / 64; ++i) r = fmaxf(r, part[i]);
   return r;
 }
 
@@ -118,56 +120,55 @@ __device__ __forceinline__ float clamp_keep_nan(float y, float fmax) {
   return fmax < y ? fmax : y;
 }
 
-constexpr int kQuantGroups = 4;  // groups of 16 values a thread keeps in registers in the one-pass form
-
-// One workgroup per row.  ONE_PASS: k is a multiple of 16, at most 4096 * kQuantGroups, rows
-// aligned to 16 elements: the row is read once, into registers.  ROWWISE = 0: p.scale holds
-// one given scale (an input); 1: the row's scale is computed and written to p.scale[m].
-template <uint32_t SRC, uint32_t FMT, bool ONE_PASS>
-__global__ __launch_bounds__(256) void fp8_quant_kernel(F8QuantParams p, uint32_t rowwise) {
+// One workgroup of THREADS threads per row.  GROUPS > 0: k is a multiple of 16, at most THREADS * 16 * GROUPS, rows aligned
+// to 16 elements: the row is read once, into registers, GROUPS groups of 16 values per thread.  GROUPS = 0: any k and
+// alignment, an element at a time, the row read twice.  ROWWISE = 0: p.scale holds one given scale (an input); 1: the row's
+// scale is computed and written to p.scale[m].
+template <uint32_t SRC, uint32_t FMT, int THREADS, int GROUPS>
+__global__ __launch_bounds__(THREADS) void fp8_quant_kernel(F8QuantParams p, uint32_t rowwise) {
   const uint32_t m = blockIdx.x, tid = threadIdx.x;
   const float fmax = FMT == VKT_E4M3 ? 448.0f : 57344.0f;
   const uint64_t row = p.src + uint64_t(m) * p.lds * item_size(SRC), out = p.dst + uint64_t(m) * p.ldd;
-  float x[kQuantGroups][16];
+  float x[GROUPS > 0 ? GROUPS : 1][16];
   const uint32_t groups = p.k / 16;
   float a;
   if (rowwise) {
     float amax = 0.0f;
-    if constexpr (ONE_PASS) {
+    if constexpr (GROUPS > 0) {
 #pragma unroll
-      for (int i = 0; i < kQuantGroups; ++i)
-        if (tid + 256 * i < groups) load16_any<SRC>(row + uint64_t(tid + 256 * i) * 16 * item_size(SRC), x[i]);
+      for (int i = 0; i < GROUPS; ++i)
+        if (tid + THREADS * i < groups) load16_any<SRC>(row + uint64_t(tid + THREADS * i) * 16 * item_size(SRC), x[i]);
 #pragma unroll
-      for (int i = 0; i < kQuantGroups; ++i)
-        if (tid + 256 * i < groups) {
+      for (int i = 0; i < GROUPS; ++i)
+        if (tid + THREADS * i < groups) {
 #pragma unroll
           for (int e = 0; e < 16; ++e) amax = fmaxf(amax, fabsf(x[i][e]));  // (fmaxf drops NaN)
         }
     } else {
-      for (uint32_t k = tid; k < p.k; k += 256) amax = fmaxf(amax, fabsf(load1_any<SRC>(row, k)));
+      for (uint32_t k = tid; k < p.k; k += THREADS) amax = fmaxf(amax, fabsf(load1_any<SRC>(row, k)));
     }
-    a = fmaxf(block_max(amax), 1e-12f);
+    a = fmaxf(block_max<THREADS>(amax), 1e-12f);
     if (tid == 0) stg<float>(p.scale + 4ull * m, a / fmax);
   } else {
     a = ldg<float>(p.scale) * fmax;  // the given scale is a / fmax
-    if constexpr (ONE_PASS) {
+    if constexpr (GROUPS > 0) {
 #pragma unroll
-      for (int i = 0; i < kQuantGroups; ++i)
-        if (tid + 256 * i < groups) load16_any<SRC>(row + uint64_t(tid + 256 * i) * 16 * item_size(SRC), x[i]);
+      for (int i = 0; i < GROUPS; ++i)
+        if (tid + THREADS * i < groups) load16_any<SRC>(row + uint64_t(tid + THREADS * i) * 16 * item_size(SRC), x[i]);
     }
   }
   const float inv = fmax / a;
-  if constexpr (ONE_PASS) {
+  if constexpr (GROUPS > 0) {
 #pragma unroll
-    for (int i = 0; i < kQuantGroups; ++i)
-      if (tid + 256 * i < groups) {
+    for (int i = 0; i < GROUPS; ++i)
+      if (tid + THREADS * i < groups) {
         float y[16];
 #pragma unroll
         for (int e = 0; e < 16; ++e) y[e] = clamp_keep_nan(x[i][e] * inv, fmax);
-        store16_any<FMT>(out + uint64_t(tid + 256 * i) * 16, y);
+        store16_any<FMT>(out + uint64_t(tid + THREADS * i) * 16, y);
       }
   } else {
-    for (uint32_t k = tid; k < p.k; k += 256)
+    for (uint32_t k = tid; k < p.k; k += THREADS)
       store1_any<FMT>(out, k, clamp_keep_nan(load1_any<SRC>(row, k) * inv, fmax));
   }
 }
@@ -185,12 +186,22 @@ int launch_cast_from(const CastParams& p, uint32_t vector, uint32_t groups, hipS
   return -1;
 }
 
+// The forms by row length and count.  What bounds few rows is the latency of one workgroup's chain, many rows the memory.  Rows
+// of up to 16384 values: 256 threads where there are enough rows to fill the machine; with fewer rows than compute units 1024 threads
+// with a group each (16 x 8192 bfloat16, by the clock around 30 calls: 5.7 -> 5.3 us, 255 x 8192 5.8 -> 5.4).  Rows of up to 65536
+// values: 1024 threads with four groups; read twice, an element at a time, 16 x 28672 took 67.7 us in the kernel trace (now 5.0),
+// 4096 x 28672 259 us (80), 8192 x 28672 532 us (149, 4.7 TB/s).
 template <uint32_t SRC, uint32_t FMT>
-void launch_quant(const F8QuantParams& p, uint32_t rowwise, hipStream_t stream) {
-  const bool one_pass = p.k % 16 == 0 && p.k <= 4096u * kQuantGroups && (p.src % (16 * item_size(SRC))) == 0 &&
-                        (uint64_t(p.lds) * item_size(SRC)) % (16 * item_size(SRC)) == 0 && p.dst % 16 == 0 && p.ldd % 16 == 0;
-  if (one_pass) hipLaunchKernelGGL((fp8_quant_kernel<SRC, FMT, true>), dim3(p.m), dim3(256), 0, stream, p, rowwise);
-  else hipLaunchKernelGGL((fp8_quant_kernel<SRC, FMT, false>), dim3(p.m), dim3(256), 0, stream, p, rowwise);
+void launch_quant(const F8QuantParams& p, uint32_t rowwise, const Machine& mc, hipStream_t stream) {
+  const bool aligned = p.k % 16 == 0 && (p.src % (16 * item_size(SRC))) == 0 &&
+                       (uint64_t(p.lds) * item_size(SRC)) % (16 * item_size(SRC)) == 0 && p.dst % 16 == 0 && p.ldd % 16 == 0;
+  const bool few = p.m < uint32_t(mc.compute_units) && p.k > 4096;
+#define VKT_QUANT_FORM(T, G) hipLaunchKernelGGL((fp8_quant_kernel<SRC, FMT, T, G>), dim3(p.m), dim3(T), 0, stream, p, rowwise)
+  if (!aligned || p.k > 65536) VKT_QUANT_FORM(256, 0);
+  else if (p.k > 16384) VKT_QUANT_FORM(1024, 4);
+  else if (few) VKT_QUANT_FORM(1024, 1);
+  else VKT_QUANT_FORM(256, 4);
+#undef VKT_QUANT_FORM
 }
 
 }  // namespace
@@ -253,7 +264,7 @@ int launch_cast_strided(const StridedParams& s, int src_dtype, int dst_dtype, co
   return 0;
 }
 
-int launch_fp8_quant(const F8QuantParams& p, uint32_t rowwise, const Machine&, hipStream_t stream, std::string* err) {
+int launch_fp8_quant(const F8QuantParams& p, uint32_t rowwise, const Machine& mc, hipStream_t stream, std::string* err) {
   if (p.m == 0 || p.k == 0) return 0;
   if (p.src_dtype > VKT_BF16 || !is_fp8_host(p.dst_fmt)) {
     *err = "fp8_quant: float32 / float16 / bfloat16 in, e4m3fn / e5m2 out";
@@ -272,7 +283,7 @@ int launch_fp8_quant(const F8QuantParams& p, uint32_t rowwise, const Machine&, h
     return -1;
   }
 #define VKT_QUANT_CASE(S, F) \
-  if (p.src_dtype == S && p.dst_fmt == F) launch_quant<S, F>(p, rowwise, stream);
+  if (p.src_dtype == S && p.dst_fmt == F) launch_quant<S, F>(p, rowwise, mc, stream);
   VKT_QUANT_CASE(VKT_F32, VKT_E4M3) VKT_QUANT_CASE(VKT_F32, VKT_E5M2)
   VKT_QUANT_CASE(VKT_F16, VKT_E4M3) VKT_QUANT_CASE(VKT_F16, VKT_E5M2)
   VKT_QUANT_CASE(VKT_BF16, VKT_E4M3) VKT_QUANT_CASE(VKT_BF16, VKT_E5M2)
