@@ -165,8 +165,9 @@ typedef struct Q4PackParams {
  * product; PHASE 2 does both: with LAYOUT 0 in one launch per 4 rows where the rows can
  * be quantised from registers (k a multiple of 8, at most 16384), otherwise as PHASE 0
  * then 1.  Results are bit-identical to qmm4.  With LAYOUT 1, bits 4-7 of PHASE override the choice
- * between the two product kernels, which give the same bits (tests, tuning): 16 keeps the kernel whose four waves
- * split K, 32 forces the one whose waves each walk all of K (| 64, 128, 192: 1, 2, 4 tiles of 16 x 16 per wave).
+ * between the product kernels, which give the same bits (tests, tuning): 16 keeps the kernel whose four waves
+ * split K, 32 forces those whose waves each walk all of K (| 64, 128, 192: 1, 2, 4 tiles of 16 x 16 per wave; blocks of 32 and 64:
+ * 1, 4, 8, the latter two against the runtime's workspace, to which PHASE 2 then writes the activations instead of to q).
  * With LAYOUT 0, PHASE 2 with 1, 2 or 3 in bits 8-9 fixes the column tiles per workgroup (same bits). */
 typedef struct Q4CParams {
   uint64_t inp, q, rows, compact, out;

@@ -702,14 +702,47 @@ __device__ __forceinline__ uint64_t operand_offset(uint32_t m, uint32_t g, uint3
   return (((uint64_t(m >> 4) * quads + (unit >> 2)) * 2 + (j >> 1)) * 64 + kg * 16 + (m & 15)) * 16 + (j & 1) * 8;
 }
 
-// Phase 0 for the matrix layout, one workgroup per row.  FAST: k is a multiple of 8, at most
-// 2048 * kFusedGroups, rows 16-byte aligned: the row is read once, into registers.
-template <class T, bool FAST>
-__global__ __launch_bounds__(256) void qmm4m_rowquant(Q4CParams p, uint32_t groupwise, uint32_t quads) {
+// The same 8 values less the zero point as float16, which holds -255 .. 255 exactly, for qmm4m_half: the pairs (0, 4), (1, 5),
+// (2, 6), (3, 7), in which a word of nibbles comes apart.  [row tile][unit][lane = kg * 16 + m % 16] x 16 bytes, the
+// order of qmm4m_half's lanes.  (A row's workgroup writes 16 bytes of a line; with 128 bytes of a row side by side it takes
+// 10.7 instead of 18.1 us for 2048 x 4096 values, but the product that reads them 451 instead of 331.)
+using V2H = _Float16 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ U4 operand_halves(const int (&a)[8]) {
+  U4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = __builtin_bit_cast(uint32_t, V2H{_Float16(float(a[i])), _Float16(float(a[i + 4]))});
+  return r;
+}
+__device__ __forceinline__ uint64_t halves_offset(uint32_t m, uint32_t g, uint32_t quads) {
+  return ((uint64_t(m >> 4) * (quads * 4) + (g >> 2)) * 64 + (g & 3) * 16 + (m & 15)) * 16;
+}
+
+// Phase 0 for the matrix layout, one workgroup per row, from row m0 on.  FAST: k is a multiple of 8, at most
+// 2048 * kFusedGroups, rows 16-byte aligned: the row is read once, into registers.  HALVES: the values go to `dst` as
+// qmm4m_half's operand, row m0 first, instead of to p.q.
+template <class T, bool FAST, bool HALVES>
+__global__ __launch_bounds__(256) void qmm4m_rowquant(Q4CParams p, uint32_t groupwise, uint32_t quads, uint64_t dst, uint32_t m0) {
   constexpr uint64_t item = sizeof(typename T::storage);
-  const uint32_t m = blockIdx.x, tid = threadIdx.x;
+  const uint32_t m = m0 + blockIdx.x, tid = threadIdx.x;
   const uint64_t row = p.inp + uint64_t(m) * p.k * item;
   const uint32_t groups_all = quads * 16;
+  RowQuant rq;
+  auto scale_of_row = [&](float mn, float mx) {
+    rq = row_quant(mn, mx, groupwise != 0);
+    if (tid == 0) {
+      stg<uint32_t>(p.rows + 8ull * m, f32_bits(rq.recip));
+      stg<int32_t>(p.rows + 8ull * m + 4, -rq.izp);
+    }
+  };
+  auto put = [&](uint32_t g, int (&q)[8]) {
+    if constexpr (HALVES) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) q[e] -= rq.izp;
+      stg<U4>(dst + halves_offset(blockIdx.x, g, quads), operand_halves(q));
+    } else {
+      stg<U2>(p.q + operand_offset(m, g, quads), operand_bytes(q));
+    }
+  };
   if constexpr (FAST) {
     const uint32_t groups = p.k / 8;
     float x[kFusedGroups][8];
@@ -727,33 +760,23 @@ __global__ __launch_bounds__(256) void qmm4m_rowquant(Q4CParams p, uint32_t grou
       }
     }
     block_range(&mn, &mx);
-    const RowQuant rq = row_quant(mn, mx, groupwise != 0);
-    if (tid == 0) {
-      stg<uint32_t>(p.rows + 8ull * m, f32_bits(rq.recip));
-      stg<int32_t>(p.rows + 8ull * m + 4, -rq.izp);
-    }
+    scale_of_row(mn, mx);
 #pragma unroll
     for (int i = 0; i < kFusedGroups; ++i) {
       const uint32_t g = tid + 256 * i;
       if (g < groups_all) {
-        U2 v = {0u, 0u};
+        int q[8] = {0, 0, 0, 0, 0, 0, 0, 0};
         if (g < groups) {
-          int q[8];
 #pragma unroll
           for (int e = 0; e < 8; ++e) q[e] = quantise(x[i][e], rq);
-          v = operand_bytes(q);
         }
-        stg<U2>(p.q + operand_offset(m, g, quads), v);
+        put(g, q);
       }
     }
   } else {
     float mn, mx;
     row_range<T>(row, p.k, &mn, &mx);
-    const RowQuant rq = row_quant(mn, mx, groupwise != 0);
-    if (tid == 0) {
-      stg<uint32_t>(p.rows + 8ull * m, f32_bits(rq.recip));
-      stg<int32_t>(p.rows + 8ull * m + 4, -rq.izp);
-    }
+    scale_of_row(mn, mx);
     for (uint32_t g = tid; g < groups_all; g += 256) {
       int q[8];
 #pragma unroll
@@ -761,7 +784,7 @@ __global__ __launch_bounds__(256) void qmm4m_rowquant(Q4CParams p, uint32_t grou
         const uint32_t k = g * 8 + e;
         q[e] = k < p.k ? quantise(load_f32<T>(row + k * item), rq) : 0;
       }
-      stg<U2>(p.q + operand_offset(m, g, quads), operand_bytes(q));
+      put(g, q);
     }
   }
 }
@@ -1123,13 +1146,197 @@ __global__ __launch_bounds__(256) void qmm4m_rows(Q4CParams p, MatrixLayout L, u
   }
 }
 
+// ------------------------------------------------------------------ many rows, blocks of 32 and 64: float16 products
+
+// A load at a wave-uniform address plus a lane's offset.
+template <class X>
+__device__ __forceinline__ X ldg_at(uint64_t base, uint32_t offset) {
+  return *reinterpret_cast<const VKT_GLOBAL X*>(reinterpret_cast<const VKT_GLOBAL char*>(base) + offset);
+}
+
+using V4F = float __attribute__((ext_vector_type(4)));
+using V8H = _Float16 __attribute__((ext_vector_type(8)));
+
+// Rows that a PHASE 0 has left in p.q, `rows` of them from row m0 on (a multiple of 16), as qmm4m_half's operand: one thread per 8
+// values, whole row tiles (what stands in the rows past p.m is any integer of the range and goes nowhere).
+__global__ __launch_bounds__(256) void qmm4m_expand(Q4CParams p, uint64_t dst, uint32_t m0, uint32_t rows, uint32_t quads) {
+  const uint64_t id = uint64_t(blockIdx.x) * 256 + threadIdx.x;
+  const uint32_t lane = id & 63, unit = uint32_t((id >> 6) % (quads * 4));
+  const uint64_t rt = (id >> 6) / (quads * 4);
+  if (rt * 16 >= rows) return;
+  const uint32_t m = m0 + uint32_t(rt) * 16 + (lane & 15);
+  const U2 v = ldg<U2>(p.q + operand_offset(m, unit * 4 + (lane >> 4), quads));  // bytes 0, 2, 4, 6 and 1, 3, 5, 7
+  const int nzp = ldg<int32_t>(p.rows + 8ull * (m < p.m ? m : p.m - 1) + 4);
+  int a[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) a[e] = int(int8_t(((e & 1) ? v.y : v.x) >> (8 * (e >> 1)))) + nzp;
+  stg<U4>(dst + id * 16, operand_halves(a));
+}
+
+// Many rows, a wave per RT x CT matrix-core tiles that walks all of K, as qmm4m_rows, with the block sums on
+// v_mfma_f32_16x16x32_f16, exactly: a unit (32 values of k) is one instruction, and its sum arrives as the float32 number that
+// the block's scale multiplies.  A nibble v becomes a float16 with one AND and one OR (v_and_or_b32): 0x6400 | v is 1024 + v, and
+// 0x5400 | (v << 4), the upper nibble of a byte where it stands, is 64 + v, so a word of 8 nibbles takes 4 of them and a shift.
+// The surplus (1032 or 72 over nibble - 8) times the row's values of the block is one more product against a constant operand, common to
+// the CT column tiles, which enters the others as their accumulator input.  All sums are whole numbers below 2^24, whatever the
+// order: at most 64 x 255 x (1039 + 79) / 2 = 9.1e6.  That bounds the blocks to 64 values; longer ones stay on the integer form.
+// What bounds it: vector-unit issue.  Block-by-block float32 sums cost a product and an addition per output and block (8 instructions
+// per unit and tile), the nibbles 5 per unit and column tile, which RT row tiles share.  The integer
+// form (qmm4m_rows) takes 15 and four half-rate products.  2048 x 4096 x 11008, blocks of 32, kernel alone: 527 -> 318 us, 80 % of
+// the vector units' issue at the 2.05 GHz that the card holds in it.  2 x 4 tiles per wave (196 registers: two waves per SIMD) against
+// 2 x 2 and 4 x 2, whole call: 325, 360, 346 us.
+template <class T, int UPB, int RT, int CT>
+__global__ __launch_bounds__(256, 2) void qmm4m_half(Q4CParams p, MatrixLayout L, uint64_t halves, uint32_t m0, uint32_t rows) {
+  static_assert(UPB == 1 || UPB == 2, "sums below 2^24");
+  constexpr uint64_t item = sizeof(typename T::storage);
+  const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t col = lane & 15, kg = lane >> 4;
+  // Workgroups to operand panels: workgroup i runs on XCD i % 8, each with an L2 of its own, so an XCD takes a contiguous eighth
+  // of an order that walks down kPanel row groups before it moves on to the next column group.  (In the plain order an XCD's 64
+  // workgroups touch 43 column groups: a third of the reads hit L2, 2 GB came from beyond it, 352 us instead of 325.)
+  constexpr uint32_t kPanel = 8;
+  const uint32_t col_groups = (L.tiles + 4 * CT - 1) / (4 * CT), row_groups = (rows + 16 * RT - 1) / (16 * RT);
+  const uint32_t total = col_groups * row_groups, per = (total + 7) / 8, at = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((blockIdx.x >> 3) >= per || at >= total) return;
+  const uint32_t panel = at / (kPanel * col_groups), in_panel = at % (kPanel * col_groups);
+  const uint32_t panel_rows = row_groups - panel * kPanel < kPanel ? row_groups - panel * kPanel : kPanel;
+  const uint32_t tile0 = (in_panel / panel_rows * 4 + wave) * CT;
+  const uint32_t first = (panel * kPanel + in_panel % panel_rows) * (16 * RT);  // this wave's rows, counted from m0
+  if (tile0 >= L.tiles) return;  // (a whole wave, and the kernel has no barrier)
+
+  // (addresses: wave-uniform bases, on the scalar unit, plus a constant offset per lane)
+  uint64_t abase[RT], wbase[CT], sbase[CT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    const uint32_t rt = first + 16 * t < rows ? first + 16 * t : first;  // (a row tile past the end: the first again, not stored)
+    abase[t] = halves + uint64_t(rt >> 4) * L.quads * 4096;
+  }
+#pragma unroll
+  for (int c = 0; c < CT; ++c) {
+    const uint32_t tile = tile0 + c < L.tiles ? tile0 + c : tile0;
+    wbase[c] = p.compact + uint64_t(tile) * 1024;
+    sbase[c] = p.compact + L.scale_off + uint64_t(tile) * 256;
+  }
+  const uint64_t wstep = uint64_t(L.tiles) * 1024, sstep = uint64_t(L.tiles) * 256;
+  const uint32_t lane_at = lane * 16, scale_at = col * 16;
+
+  struct Set {
+    U4 w[CT], a[RT][4];
+    F4 s[CT];
+  };
+  auto request = [&](Set& set, uint32_t quad) {
+    quad = quad < L.quads ? quad : L.quads - 1;
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      set.w[c] = ldg_at<U4>(wbase[c] + quad * wstep, lane_at);
+      set.s[c] = ldg_at<F4>(sbase[c] + quad * sstep, scale_at);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int t = 0; t < RT; ++t) set.a[t][j] = ldg_at<U4>(abase[t] + uint64_t(quad) * 4096, lane_at + j * 1024);
+  };
+
+  float acc[RT][CT][4];
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[t][c][r] = -0.0f;
+  const U4 surplus_bits = {0xe408e408u, 0xd480d480u, 0xe408e408u, 0xd480d480u};  // -1032, -72, -1032, -72, twice each
+  const V8H surplus = __builtin_bit_cast(V8H, surplus_bits);
+  // (v_and_or_b32 takes no literals and one scalar: the masks are kept in vector registers, which an empty statement hides
+  // from the compiler; left to it, each nibble pair is an AND and an OR)
+  uint32_t low = 0x000f000fu, high = 0x00f000f0u;
+  asm volatile("" : "+v"(low), "+v"(high));
+  auto nibbles = [&](uint32_t v) {
+    const uint32_t v8 = v >> 8;
+    const U4 b = {(v & low) | 0x64006400u, (v & high) | 0x54005400u, (v8 & low) | 0x64006400u, (v8 & high) | 0x54005400u};
+    return __builtin_bit_cast(V8H, b);
+  };
+  auto process = [&](const Set& set) {
+    V4F x[2][RT], start[RT];  // the sums of this column tile and of the one before it, whose float32 work fills the wait for them
+    constexpr int TILES = 4 / UPB * CT;
+#pragma unroll
+    for (int i = 0; i <= TILES; ++i) {
+      const int j = i / CT * UPB, c = i % CT;
+      if (i < TILES) {
+        if (c == 0) {
+#pragma unroll
+          for (int t = 0; t < RT; ++t) {
+            start[t] = V4F{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int u = 0; u < UPB; ++u)
+              start[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(V8H, set.a[t][j + u]), surplus, start[t], 0, 0, 0);
+          }
+        }
+        V8H b[UPB];
+#pragma unroll
+        for (int u = 0; u < UPB; ++u) b[u] = nibbles(set.w[c][j + u]);
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+          x[i & 1][t] = start[t];
+#pragma unroll
+          for (int u = 0; u < UPB; ++u)
+            x[i & 1][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(V8H, set.a[t][j + u]), b[u], x[i & 1][t], 0, 0, 0);
+        }
+      }
+      if (i > 0) {
+        const int cb = (i - 1) % CT, jb = (i - 1) / CT * UPB;
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[t][cb][r] = acc[t][cb][r] + x[(i - 1) & 1][t][r] * set.s[cb][jb];  // in block order
+      }
+      __builtin_amdgcn_sched_barrier(0);  // (left to itself the scheduler puts sums next to the instruction that makes them: 378 us instead of 366)
+    }
+  };
+  Set even, odd;
+  request(even, 0);
+  for (uint32_t quad = 0; quad < L.quads; quad += 2) {  // (quads is a multiple of 16)
+    request(odd, quad + 1);
+    process(even);
+    request(even, quad + 2);  // (past the end the last quad again, so that the loop is straight-line code)
+    process(odd);
+  }
+#pragma unroll
+  for (int c = 0; c < CT; ++c) {
+    const uint32_t n = (tile0 + c) * kTileCols + col;
+    if (tile0 + c >= L.tiles || n >= p.n) continue;
+    const float bias = ldg<float>(p.compact + L.bias_off + n * 4ull);
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const uint32_t in = first + 16 * t + kg * 4 + r, m = m0 + in;
+        if (in >= rows) continue;
+        finish_store<T>(p.out + (uint64_t(m) * p.n + n) * item, acc[t][c][r], bits_f32(ldg<uint32_t>(p.rows + 8ull * m)), p.has_bias != 0, bias);
+      }
+  }
+}
+
+template <class T, int UPB, int RT, int CT>
+void launch_half(const Q4CParams& p, const MatrixLayout& M, uint64_t halves, uint32_t m0, uint32_t rows, hipStream_t stream) {
+  const uint64_t total = uint64_t((M.tiles + 4 * CT - 1) / (4 * CT)) * ((rows + 16 * RT - 1) / (16 * RT));
+  const dim3 grid(uint32_t((total + 7) / 8 * 8));
+  hipLaunchKernelGGL((qmm4m_half<T, UPB, RT, CT>), grid, dim3(256), 0, stream, p, M, halves, m0, rows);
+}
+
+// (blocks of 32 and 64: one tile per wave only)
 template <class T, int RT, int CT>
 int launch_rows(const Q4CParams& p, const MatrixLayout& M, uint32_t m0, uint32_t rows, hipStream_t stream) {
   const dim3 grid((M.tiles + 4 * CT - 1) / (4 * CT), (rows + 16 * RT - 1) / (16 * RT));
   switch (M.upb) {
     case 0: hipLaunchKernelGGL((qmm4m_rows<T, 0, RT, CT>), grid, dim3(256), 0, stream, p, M, m0); break;
-    case 1: hipLaunchKernelGGL((qmm4m_rows<T, 1, RT, CT>), grid, dim3(256), 0, stream, p, M, m0); break;
-    case 2: hipLaunchKernelGGL((qmm4m_rows<T, 2, RT, CT>), grid, dim3(256), 0, stream, p, M, m0); break;
+    case 1:
+      if constexpr (RT * CT == 1) hipLaunchKernelGGL((qmm4m_rows<T, 1, 1, 1>), grid, dim3(256), 0, stream, p, M, m0);
+      else return -1;
+      break;
+    case 2:
+      if constexpr (RT * CT == 1) hipLaunchKernelGGL((qmm4m_rows<T, 2, 1, 1>), grid, dim3(256), 0, stream, p, M, m0);
+      else return -1;
+      break;
     case 4: hipLaunchKernelGGL((qmm4m_rows<T, 4, RT, CT>), grid, dim3(256), 0, stream, p, M, m0); break;
     case 8: hipLaunchKernelGGL((qmm4m_rows<T, 8, RT, CT>), grid, dim3(256), 0, stream, p, M, m0); break;
     default: return -1;
@@ -1321,7 +1528,7 @@ int launch_qmm4c_pack(const Q4PackParams& p, uint32_t layout, const Machine&, hi
 
 // The matrix-layout form of the product: phase 0, 1 or 2 (= 0 then 1).
 template <class T>
-int launch_matrix(const Q4CParams& p, uint32_t phase_and_flags, uint32_t groupwise, hipStream_t stream, std::string* err) {
+int launch_matrix(const Q4CParams& p, uint32_t phase_and_flags, uint32_t groupwise, const Machine& mc, hipStream_t stream, std::string* err) {
   constexpr uint32_t item = sizeof(typename T::storage);
   const uint32_t phase = phase_and_flags & 15u, flags = phase_and_flags & ~15u;
   MatrixLayout M;
@@ -1333,30 +1540,59 @@ int launch_matrix(const Q4CParams& p, uint32_t phase_and_flags, uint32_t groupwi
     *err = "qmm4c: null or unaligned tensor address";
     return -1;
   }
-  if (phase == 0 || phase == 2) {
-    if (p.m > 65535) {
-      *err = "qmm4c: at most 65535 rows per dispatch";
-      return -1;
+  if ((phase == 1 || phase == 2) && (!p.compact || (p.compact & 15))) {
+    *err = "qmm4c: null or unaligned side-car address";
+    return -1;
+  }
+  if (phase != 1 && p.m > 65535) {
+    *err = "qmm4c: at most 65535 rows per dispatch";
+    return -1;
+  }
+  const bool fast = p.k % 8 == 0 && p.k <= 2048u * kFusedGroups && (p.inp & 15) == 0 && (uint64_t(p.k) * item) % 16 == 0;
+  // Enough row tiles x column tiles to give every SIMD two waves (two and a half channelwise): a wave per tile walks all of K; fewer: the
+  // one-row-tile kernel, whose four waves split K.  Phase values 1 | 2 with bit 4 (16) set keep the one-row-tile
+  // kernel, with bit 5 (32) force the wave-per-tile kernels (tests, tuning; flag bits 6-7 choose among those).
+  const bool rows_kernel = ((uint64_t((p.m + 15) / 16) * M.tiles >= (M.upb ? 2048u : 2560u) && !(flags & 16)) || (flags & 32));
+  // Blocks of 32 and 64, many tiles: the products in float16 (qmm4m_half), 2 x 4 or 2 x 2 tiles per wave, against a workspace that
+  // holds the rows' values, in pieces of rows that fit it.  Fewer waves than four for every five SIMDs of 2 x 2: the integer kernel, a
+  // wave per tile (us at blocks of 32, waves of 2 x 2 in brackets: 128 x 11008 x 4096 [512] integers 59, float16 67; 64 x 4096 x
+  // 11008 [688] 30, 30; 256 x 4096 x 4096 [1024] 36.5, 34; 128 x 4096 x 11008 [1376] 50, 43.5; 64 x 4096 x 28672 [1792] 61, 45).
+  // 2 x 4 from three waves for two SIMDs on (128 x 4096 x 11008 [688 of 2 x 4] 48.5 against 43.5; 64 x 4096 x 28672 [896] 49.5, 45;
+  // 100 x 4096 x 27777 in blocks of 64 [1738] 67, 80; 512 x 4096 x 11008 [2752] 108, 110).
+  const uint64_t row_bytes = uint64_t(M.quads) * 256;
+  const uint64_t row_pairs = (uint64_t(p.m) + 31) / 32, simds = uint64_t(mc.compute_units) * 4;
+  uint32_t piece = uint32_t((mc.workspace_bytes / row_bytes < 16384 ? mc.workspace_bytes / row_bytes : 16384) & ~63ull);
+  const uint32_t asked = (flags & 32) ? (flags >> 6) & 3u : 0;
+  const bool eight = asked ? asked == 3 : row_pairs * ((M.tiles + 3) / 4) * 2 >= simds * 3;
+  const bool halves = (M.upb == 1 || M.upb == 2) && rows_kernel && piece >= 64 &&
+                      (asked ? asked >= 2 : row_pairs * ((M.tiles + 1) / 2) * 5 >= simds * 4);
+  if (halves && phase != 0) {
+    const uint32_t pieces = (p.m + piece - 1) / piece;
+    piece = ((p.m + pieces - 1) / pieces + 63) & ~63u;  // (of about equal size)
+    for (uint32_t m0 = 0; m0 < p.m; m0 += piece) {
+      const uint32_t rows = p.m - m0 < piece ? p.m - m0 : piece;
+      const uint64_t at = mc.workspace;
+      const uint32_t threads = (rows + 15) / 16 * 16 * M.quads * 16;  // (below the workspace's bytes / 16)
+      if (phase == 1) hipLaunchKernelGGL(qmm4m_expand, dim3(threads / 256), dim3(256), 0, stream, p, at, m0, rows, M.quads);
+      else if (fast) hipLaunchKernelGGL((qmm4m_rowquant<T, true, true>), dim3(rows), dim3(256), 0, stream, p, groupwise, M.quads, at, m0);
+      else hipLaunchKernelGGL((qmm4m_rowquant<T, false, true>), dim3(rows), dim3(256), 0, stream, p, groupwise, M.quads, at, m0);
+      if (M.upb == 1 && eight) launch_half<T, 1, 2, 4>(p, M, at, m0, rows, stream);
+      else if (M.upb == 1) launch_half<T, 1, 2, 2>(p, M, at, m0, rows, stream);
+      else if (eight) launch_half<T, 2, 2, 4>(p, M, at, m0, rows, stream);
+      else launch_half<T, 2, 2, 2>(p, M, at, m0, rows, stream);
     }
-    const bool fast = p.k % 8 == 0 && p.k <= 2048u * kFusedGroups && (p.inp & 15) == 0 && (uint64_t(p.k) * item) % 16 == 0;
-    if (fast) hipLaunchKernelGGL((qmm4m_rowquant<T, true>), dim3(p.m), dim3(256), 0, stream, p, groupwise, M.quads);
-    else hipLaunchKernelGGL((qmm4m_rowquant<T, false>), dim3(p.m), dim3(256), 0, stream, p, groupwise, M.quads);
+    return 0;
+  }
+  if (phase == 0 || phase == 2) {
+    if (fast) hipLaunchKernelGGL((qmm4m_rowquant<T, true, false>), dim3(p.m), dim3(256), 0, stream, p, groupwise, M.quads, 0ull, 0u);
+    else hipLaunchKernelGGL((qmm4m_rowquant<T, false, false>), dim3(p.m), dim3(256), 0, stream, p, groupwise, M.quads, 0ull, 0u);
   }
   if (phase == 1 || phase == 2) {
-    if (!p.compact || (p.compact & 15)) {
-      *err = "qmm4c: null or unaligned side-car address";
-      return -1;
-    }
-    // Enough row tiles x column tiles to give every SIMD two waves (two and a half channelwise): a wave per tile walks all of K; fewer: the
-    // one-row-tile kernel, whose four waves split K.  Phase values 1 | 2 with bit 4 (16) set keep the one-row-tile
-    // kernel, with bit 5 (32) force the wave-per-tile kernel (tests, tuning).
-    const bool rows_kernel = ((uint64_t((p.m + 15) / 16) * M.tiles >= (M.upb ? 2048u : 2560u) && !(flags & 16)) || (flags & 32));
-    // (wave tiles of 2 x 2, 2 x 1 or 1 x 1 matrix-core tiles: the largest that leaves every SIMD two and a half
-    //  waves; flag bits 6-7 choose: 1 = 1 x 1, 2 = 2 x 1, 3 = 2 x 2)
     for (uint32_t m0 = 0; rows_kernel && m0 < p.m; m0 += 16 * 1024) {
       const uint32_t rows = p.m - m0 < 16 * 1024 ? p.m - m0 : 16 * 1024;
       uint32_t shape = (flags >> 6) & 3u;
-      if (shape == 0)
+      if (M.upb == 1 || M.upb == 2) shape = 1;  // (the float16 form has more tiles per wave)
+      else if (shape == 0)
         shape = uint64_t((rows + 31) / 32) * ((M.tiles + 1) / 2) >= 2560 ? 3 : uint64_t((rows + 31) / 32) * M.tiles >= 2560 ? 2 : 1;
       const int rc = shape == 3 ? launch_rows<T, 2, 2>(p, M, m0, rows, stream)
                    : shape == 2 ? launch_rows<T, 2, 1>(p, M, m0, rows, stream)
@@ -1400,8 +1636,8 @@ int launch_qmm4c(const Q4CParams& p, int dtype, uint32_t phase, uint32_t groupwi
       *err = (phase & 15u) > 2 || (phase & ~255u) ? "qmm4c: PHASE must be 0, 1 or 2" : "qmm4c: null or unaligned tensor address";
       return -1;
     }
-    const int rc = dtype == VKT_F32 ? launch_matrix<f32_t>(p, phase, groupwise, stream, err)
-                                    : launch_matrix<bf16_t>(p, phase, groupwise, stream, err);
+    const int rc = dtype == VKT_F32 ? launch_matrix<f32_t>(p, phase, groupwise, mc, stream, err)
+                                    : launch_matrix<bf16_t>(p, phase, groupwise, mc, stream, err);
     if (rc != 0) return rc;
     if (hipGetLastError() != hipSuccess) {
       *err = "qmm4c: kernel launch failed";
