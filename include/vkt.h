@@ -178,7 +178,8 @@ typedef struct Q4CParams {
  * C[b] = alpha * A[b] @ B[b] (+ beta * Cin[b] when USE_CIN), 16-bit operands, float32
  * accumulation, one rounding (the reference's block, linalg.cpp:25-34, and kernel,
  * shaders/gemmcm.slang).  Strides in elements; alpha and beta hold float32 bits in their low
- * words.  112 bytes.  VARIANT (tests, tuning; 0: planned): 1-5 tile shapes, 6 the stream kernel, 7 the few-row kernel
+ * words.  112 bytes.  VARIANT (tests, tuning; 0: planned): 1-5 tile shapes, 6 the stream kernel (bits
+ * 8-9: 1, 2, 3 for 256, 192, 128 columns per tile), 7 the few-row kernel
  * (x @ w.T with up to 64 rows; bits 8-11: 16s of columns per workgroup, bits 12-16: slices of K over workgroups), 8 the
  * vector-unit kernel (x @ w.T, up to 4 rows), 9 the few-row kernel for weights stored [k, n] (x @ w with up to 64 rows;
  * bits 12-16: slices of K), 10 the 128 x 128 tile kernel with K in slices over workgroups (A in rows of k; bits 8-12: slices,

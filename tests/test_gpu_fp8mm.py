@@ -307,6 +307,23 @@ def test_scaled_mm_stream_kernel(m, k, n, rowwise, with_bias, fb):
             assert (err[fin] <= (ref_tol(want, mag / 16.0, odt) + HW_WINDOW * mag / 16.0 + step)[fin]).all()
 
 
+@pytest.mark.parametrize("columns", [1, 2, 3])  # 256, 192, 128 per tile
+@pytest.mark.parametrize("m,k,n", [(257, 256, 8), (1, 272, 200), (300, 400, 392), (130, 1024, 136), (260, 912, 576), (4400, 144, 2696)])
+def test_scaled_mm_stream_kernel_columns(m, k, n, columns):
+    """The stream kernel's three tile widths, at the edges of tiles, over several tiles per workgroup and at k that ends inside a
+    step: the same products added in the same order as the 256 x 256 tile kernel, so its bits."""
+    import _dev
+    a = torch.randn(m, k, generator=gen(1085)).to(FLOAT8[0])
+    bt = torch.randn(n, k, generator=gen(1086)).to(FLOAT8[0])
+    sa = torch.empty(m, 1).uniform_(0.5, 2, generator=gen(1087)).numpy()
+    sb = torch.empty(1, n).uniform_(0.5, 2, generator=gen(1088)).numpy()
+    bias = torch.randn(n, generator=gen(1089)).numpy()
+    for odt in (oracle.BF16, oracle.E4M3):
+        kw = dict(bias=bias, bias_dtype=oracle.F32, out_dtype=odt)
+        got, want = (_dev.scaled_mm(bits(a), oracle.E4M3, bits(bt), oracle.E4M3, sa, sb, True, variant=v, **kw) for v in (11 | columns << 8, 8))
+        assert np.array_equal(got, want)
+
+
 def test_scaled_mm_stream_kernel_nan_and_inf():
     """NaN and infinities through the stream kernel's epilogue, whose bfloat16 conversion looks at its values one by one
     only where a wave has seen a NaN: NaN operands (both e4m3fn codes), e5m2 infinities of both signs (inf - inf and

@@ -55,6 +55,18 @@ def test_gemm16_tile_variants(dtype, variant, m, k, n):
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("variant", [6 | 1 << 8, 6 | 2 << 8, 6 | 3 << 8])
+@pytest.mark.parametrize("m,k,n", [(257, 128, 8), (1, 136, 200), (300, 200, 392), (260, 456, 576)])
+def test_gemm16_stream_kernel_columns(dtype, variant, m, k, n):
+    """256, 192 and 128 columns per tile of the stream kernel, at the edges of tiles and at k that ends inside a step."""
+    import _dev
+    a = bits((torch.randn(m, k, generator=gen(90)) * 0.5).to(dtype))
+    w = bits((torch.randn(n, k, generator=gen(91)) * 0.5).to(dtype))
+    want, mag = oracle.gemm16(a, w.T, ODT[dtype], want_mag=True)
+    close(_dev.gemm16(a, w.T, ODT[dtype], variant=variant), want, mag, dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
 @pytest.mark.parametrize("variant", [0, 7, 7 | 1 << 8, 7 | 2 << 8, 7 | 4 << 8])
 @pytest.mark.parametrize("m,k,n", [(1, 512, 64), (7, 1032, 200), (16, 2048, 1000), (17, 520, 77), (33, 1536, 4100), (64, 2048, 1032), (50, 4096, 520),
                                    (3, 4096, 264), (12, 8192, 100)])  # (few columns against long rows: 8 columns and 16 waves per workgroup)

@@ -351,12 +351,12 @@ int launch_tile(const F8Params& p, int compute_units, hipStream_t stream, std::s
 
 // The stream kernel, where it serves the problem (bfloat16 or float8 output in aligned rows); -2: it does not.
 template <int FA, int FB>
-int launch_stream(const F8Params& p, int compute_units, hipStream_t stream, std::string* err) {
+int launch_stream(const F8Params& p, uint32_t columns, int compute_units, hipStream_t stream, std::string* err) {
   F8Problem problem;
   static_cast<F8Params&>(problem) = p;
   const bool float8_out = p.out_dtype == VKT_E4M3 || p.out_dtype == VKT_E5M2;
   if (!(p.out_dtype == VKT_BF16 || float8_out) || p.ldo % 8 || p.out % (float8_out ? 8 : 16) || !mma_stream_serves(problem)) return -2;
-  return launch_mma_stream<FA, FB, kMathFp8>(problem, compute_units, stream, err, "fp8mm");
+  return launch_mma_stream<FA, FB, kMathFp8>(problem, columns, compute_units, stream, err, "fp8mm");
 }
 
 template <int FA, int FB>
@@ -413,13 +413,18 @@ int launch_formats(const F8Params& p, uint32_t variant, const Machine& mc, hipSt
     }
     variant = 0;
   }
-  // (256 x 256 tiles where they give the machine enough workgroups, else 128 x 128: the exact path from one tile per
-  //  compute unit on (2048 x 4096 x 4096: 94 us on 128 x 128 tiles against 116; 1024 x 8192 x 8192: 164 against 200),
-  //  the float8 path from one per four units on (512 x 8192 x 8192: 64 against 82 us; at 1024 rows the stream kernel
-  //  is ahead, 91 against 99))
+  // (The exact path: 256 x 256 tiles from one per compute unit on, else 128 x 128: 2048 x 4096 x 4096: 94 us on 128 x 128 tiles against 116;
+  //  1024 x 8192 x 8192: 164 against 200.  The float8 path: the stream kernel from half a 128 x 128 tile per compute unit on, with the columns
+  //  per tile that suit the shape (us, 128 x 128 tiles / stream: 160 tiles of 512 x 5120 x 8192 61 / 54, 256 of 512 x 8192 x 8192 66 / 56, 258 of
+  //  300 x 11008 x 4096 49 / 33, 288 of 1500 x 3072 x 8192 84 / 56); with fewer tiles the smaller ones leave less of the machine idle.  Where
+  //  it does not serve: 256 x 256 tiles from one per four units on, else 128 x 128.)
   const uint64_t tiles256 = uint64_t((p.m + 255) / 256) * ((p.n + 255) / 256), cus = uint64_t(compute_units);
-  if (variant == 0)
-    variant = (p.out_dtype == VKT_F32 || p.out_dtype == VKT_F16) ? (big && tiles256 >= cus ? 6 : 7) : (big && 4 * tiles256 > cus ? 11 : 1);
+  const uint64_t tiles128 = uint64_t((p.m + 127) / 128) * ((p.n + 127) / 128);
+  bool small = false;  // what the stream kernel's products run on where it does not serve
+  if (variant == 0 && (p.out_dtype == VKT_F32 || p.out_dtype == VKT_F16)) variant = big && tiles256 >= cus ? 6 : 7;
+  else if (variant == 0) variant = 2 * tiles128 > cus ? 11 : 1, small = !(big && 4 * tiles256 > cus);
+  const uint32_t columns = (variant & ~0x300u) == 11 ? variant >> 8 : 0;  // (bits 8-9: columns per tile, mma_stream.h)
+  if (columns) variant = 11;
   if ((variant & 0xff) == 14) return launch_sliced<FA, FB>(p, (variant >> 8) & 31u, mc, stream, err);
   switch (variant) {
     case 6: return launch_tile<2, 2, 8, 8, FA, FB, true, true, true>(p, compute_units, stream, err);
@@ -430,8 +435,9 @@ int launch_formats(const F8Params& p, uint32_t variant, const Machine& mc, hipSt
     case 4: return launch_tile<2, 2, 8, 8, FA, FB, true>(p, compute_units, stream, err);
     case 9: return launch_tile<4, 2, 4, 8, FA, FB, true, true, true>(p, compute_units, stream, err);  // as 6 with 8 waves of 64x128
     case 11: {  // the stream kernel (mma_stream.h), else 8
-      const int rc = launch_stream<FA, FB>(p, compute_units, stream, err);
+      const int rc = launch_stream<FA, FB>(p, columns, compute_units, stream, err);
       if (rc != -2) return rc;
+      if (small) return launch_tile<2, 2, 4, 4, FA, FB>(p, compute_units, stream, err);
     }
       [[fallthrough]];
     case 8: return launch_tile<4, 2, 4, 8, FA, FB, true, true>(p, compute_units, stream, err);  // 256x256 tiles over 8 waves of 64x128 (two waves per SIMD), direct loads

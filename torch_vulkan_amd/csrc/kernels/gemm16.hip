@@ -300,6 +300,7 @@ int launch_tiles(const GemmParams& p, uint32_t use_cin, uint32_t batch, uint32_t
   // variant 0: planned; 1: 128x128 tiles; 2: 256x128; 3: 256x256 with direct loads; 4: 128x128 with direct loads;
   // 5: 256x256 with direct loads over 8 waves; 6: the stream kernel (mma_stream.h; else 3)
   // (k-major operands run on the direct forms only)
+  uint32_t small = 3;  // what the stream kernel's products run on where it does not serve
   if (variant == 0) {
     // 256 x 256 tiles where they give every compute unit one, else 128 x 128
     // (from five eighths of a tile per unit on: 1024 x 4096 x 14336 is 224 tiles on 256 units, 121 us on the stream
@@ -308,15 +309,20 @@ int launch_tiles(const GemmParams& p, uint32_t use_cin, uint32_t batch, uint32_t
     // (both operands k-major: 8 waves, whose transposing LDS reads cover each other: 8192^3 0.94 -> 1.11-1.13 PFLOP/s;
     //  with k-contiguous operands the 8-wave form reads 1.5x the LDS bytes and is 3-5 % slower)
     variant = large ? (TRA && TRB ? 5 : 3) : (TRA || TRB ? 4 : 1);
-    // both operands contiguous along k (x @ w.T): the stream kernel where it serves (8192^3: 0.94-1.00 -> 0.89 ms)
-    if (!TRA && !TRB && variant == 3) variant = 6;
+    // both operands contiguous along k (x @ w.T): the stream kernel where it serves (8192^3: 0.94-1.00 -> 0.89 ms), with the columns per
+    // tile that suit the shape also below that line, from more 128 x 128 tiles than compute units on (us, 128 x 128 tiles / stream: 258
+    // tiles of 300 x 11008 x 4096 72 / 57, 288 of 1500 x 3072 x 8192 137 / 105, 512 of 2048 x 4096 x 4096 84 / 69; up to 256 tiles they are
+    // level: 512 x 8192 x 4096 56.1 / 55.5, 512 x 5120 x 4096 52.3 / 53.7)
+    const bool more = uint64_t((p.m + 127) / 128) * ((p.n + 127) / 128) * batch > uint64_t(mc.compute_units);
+    if (!TRA && !TRB && (variant == 3 || more)) small = variant, variant = 6;
   }
   const bool stream_ok = g.k > BK && p.n % 8 == 0 && p.c_sm % 8 == 0 && p.c_sb % 8 == 0 && p.c % 16 == 0 &&
                          mma_stream_strides_ok(g.lda, g.ldb);
-  if (variant == 6 && !stream_ok) variant = 3;
+  const uint32_t columns = (variant & ~0x300u) == 6 ? variant >> 8 : 0;  // (bits 8-9: columns per tile, mma_stream.h)
+  if ((variant & ~0x300u) == 6) variant = stream_ok ? 6 : small;
   if constexpr (!TRA && !TRB) {
     // 6: the stream kernel (mma_stream.h) where it serves the problem: more than 64 values of k, n a multiple of 8, C in 16-byte aligned rows
-    if (variant == 6) return launch_mma_stream<0, 0, MATH>(g, mc.compute_units, stream, err, "gemmcm");
+    if (variant == 6) return launch_mma_stream<0, 0, MATH>(g, columns, mc.compute_units, stream, err, "gemmcm");
     if (variant == 1) return launch_mma_tile<2, 2, 4, 4, 0, 0, true, false, MATH>(g, mc.compute_units, stream, err, "gemmcm");
     if (variant == 2) return launch_mma_tile<2, 2, 8, 4, 0, 0, true, false, MATH>(g, mc.compute_units, stream, err, "gemmcm");
   }
@@ -461,9 +467,11 @@ int launch_q8_gemm_t(const Q8Params& p, const Machine& mc, hipStream_t stream, s
   Q8GemmProblem<T> g;
   g.a = p.a, g.b = mc.scratch, g.m = p.m, g.n = p.n, g.k = p.k * 2, g.lda = uint32_t(p.a_sm) * 2, g.ldb = p.k * 2;
   g.batches = 1, g.a_batch = 0, g.b_batch = 0, g.c = p.c, g.scales = p.scales;
+  // (the stream kernel throughout: there are as many 128 x 128 tiles as compute units, and it is level there, 1024 x 4096 x 4096 69.2 against
+  //  68.0 us, and ahead from there on; see the 16-bit product)
+  if (g.k > BK && p.n % 8 == 0 && p.c % 16 == 0 && p.scales % 16 == 0 && mma_stream_strides_ok(g.lda, g.ldb))
+    return launch_mma_stream<0, 0, MATH>(g, 0, mc.compute_units, stream, err, "qmm8");
   const bool large = uint64_t((p.m + 255) / 256) * ((p.n + 255) / 256) * 8 >= uint64_t(mc.compute_units) * 5;  // (as for the 16-bit product)
-  if (large && g.k > BK && p.n % 8 == 0 && p.c % 16 == 0 && p.scales % 16 == 0 && mma_stream_strides_ok(g.lda, g.ldb))
-    return launch_mma_stream<0, 0, MATH>(g, mc.compute_units, stream, err, "qmm8");
   if (large) return launch_mma_tile<2, 2, 8, 8, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "qmm8");
   return launch_mma_tile<2, 2, 4, 4, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "qmm8");
 }

@@ -1,6 +1,7 @@
 // The matrix-core kernel for large products with 16-bit outputs (float8 operands for _scaled_mm, 16-bit operands for
 // the matrix product and the many-row int8 product): 256 x 256 tiles of A [m, k] x B [n, k]^T (rows of k contiguous
-// bytes, as in mma_tile.h) on 8 waves of 64 x 128, K in steps of 128 bytes through two LDS stages of 64 KiB.
+// bytes, as in mma_tile.h) on 8 waves of 64 x 128, K in steps of 128 bytes through two LDS stages of 64 KiB.  (Or 256 x 192 and 256 x
+// 128 tiles, waves of 64 x 96 and 64 x 64: mma_stream_columns.)
 // It differs from mma_tile in how a workgroup's time is laid out, after measuring where mma_tile's goes (one wave's
 // clock read at four points of every step): the matrix cores were busy 58-66 % of the cycles; the rest was the wave
 // issuing address arithmetic for its LDS-direct loads (380 cycles a step) and all eight waves starting every step
@@ -47,13 +48,14 @@ __device__ __forceinline__ void load_to_lds_at(uint64_t address, uint32_t lds_at
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off offset:%2" ::"v"(address), "s"(lds_at), "i"(OFF) : "memory");
 }
 
-template <int FA, int FB, int MATH, bool TAIL, class P>
+template <int FA, int FB, int MATH, int COLUMNS, bool TAIL, class P>
 __global__ __launch_bounds__(512) void mma_stream(P p, uint32_t tiles_m, uint32_t tiles_n) {
   static_assert(!P::kTransA && !P::kTransB, "operands contiguous along k");
   constexpr int WM = 4;  // waves along m: 8 waves of 64 x 128
-  constexpr uint32_t BM = 256, BN = 256, STAGE = (BM + BN) * BK, B_AT = BM * BK;
-  constexpr int WAVES = WM * 2, TM2 = 8 / WM, TN2 = 4;  // a wave's (256 / WM) x 128 as 32 x 32 matrix-core tiles
-  constexpr int ROWS = 256 / WAVES, PER = ROWS / 8;    // rows of each operand tile a wave brings; loads per operand and step
+  constexpr uint32_t BM = 256, BN = COLUMNS, STAGE = (BM + BN) * BK, B_AT = BM * BK;
+  constexpr int WAVES = WM * 2, TM2 = 8 / WM, TN2 = BN / 64;  // a wave's (256 / WM) x (BN / 2) as 32 x 32 matrix-core tiles
+  constexpr int ROWS_A = BM / WAVES, ROWS_B = BN / WAVES;     // rows of each operand tile a wave brings
+  constexpr int PER_A = ROWS_A / 8, PER_B = ROWS_B / 8, PER = PER_A + PER_B;  // its loads of each and of both per step
   constexpr int NM = TM2 * TN2;                        // matrix-core tiles per half step
   constexpr uint32_t BIAS = 3072;  // keeps the per-lane offsets non-negative (they carry -1024 (i % 4) for load i)
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -85,7 +87,7 @@ __global__ __launch_bounds__(512) void mma_stream(P p, uint32_t tiles_m, uint32_
   // the swizzle keeps in its slot.
   uint32_t load_tile = 0, load_s = 0;
   uint64_t load_a = 0, load_b = 0;  // uniform: the tile's first row, less BIAS
-  uint32_t off_a[PER], off_b[PER];
+  uint32_t off_a[PER_A], off_b[PER_B];
   auto load_setup = [&](uint32_t index) {
     const Tile t = tile_at(index);
     load_a = p.a + uint64_t(t.batch) * p.a_batch + uint64_t(t.m0) * p.lda - BIAS;
@@ -97,25 +99,30 @@ __global__ __launch_bounds__(512) void mma_stream(P p, uint32_t tiles_m, uint32_
     uint32_t ln;
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
 #pragma unroll
-    for (uint32_t i = 0; i < uint32_t(PER); ++i) {
-      const uint32_t r = wave * ROWS + 8 * i + (ln >> 3), c = (ln & 7u) ^ ((r >> 1) & 7u);
-      const uint32_t ra = t.m0 + r < p.m ? r : p.m - 1 - t.m0, rb = t.n0 + r < p.n ? r : p.n - 1 - t.n0;  // rows past the end repeat the last one
+    for (uint32_t i = 0; i < uint32_t(PER_A); ++i) {
+      const uint32_t r = wave * ROWS_A + 8 * i + (ln >> 3), c = (ln & 7u) ^ ((r >> 1) & 7u);
+      const uint32_t ra = t.m0 + r < p.m ? r : p.m - 1 - t.m0;  // rows past the end repeat the last one
       off_a[i] = ra * p.lda + c * 16 + BIAS - 1024 * (i & 3u);
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < uint32_t(PER_B); ++i) {
+      const uint32_t r = wave * ROWS_B + 8 * i + (ln >> 3), c = (ln & 7u) ^ ((r >> 1) & 7u);
+      const uint32_t rb = t.n0 + r < p.n ? r : p.n - 1 - t.n0;
       off_b[i] = rb * p.ldb + c * 16 + BIAS - 1024 * (i & 3u);
     }
   };
-  auto load_piece = [&](int piece, uint32_t stage) {  // pieces 0 .. PER - 1: the first operand's, PER .. 2 PER - 1: the second's
-    const bool second = piece >= PER;
-    const int i = second ? piece - PER : piece;
+  auto load_piece = [&](int piece, uint32_t stage) {  // pieces 0 .. PER_A - 1: the first operand's, then the second's
+    const bool second = piece >= PER_A;
+    const int i = second ? piece - PER_A : piece;
     const uint64_t base = (second ? load_b : load_a) + uint64_t(load_s) * BK;
-    const uint32_t at = lds0 + stage * STAGE + (second ? B_AT : 0u) + wave * (ROWS * BK) + uint32_t(i >> 2) * 4096;
-    const uint32_t offset = second ? off_b[i < PER ? i : 0] : off_a[i < PER ? i : 0];
+    const uint32_t at = lds0 + stage * STAGE + (second ? B_AT + wave * (ROWS_B * BK) : wave * (ROWS_A * BK)) + uint32_t(i >> 2) * 4096;
+    const uint32_t offset = second ? off_b[i < PER_B ? i : 0] : off_a[i < PER_A ? i : 0];
     if constexpr (TAIL) {
       // the last step of a tile: lanes whose chunk lies past k fetch zeros instead (kZeroChunk)
       if (load_s + 1 == steps) {
         uint32_t ln;
         asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
-        const uint32_t c = (ln & 7u) ^ ((4 * i + (ln >> 4)) & 7u);  // (rows 32 wave + 8 i + ln / 8)
+        const uint32_t c = (ln & 7u) ^ ((wave * ((second ? ROWS_B : ROWS_A) / 2) + 4 * i + (ln >> 4)) & 7u);  // (rows ROWS wave + 8 i + ln / 8)
         uint64_t address = base + offset;
         if (load_s * BK + c * 16 >= p.k) address = reinterpret_cast<uint64_t>(&kZeroChunk[0]) - 1024 * (i & 3);
         switch (i & 3) {
@@ -157,7 +164,7 @@ __global__ __launch_bounds__(512) void mma_stream(P p, uint32_t tiles_m, uint32_
   for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
     for (int c = 0; c < 2; ++c) at[kk][c] = (x0 ^ (kk * 64) ^ (c * 16)) + wm * (TM2 * 32 * BK);
-  const uint32_t a_to_b = B_AT + wn * (128 * BK) - wm * (TM2 * 32 * BK);
+  const uint32_t a_to_b = B_AT + wn * (TN2 * 32 * BK) - wm * (TM2 * 32 * BK);
   auto fragment = [&](const uint32_t (&at)[2], uint32_t uniform) {
     const V4I lo = *reinterpret_cast<const V4I*>(lds + uniform + at[0]);
     const V4I hi = *reinterpret_cast<const V4I*>(lds + uniform + at[1]);
@@ -195,7 +202,7 @@ __global__ __launch_bounds__(512) void mma_stream(P p, uint32_t tiles_m, uint32_
   // 8192 x 8192 bfloat16 outputs); with whole lines the count is the output's size.  Non-temporal stores are 1.5 times
   // slower, and waiting after every few stores, or starting the workgroups a few microseconds apart, only costs.
   auto epilogue = [&](const Tile& t) {
-    const uint32_t wm0 = t.m0 + wm * (TM2 * 32), wn0 = t.n0 + wn * 128;
+    const uint32_t wm0 = t.m0 + wm * (TM2 * 32), wn0 = t.n0 + wn * (TN2 * 32);
     typename P::Rows rows[TM2];
 #pragma unroll
     for (int i = 0; i < TM2; ++i) {
@@ -248,11 +255,12 @@ __global__ __launch_bounds__(512) void mma_stream(P p, uint32_t tiles_m, uint32_
       right = upper8 ? right : got;
     };
 #pragma unroll
-    for (int jp = 0; jp < TN2 / 2; ++jp) {
+    for (int jp = 0; jp < (TN2 + 1) / 2; ++jp) {
       Packed left[TM2];
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj) {
         const int j = 2 * jp + jj;
+        if (j >= TN2) break;
         uint32_t first_column[4];  // of this lane's four columns in chunk q of column block j (inside the matrix)
         typename P::Columns4 columns[4];
 #pragma unroll
@@ -265,6 +273,20 @@ __global__ __launch_bounds__(512) void mma_stream(P p, uint32_t tiles_m, uint32_
         for (int i = 0; i < TM2; ++i) {
           if (jj == 0) {
             left[i] = packed_tile(i, j, first_column, columns);
+            if (j + 1 < TN2) continue;
+            // (a last block without a neighbour: 64 bytes of a row per store)
+            const uint32_t n = wn0 + 32 * j + 8 * (2 * ((lane >> 4) & 1u) + h);
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+              const uint32_t mm = wm0 + 32 * i + 16 * half + (lane & 15u);
+              const uint32_t(&w)[4] = left[i].w[half];
+              const bool inside = mm < p.m && n + 8 <= p.n;
+              if (!narrow) {
+                if (inside) p.store8(t.batch, mm, n, U4{w[0], w[1], w[2], w[3]});
+              } else {
+                if (inside) p.store8_narrow(t.batch, mm, n, U2{w[0], w[1]});
+              }
+            }
             continue;
           }
           Packed right = packed_tile(i, j, first_column, columns);
@@ -293,12 +315,12 @@ __global__ __launch_bounds__(512) void mma_stream(P p, uint32_t tiles_m, uint32_
   const uint32_t stream = mine * steps;
   load_setup(0);
 #pragma unroll
-  for (int c = 0; c < 2 * PER; ++c) load_piece(c, 0);
+  for (int c = 0; c < PER; ++c) load_piece(c, 0);
   load_advance();
 #pragma unroll
-  for (int c = 0; c < 2 * PER; ++c) load_piece(c, 1);  // (steps >= 2: a second step always exists)
+  for (int c = 0; c < PER; ++c) load_piece(c, 1);  // (steps >= 2: a second step always exists)
   load_advance();
-  __builtin_amdgcn_s_waitcnt(0x0f70 | (2 * PER));  // vmcnt(2 PER): stage 0 has landed
+  __builtin_amdgcn_s_waitcnt(0x0f70 | PER);  // vmcnt(PER): stage 0 has landed
   __syncthreads();
   V8I a_first[TM2], a_second[TM2], b_first[TN2], b_second[TN2];  // of the first / second half of k (kk = 0 / 1)
   // the fragments of a half step, read between the first TN2 matrix-core instructions of the half step before, in the
@@ -338,9 +360,9 @@ __global__ __launch_bounds__(512) void mma_stream(P p, uint32_t tiles_m, uint32_
     for (int n = 0; n < NM; ++n) {
       const int i = n / TN2, j = n % TN2;
       acc[i][j] = multiply(b_second[j], a_second[i], acc[i][j]);
-      if (n < PER && more) {
-        load_piece(2 * n, stage);
-        load_piece(2 * n + 1, stage);
+      if (more) {
+        if (2 * n < PER) load_piece(2 * n, stage);
+        if (2 * n + 1 < PER) load_piece(2 * n + 1, stage);
       }
       read_fragments(n, a_first, b_first, 0, stage ^ 1u);
       __builtin_amdgcn_sched_barrier(0);
@@ -362,10 +384,10 @@ bool mma_stream_serves(const P& p) {
   return p.k % 16 == 0 && p.k > BK && p.n % 8 == 0 && p.n >= 8 && p.m >= 1 && mma_stream_strides_ok(p.lda, p.ldb);
 }
 
-template <int FA, int FB, int MATH, bool TAIL, class P>
+template <int FA, int FB, int MATH, int BN, bool TAIL, class P>
 int launch_mma_stream_one(const P& p, int compute_units, hipStream_t stream, std::string* err, const char* who) {
-  constexpr uint32_t lds_bytes = 2 * (256 + 256) * BK;
-  auto kernel = mma_stream<FA, FB, MATH, TAIL, P>;
+  constexpr uint32_t lds_bytes = 2 * (256 + BN) * BK;
+  auto kernel = mma_stream<FA, FB, MATH, BN, TAIL, P>;
   static bool configured = false;  // guarded by the runtime's stream mutex
   if (!configured) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess) {
@@ -375,7 +397,7 @@ int launch_mma_stream_one(const P& p, int compute_units, hipStream_t stream, std
     }
     configured = true;
   }
-  const uint32_t tiles_m = (p.m + 255) / 256, tiles_n = (p.n + 255) / 256;
+  const uint32_t tiles_m = (p.m + 255) / 256, tiles_n = (p.n + BN - 1) / BN;
   const uint64_t total = uint64_t(tiles_m) * tiles_n * p.batches;
   if (total * ((p.k + BK - 1) / BK) >= (1ull << 31)) {
     *err = std::string(who) + ": too many tiles";
@@ -387,10 +409,33 @@ int launch_mma_stream_one(const P& p, int compute_units, hipStream_t stream, std
   return 0;
 }
 
+// Columns per tile: 256, or 192 or 128 where they take fewer or fuller rounds of a tile per compute unit.  A round costs about 100,
+// 81 and 64 parts of the same step (4096 x 14336 x 4096 in bfloat16, full rounds: 106, 86 and 64 us each; 4096 x 28672 x 8192 in float8: 102,
+// 83 and 66), and fewer columns read more bytes per product, so a tie goes to the wider tile.  us, 256 / 192 / 128 (rounds): float8 1024 x
+// 8192 x 8192 88 / 77 / 64 (1, 1, 1); 2000 x 10240 x 8192 184 / 155 / 176 (2, 2, 3); 700 x 22016 x 4096 95 / 80 / 90 (2, 2, 3); 4096 x 28672
+// x 8192 712 / 828 / 923 (7, 10, 14); bfloat16 1537 x 13824 x 5120 252 / 218 / 235 (2, 2, 3); 1024 x 14336 x 4096 107 / 149 / 121 (1, 2, 2).
+inline uint32_t mma_stream_columns(uint32_t m, uint32_t n, uint32_t batches, uint32_t cus) {
+  const uint32_t columns[3] = {256, 192, 128}, cost[3] = {100, 81, 64};
+  uint32_t best = 0;
+  uint64_t best_cost = 0;
+  for (int i = 0; i < 3; ++i) {
+    const uint64_t tiles = uint64_t((m + 255) / 256) * ((n + columns[i] - 1) / columns[i]) * batches;
+    const uint64_t c = (tiles + cus - 1) / cus * cost[i];
+    if (best == 0 || c < best_cost) best = columns[i], best_cost = c;
+  }
+  return best;
+}
+
+// forced: 1, 2, 3 for 256, 192, 128 columns per tile (tests, tuning), 0: planned.
 template <int FA, int FB, int MATH, class P>
-int launch_mma_stream(const P& p, int compute_units, hipStream_t stream, std::string* err, const char* who) {
-  return p.k % BK == 0 ? launch_mma_stream_one<FA, FB, MATH, false>(p, compute_units, stream, err, who)
-                       : launch_mma_stream_one<FA, FB, MATH, true>(p, compute_units, stream, err, who);
+int launch_mma_stream(const P& p, uint32_t forced, int compute_units, hipStream_t stream, std::string* err, const char* who) {
+  const uint32_t columns = forced ? 320 - 64 * forced : mma_stream_columns(p.m, p.n, p.batches, uint32_t(compute_units));
+  const bool tail = p.k % BK != 0;
+#define VKT_STREAM(BN)                                                                          \
+  (tail ? launch_mma_stream_one<FA, FB, MATH, BN, true>(p, compute_units, stream, err, who) \
+        : launch_mma_stream_one<FA, FB, MATH, BN, false>(p, compute_units, stream, err, who))
+  return columns == 256 ? VKT_STREAM(256) : columns == 192 ? VKT_STREAM(192) : VKT_STREAM(128);
+#undef VKT_STREAM
 }
 
 }  // namespace
