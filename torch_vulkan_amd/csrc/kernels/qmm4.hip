@@ -999,12 +999,9 @@ __global__ __launch_bounds__(256) void qmm4m_rows(Q4CParams p, MatrixLayout L, u
   }
   const long minus8 = long(0xf8f8f8f8f8f8f8f8ull);
   const V4I minus8x4 = V4I{int(0xf8f8f8f8u), int(0xf8f8f8f8u), int(0xf8f8f8f8u), int(0xf8f8f8f8u)};
-  V4I nz_a4[RT], nz_b4[RT];
-#pragma unroll
-  for (int t = 0; t < RT; ++t) {
-    nz_a4[t] = V4I{int(nz_a[t]), int(nz_a[t]), int(nz_a[t]), int(nz_a[t])};
-    nz_b4[t] = V4I{int(nz_b[t]), int(nz_b[t]), int(nz_b[t]), int(nz_b[t])};
-  }
+  const V4I ones = V4I{0x01010101, 0x01010101, 0x01010101, 0x01010101};
+  const V4I nz_a4 = V4I{int(nz_a[0]), int(nz_a[0]), int(nz_a[0]), int(nz_a[0])};  // (one tile per wave)
+  const V4I nz_b4 = V4I{int(nz_b[0]), int(nz_b[0]), int(nz_b[0]), int(nz_b[0])};
   uint64_t wbase[CT], sbase[CT];
 #pragma unroll
   for (int c = 0; c < CT; ++c) {
@@ -1036,12 +1033,16 @@ __global__ __launch_bounds__(256) void qmm4m_rows(Q4CParams p, MatrixLayout L, u
   for (int i = 0; i < kRowsAhead; ++i) request(sets[i], i);
 
   float acc[RT][CT][4];
-  V4I d[RT][CT], d2[RT][CT];
+  V4I d[RT][CT], row_sum[RT], col_sum[CT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) row_sum[t] = V4I{0, 0, 0, 0};
+#pragma unroll
+  for (int c = 0; c < CT; ++c) col_sum[c] = V4I{0, 0, 0, 0};
 #pragma unroll
   for (int t = 0; t < RT; ++t)
 #pragma unroll
     for (int c = 0; c < CT; ++c) {
-      d[t][c] = d2[t][c] = V4I{0, 0, 0, 0};
+      d[t][c] = V4I{0, 0, 0, 0};
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[t][c][r] = -0.0f;
     }
@@ -1078,8 +1079,12 @@ __global__ __launch_bounds__(256) void qmm4m_rows(Q4CParams p, MatrixLayout L, u
           }
         }
       } else {
-        // Blocks of two units and more: two units, 64 values of k, per matrix-core instruction (the full-rate form),
-        // and the zero-point products as a chain of their own (integers: any order).
+        // Blocks of two units and more: two units, 64 values of k, per matrix-core instruction (the full-rate form).  The sums of
+        // a row's values times -8 are the same for all column tiles, the sums of a column's nibbles, which the zero points
+        // multiply once per block, the same for all row tiles: one product of each per tile of its side (integers: any order).
+        // 8 products for 2 x 2 tiles; as chains per tile, the zero point in two halves, they were 16 (us, 2048 x 4096 x 11008 in blocks of
+        // 128 492 -> 418, channelwise 425 -> 335; 1024 x 8192 x 8192 channelwise 263 -> 197).  One tile per wave shares nothing and keeps
+        // the chains: 4 products, but no integer work for the vector unit (64 x 11008 x 4096 in blocks of 64: 27 against 39 us).
 #pragma unroll
         for (int j = 0; j < 4; j += 2) {
           const int u = i * 4 + j;
@@ -1089,27 +1094,34 @@ __global__ __launch_bounds__(256) void qmm4m_rows(Q4CParams p, MatrixLayout L, u
           for (int c = 0; c < CT; ++c) {
             const uint32_t v0 = cur.w[c][j], v1 = cur.w[c][j + 1];
             b[c] = V4I{int(v0 & 0x0f0f0f0fu), int((v0 >> 4) & 0x0f0f0f0fu), int(v1 & 0x0f0f0f0fu), int((v1 >> 4) & 0x0f0f0f0fu)};
+            if constexpr (RT * CT > 1) col_sum[c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, b[c], first ? V4I{0, 0, 0, 0} : col_sum[c], 0, 0, 0);
           }
 #pragma unroll
           for (int t = 0; t < RT; ++t) {
             const U4& qq = j < 2 ? cur.q0[t] : cur.q1[t];
             const V4I a = V4I{int(qq[0]), int(qq[1]), int(qq[2]), int(qq[3])};
-#pragma unroll
-            for (int c = 0; c < CT; ++c) {
-              V4I x = first ? unit_const[t] * (UPB ? UPB : 1) : d[t][c];
-              V4I y = first ? V4I{0, 0, 0, 0} : d2[t][c];
-              x = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b[c], x, 0, 0, 0);
-              y = __builtin_amdgcn_mfma_i32_16x16x64_i8(nz_a4[t], b[c], y, 0, 0, 0);
-              x = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, minus8x4, x, 0, 0, 0);
-              y = __builtin_amdgcn_mfma_i32_16x16x64_i8(nz_b4[t], b[c], y, 0, 0, 0);
-              d2[t][c] = y;
-              if (last) {  // the block's term, added in block order
-                x = x + y;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[t][c][r] = acc[t][c][r] + float(x[r]) * cur.s[c][j + 1];
-              }
-              d[t][c] = x;
+            if constexpr (RT * CT == 1) {
+              V4I x = first ? unit_const[0] * (UPB ? UPB : 1) : d[0][0], y = first ? V4I{0, 0, 0, 0} : row_sum[0];
+              x = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b[0], x, 0, 0, 0);
+              y = __builtin_amdgcn_mfma_i32_16x16x64_i8(nz_a4, b[0], y, 0, 0, 0);
+              d[0][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, minus8x4, x, 0, 0, 0);
+              row_sum[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(nz_b4, b[0], y, 0, 0, 0);  // (here the zero-point products)
+              continue;
             }
+            row_sum[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, minus8x4, first ? unit_const[t] * (UPB ? UPB : 1) : row_sum[t], 0, 0, 0);
+#pragma unroll
+            for (int c = 0; c < CT; ++c) d[t][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b[c], first ? V4I{0, 0, 0, 0} : d[t][c], 0, 0, 0);
+          }
+          if (last) {  // the blocks' terms, added in block order
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+#pragma unroll
+              for (int c = 0; c < CT; ++c)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                  const int sum = d[t][c][r] + row_sum[t][r] + (RT * CT > 1 ? __mul24(nzp_r[t][r], col_sum[c][r]) : 0);
+                  acc[t][c][r] = acc[t][c][r] + float(sum) * cur.s[c][j + 1];
+                }
           }
         }
       }
@@ -1140,7 +1152,7 @@ __global__ __launch_bounds__(256) void qmm4m_rows(Q4CParams p, MatrixLayout L, u
         const uint32_t m = row0 + 16 * t + kg * 4 + r;
         if (m >= p.m) continue;
         float v = acc[t][c][r];
-        if constexpr (UPB == 0) v = float(d[t][c][r] + d2[t][c][r] - 256 * nzp_r[t][r] * int(L.quads * 4)) * s;
+        if constexpr (UPB == 0) v = float(d[t][c][r] + row_sum[t][r] + nzp_r[t][r] * (col_sum[c][r] - 256 * int(L.quads * 4))) * s;
         finish_store<T>(p.out + (uint64_t(m) * p.n + n) * item, v, bits_f32(ldg<uint32_t>(p.rows + 8ull * m)), p.has_bias != 0, bias);
       }
   }
@@ -1591,9 +1603,11 @@ int launch_matrix(const Q4CParams& p, uint32_t phase_and_flags, uint32_t groupwi
     for (uint32_t m0 = 0; rows_kernel && m0 < p.m; m0 += 16 * 1024) {
       const uint32_t rows = p.m - m0 < 16 * 1024 ? p.m - m0 : 16 * 1024;
       uint32_t shape = (flags >> 6) & 3u;
+      // (the largest wave tile that leaves every SIMD two and a half waves, two for 2 x 1: 90 x 11008 x 4096 in blocks of 128 as 2064 waves of
+      //  2 x 1 takes 37 us, as 4128 of 1 x 1 42)
       if (M.upb == 1 || M.upb == 2) shape = 1;  // (the float16 form has more tiles per wave)
       else if (shape == 0)
-        shape = uint64_t((rows + 31) / 32) * ((M.tiles + 1) / 2) >= 2560 ? 3 : uint64_t((rows + 31) / 32) * M.tiles >= 2560 ? 2 : 1;
+        shape = uint64_t((rows + 31) / 32) * ((M.tiles + 1) / 2) >= 2560 ? 3 : uint64_t((rows + 31) / 32) * M.tiles >= 2048 ? 2 : 1;
       const int rc = shape == 3 ? launch_rows<T, 2, 2>(p, M, m0, rows, stream)
                    : shape == 2 ? launch_rows<T, 2, 1>(p, M, m0, rows, stream)
                                 : launch_rows<T, 1, 1>(p, M, m0, rows, stream);
