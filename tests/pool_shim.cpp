@@ -94,4 +94,7 @@ uint64_t shim_k_slices(uint32_t chunks, uint32_t wanted) {
   return uint64_t(s.slices) | uint64_t(s.chunks_per_slice) << 32;
 }
 
+// the byte of a row that a lane of the register-staged tile kernel loads (kernels/limits.h)
+uint32_t shim_tile_chunk_at(uint32_t k_bytes, uint32_t step, uint32_t chunk) { return vkt::tile_chunk_at(k_bytes, step, chunk); }
+
 }  // extern "C"

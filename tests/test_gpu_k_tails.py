@@ -65,11 +65,31 @@ def test_uneven_slices(dtype, layout, k, variant):
 
 @pytest.mark.parametrize("k", [144, 176, 1040, 2112])
 @pytest.mark.parametrize("variant,out", [(0, torch.bfloat16), (8, torch.bfloat16), (5, torch.float8_e4m3fn), (11, torch.bfloat16),
-                                         (11, torch.float8_e5m2), (6, torch.float32), (9, torch.float16), (14 | 3 << 8, torch.bfloat16)])
+                                         (11, torch.float8_e5m2), (6, torch.float32), (9, torch.float16), (14 | 3 << 8, torch.bfloat16),
+                                         (14 | 3 << 8, torch.float32), (14 | 3 << 8, torch.float16)])
 def test_float8(k, variant, out):
     if variant >> 8 and k < 1024:
         pytest.skip("shorter than three slices of 128 bytes")
     run_case(300, k, 264, FLOAT8[0], FLOAT8[1], out, True, torch.float32, None if out.itemsize > 1 else 2.0, variant=variant, seed=k)
+
+
+@pytest.mark.parametrize("out", [torch.bfloat16, torch.float32, torch.float16, torch.float8_e4m3fn])
+def test_float8_last_slice_shorter_than_a_step(out):
+    """Planned: 16 slices of 9 steps, the last of them 64 bytes."""
+    run_case(100, 17344, 520, FLOAT8[0], FLOAT8[1], out, True, torch.float32, None if out.itemsize > 1 else 2.0, seed=17)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+def test_last_slice_shorter_than_a_step(dtype, layout):
+    """The same for 16-bit operands, whose rows go on with NaN."""
+    import _dev
+    m, k, n = 100, 8672, 264
+    a = bits((torch.randn(m, k, generator=gen(32)) * 0.5).to(dtype))
+    w = bits((torch.randn(n, k, generator=gen(33)) * 0.5).to(dtype))
+    want, mag = oracle.gemm16(a, w.T, ODT[dtype], want_mag=True)
+    wide = lambda x: np.concatenate([x, np.full((x.shape[0], 64), 0x7FC1 if dtype == torch.bfloat16 else 0x7E01, np.uint16)], 1)[:, :x.shape[1]]  # noqa: E731
+    close(_dev.gemm16(wide(a), wide(w).T if layout == "nt" else wide(np.ascontiguousarray(w.T)), ODT[dtype]), want, mag, dtype)
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=str)

@@ -207,3 +207,29 @@ def test_k_slices_leave_no_slice_empty():
             assert (slices - 1) * per < chunks <= slices * per, (chunks, wanted, slices, per)
     r = L.shim_k_slices(65, 16)
     assert (r & 0xffffffff, r >> 32) == (13, 5)
+
+
+def test_tile_loads_stay_inside_their_rows():
+    """Every 16-byte load of the register-staged tile kernel lies inside the k bytes of its row: rows from 16 bytes on, whole or
+    in slices of K of whole 128-byte steps, whose last one may be shorter than a step (17344 bytes in 16 slices of 9 steps: the
+    last holds 64 bytes); where the lane's own 16 bytes exist it loads those."""
+    L = ctypes.CDLL(os.path.join(os.path.dirname(abi.LIB_PATH), "libvkt_hosttest.so"))
+    L.shim_k_slices.argtypes = [ctypes.c_uint32, ctypes.c_uint32]
+    L.shim_k_slices.restype = ctypes.c_uint64
+    L.shim_tile_chunk_at.argtypes = [ctypes.c_uint32] * 3
+    L.shim_tile_chunk_at.restype = ctypes.c_uint32
+    seen_short = 0
+    for k in list(range(16, 4400, 16)) + [17296, 17344, 17392, 19264, 30832]:
+        steps = (k + 127) // 128
+        for wanted in range(1, 17):
+            r = L.shim_k_slices(steps, wanted)
+            slices, length = r & 0xffffffff, (r >> 32) * 128
+            begin = (slices - 1) * length  # the last slice; the others are whole steps
+            here = min(length, k - begin)
+            seen_short += begin > 0 and here < 128
+            for step in range(here // 128 * 128, here, 128):  # (whole steps are loaded as they are)
+                for chunk in range(0, 128, 16):
+                    at = L.shim_tile_chunk_at(here, step, chunk)
+                    assert begin + at + 16 <= k, (k, wanted, step, chunk, at)
+                    assert at == step + chunk or step + chunk >= here
+    assert seen_short

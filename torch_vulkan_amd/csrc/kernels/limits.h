@@ -24,4 +24,13 @@ constexpr KSlices k_slices(uint32_t chunks, uint32_t wanted) {
   return KSlices{chunks ? (chunks + per - 1) / per : 1, per};
 }
 
+// The register-staged tile kernel brings 16 bytes per lane and step: `chunk` bytes into a step of 128 that begins `step`
+// bytes into the row (or into the row's slice of K).  Where that lies past the row's k bytes (the last step of a k that
+// is no multiple of 128) the lane puts zeros into LDS, but it loads all the same, so that no branch stands before the
+// loads: the row's first 16 bytes.  (Not chunk `chunk` of the first step: a row or a slice can be shorter than that.)
+// k_bytes: a multiple of 16, at least 16.  What it returns is a byte offset into the row, at most k_bytes - 16.
+constexpr uint32_t tile_chunk_at(uint32_t k_bytes, uint32_t step, uint32_t chunk) {
+  return step + chunk < k_bytes ? step + chunk : 0;
+}
+
 }  // namespace vkt

@@ -27,6 +27,7 @@
 #include <string>
 
 #include "common.h"
+#include "limits.h"
 
 namespace vkt {
 namespace {
@@ -138,7 +139,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
 
   // global -> register staging: chunk id = tid + NT * i -> (row, chunk)
   uint64_t a_src[A_CHUNKS], b_src[B_CHUNKS];
-  uint32_t a_dst[A_CHUNKS], b_dst[B_CHUNKS], a_k[A_CHUNKS], b_k[B_CHUNKS];
+  uint32_t a_dst[A_CHUNKS], b_dst[B_CHUNKS];
 #pragma unroll
   for (int i = 0; i < A_CHUNKS; ++i) {
     // DIRECT: the load lands at LDS slot id (lane order), so the lane fetches the logical
@@ -148,14 +149,13 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
       const uint32_t id = tid + NT * i, row = id / (BM / 8), c = (id % (BM / 8)) ^ ((row & 3u) << 2);
       const uint32_t mc = m0 / 8 + c < p.m / 8 ? m0 / 8 + c : p.m / 8 - 1;
       a_src[i] = a_base + uint64_t(row) * p.lda + mc * 16;
-      a_dst[i] = 0, a_k[i] = 0;
+      a_dst[i] = 0;
       continue;
     }
     const uint32_t id = tid + NT * i, row = id >> 3, c = DIRECT ? (id & 7u) ^ ((row >> 1) & 7u) : id & 7u;
     const uint32_t m = m0 + row < p.m ? m0 + row : p.m - 1;
     a_src[i] = a_base + uint64_t(m) * p.lda + c * 16;
     a_dst[i] = tile_offset(row, c);
-    a_k[i] = c * 16;
   }
 #pragma unroll
   for (int i = 0; i < B_CHUNKS; ++i) {
@@ -163,14 +163,13 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
       const uint32_t id = tid + NT * i, row = id / (BN / 8), c = (id % (BN / 8)) ^ ((row & 3u) << 2);
       const uint32_t nc = n0 / 8 + c < p.n / 8 ? n0 / 8 + c : p.n / 8 - 1;
       b_src[i] = b_base + uint64_t(row) * p.ldb + nc * 16;
-      b_dst[i] = 0, b_k[i] = 0;
+      b_dst[i] = 0;
       continue;
     }
     const uint32_t id = tid + NT * i, row = id >> 3, c = DIRECT ? (id & 7u) ^ ((row >> 1) & 7u) : id & 7u;
     const uint32_t n = n0 + row < p.n ? n0 + row : p.n - 1;
     b_src[i] = b_base + uint64_t(n) * p.ldb + c * 16;
     b_dst[i] = BM * BK + tile_offset(row, c);
-    b_k[i] = c * 16;
   }
 
   // MF32: the wave's sub-tile as (TM/2) x (TN/2) tiles of 32x32 (V_MFMA_F32_32X32X64_F8F6F4,
@@ -213,10 +212,10 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
   };
   auto load_chunk_tail = [&](int c, uint32_t k0) {
     const uint64_t src = c < A_CHUNKS ? a_src[c < A_CHUNKS ? c : 0] : b_src[c < A_CHUNKS ? 0 : c - A_CHUNKS];
-    const uint32_t kc = c < A_CHUNKS ? a_k[c < A_CHUNKS ? c : 0] : b_k[c < A_CHUNKS ? 0 : c - A_CHUNKS];
-    const bool inside = k0 + kc < k_bytes;
-    const V4I v = ldg<V4I>(src + (inside ? k0 : 0));  // (k >= 16: chunk 0 of the row exists)
-    reg[c] = inside ? v : zero;
+    const uint32_t kc = (uint32_t(tid) & 7u) * 16;  // the chunk's place in its step, which src holds (NT is a multiple of 8: the same for all chunks)
+    const int64_t at = int32_t(tile_chunk_at(k_bytes, k0, kc)) - int32_t(kc);
+    const V4I v = ldg<V4I>(src + at);
+    reg[c] = k0 + kc < k_bytes ? v : zero;
   };
   const uint32_t full_steps = k_bytes / BK;  // steps whose 128 bytes all lie inside k
   auto load_step = [&](int c, uint32_t step) {
