@@ -111,14 +111,32 @@ def test_q4_several_tiles_per_workgroup(m, k, n, bs, bias):
 @pytest.mark.parametrize("m,k,n,bs", [(5, 32, 16, 32), (33, 96, 145, 32), (64, 2112, 520, 64), (47, 4096, 129, 32), (97, 64, 257, 64),
                                       (1030, 16384, 20, 32)])  # (the last: more rows than the workspace holds, in two pieces)
 @pytest.mark.parametrize("flags", [32 | 128, 32 | 192])
-def test_q4_float16_products(m, k, n, bs, flags):
+@pytest.mark.parametrize("bias", [True, False])
+def test_q4_float16_products(m, k, n, bs, flags, bias):
     """Blocks of 32 and 64 on the kernel that multiplies in float16: whole numbers, so the oracle's bits.  Rows at the ends of
     the quantised range (zero point -128 and 127: differences up to 255) against nibbles of 0 and 15 make its largest sums."""
     import _dev
-    w, sc, bvec = int4_weights(n, k, bs, bias=True)
+    w, sc, bvec = int4_weights(n, k, bs, bias=bias)
     w[0::3], w[1::3] = 0xff, 0x00
     x = int4_rows(m, k, torch.float32)
-    x[0], x[1], x[2::5] = 3.0, -3.0, x[2::5].abs()
+    x[0], x[1], x[2::5], x[4] = 3.0, -3.0, x[2::5].abs(), 0.0  # (the zero row, without a bias: the sign of the sums' zeros)
+    packed = torch._dyn_quant_pack_4bit_weight(w, sc, bvec, bs, k, n).numpy()
+    want = oracle.q4_matmul(bits(x), oracle.F32, packed, bs, k, n)
+    cm = _dev.CompactWeights(packed, bs, k, n, layout=1)
+    for fused in (True, False):
+        got = _dev.q4_compact(bits(x), oracle.F32, cm, fused=fused, flags=flags)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), fused
+
+
+@pytest.mark.parametrize("m,k,n,bs", [(33, 2304, 145, 256), (47, 6400, 40, 256), (65, 6400, 33, 128), (33, 6176, 49, 6176)])
+@pytest.mark.parametrize("flags", [32 | 64, 32 | 128, 32 | 192])
+def test_q4_several_tiles_per_wave(m, k, n, bs, flags):
+    """Blocks of 128 and 256 values and one scale per row over more than one round of 2048 values of k, tile counts that leave the
+    last wave short: the oracle's bits."""
+    import _dev
+    w, sc, bvec = int4_weights(n, k, bs, bias=False)
+    x = int4_rows(m, k, torch.float32)
+    x[2], x[3], x[4] = 3.0, -3.0, 0.0
     packed = torch._dyn_quant_pack_4bit_weight(w, sc, bvec, bs, k, n).numpy()
     want = oracle.q4_matmul(bits(x), oracle.F32, packed, bs, k, n)
     cm = _dev.CompactWeights(packed, bs, k, n, layout=1)

@@ -1029,8 +1029,16 @@ __global__ __launch_bounds__(256) void qmm4m_rows(Q4CParams p, MatrixLayout L, u
       if constexpr (UPB != 0) set.s[c] = ldg<F4>(sbase[c] + quad * sstep);
     }
   };
+  // Blocks of 256 with several tiles per wave: a quad's registers take the quad after next only once they are used up, and nothing moves
+  // across the requests.  Left to itself the scheduler puts these loops' loads next to their use (the chains are short, and it aims at one
+  // more wave per SIMD), five waits for memory per two quads.  us, before the shared sums / with them / with them and in place: 512 x
+  // 4096 x 11008 129 / 143 / 103, 512 x 8192 x 11008 246 / 269 / 200, 96 x 4096 x 28672 60 / 64 / 49, 2048 x 4096 x 11008 489 / 451 / 379.
+  constexpr bool kInPlace = UPB == 8 && RT * CT > 1;
 #pragma unroll
-  for (int i = 0; i < kRowsAhead; ++i) request(sets[i], i);
+  for (int i = 0; i < kRowsAhead; ++i) {
+    request(sets[i], i);
+    if constexpr (kInPlace) __builtin_amdgcn_sched_barrier(0);
+  }
 
   float acc[RT][CT][4];
   V4I d[RT][CT], row_sum[RT], col_sum[CT];
@@ -1050,8 +1058,12 @@ __global__ __launch_bounds__(256) void qmm4m_rows(Q4CParams p, MatrixLayout L, u
   for (uint32_t quad0 = 0; quad0 < L.quads; quad0 += kRowsAhead) {
 #pragma unroll
     for (int i = 0; i < kRowsAhead; ++i) {
-      const Set cur = sets[i];
-      request(sets[i], quad0 + i + kRowsAhead);
+      Set taken;
+      if constexpr (!kInPlace) {
+        taken = sets[i];
+        request(sets[i], quad0 + i + kRowsAhead);
+      }
+      const Set& cur = kInPlace ? sets[i] : taken;
       constexpr int mask = UPB ? UPB - 1 : 0;
       if constexpr (UPB == 1) {
 #pragma unroll
@@ -1124,6 +1136,11 @@ __global__ __launch_bounds__(256) void qmm4m_rows(Q4CParams p, MatrixLayout L, u
                 }
           }
         }
+      }
+      if constexpr (kInPlace) {
+        __builtin_amdgcn_sched_barrier(0);
+        request(sets[i], quad0 + i + kRowsAhead);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
     // The four matrix-core instructions of a unit are a dependent chain, 16 cycles apart: with one tile per wave the
