@@ -7,6 +7,7 @@
 #include <string>
 
 #include "limits.h"
+#include "plans.h"
 #include "pool.h"
 
 namespace {
@@ -96,5 +97,10 @@ uint64_t shim_k_slices(uint32_t chunks, uint32_t wanted) {
 
 // the byte of a row that a lane of the register-staged tile kernel loads (kernels/limits.h)
 uint32_t shim_tile_chunk_at(uint32_t k_bytes, uint32_t step, uint32_t chunk) { return vkt::tile_chunk_at(k_bytes, step, chunk); }
+
+// which wave tile a many-row 4-bit product runs on (kernels/plans.h: Q4Form)
+uint32_t shim_q4_rows_form(uint32_t m, uint32_t tiles, uint32_t quads, uint32_t upb, uint32_t simds) {
+  return vkt::q4_rows_form(m, tiles, quads, upb, simds);
+}
 
 }  // extern "C"

@@ -233,3 +233,21 @@ def test_tile_loads_stay_inside_their_rows():
                     assert begin + at + 16 <= k, (k, wanted, step, chunk, at)
                     assert at == step + chunk or step + chunk >= here
     assert seen_short
+
+
+def _q4_form(m, k, n, bs):
+    L = ctypes.CDLL(os.path.join(os.path.dirname(abi.LIB_PATH), "libvkt_hosttest.so"))
+    L.shim_q4_rows_form.argtypes = [ctypes.c_uint32] * 5
+    quads = (k + 2047) // 2048 * 16
+    return {1: "1x1", 2: "2x1", 3: "2x2", 4: "half 2x2", 5: "half 2x4"}[L.shim_q4_rows_form(m, (n + 15) // 16, quads, 0 if bs == k else bs // 32, 1024)]
+
+
+@pytest.mark.parametrize("bs", [128, 0])
+def test_q4_wave_tiles_count_real_rows(bs):
+    """4-bit products in blocks of 128 and with one scale per column: rows that only fill a pair of 16-row tiles up do not
+    make the wave tile of two rows pay (70 rows are 5 tiles of 16, not 6; 33 to 48 are 3, not 4)."""
+    for m, k, n in [(70, 4096, 11008), (80, 8192, 11008), (33, 4096, 16384), (48, 2048, 16384), (100, 2048, 8192), (128, 2048, 8192)]:
+        assert _q4_form(m, k, n, bs or k) == "1x1", (m, k, n)
+    for m, k, n in [(96, 4096, 11008), (90, 4096, 11008), (70, 4096, 16384), (150, 4096, 8192)]:
+        assert _q4_form(m, k, n, bs or k) == "2x1", (m, k, n)
+    assert _q4_form(300, 4096, 11008, bs or k) == "2x2" and _q4_form(64, 4096, 11008, bs or k) == "1x1"

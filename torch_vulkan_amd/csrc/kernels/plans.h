@@ -1,0 +1,37 @@
+// Which form of a kernel a launcher picks for a shape, as functions of sizes alone (plain C++: the host test shim includes
+// this too).  Each line between two forms stands where both were measured; the figures stand with it.
+#pragma once
+
+#include <stdint.h>
+
+namespace vkt {
+
+// ---- 4-bit products of many rows (qmm4m_rows, qmm4m_half): a wave owns 1 x 1, 2 x 1 or 2 x 2 matrix-core tiles of 16 x 16 outputs
+// (rows x columns) in integers, or 2 x 2 or 2 x 4 in float16 (blocks of 32 and 64).
+enum Q4Form { kQ4Int11 = 1, kQ4Int21 = 2, kQ4Int22 = 3, kQ4Half22 = 4, kQ4Half24 = 5 };
+
+// tiles: column tiles; quads: 128s of k, padded to 16s; upb: 32s of k per block (0: one scale per column); simds: of the machine.
+constexpr Q4Form q4_rows_form(uint32_t m, uint32_t tiles, uint32_t quads, uint32_t upb, uint32_t simds) {
+  const uint64_t rows16 = (uint64_t(m) + 15) / 16, rows32 = (uint64_t(m) + 31) / 32;
+  const uint64_t int11 = rows16 * tiles, int21 = rows32 * tiles, int22 = rows32 * ((uint64_t(tiles) + 1) / 2);  // waves of each
+  const uint64_t half22 = int22, half24 = rows32 * ((uint64_t(tiles) + 3) / 4);
+  if (upb == 1 || upb == 2) {
+    (void)quads;
+    // Fewer waves of 2 x 2 than four for every five SIMDs: the integer kernel (us at blocks of 32, waves of 2 x 2 in brackets: 128 x 11008
+    // x 4096 [512] integers 59, float16 67; 64 x 4096 x 11008 [688] 30, 30; 256 x 4096 x 4096 [1024] 36.5, 34; 128 x 4096 x 11008
+    // [1376] 50, 43.5; 64 x 4096 x 28672 [1792] 61, 45).  2 x 4 from three waves for two SIMDs on (128 x 4096 x 11008 [688 of 2 x 4] 48.5 against
+    // 43.5; 64 x 4096 x 28672 [896] 49.5, 45; 100 x 4096 x 27777 in blocks of 64 [1738] 67, 80; 512 x 4096 x 11008 [2752] 108, 110).
+    const bool halves = half22 * 5 >= uint64_t(simds) * 4;
+    return !halves ? kQ4Int11 : half24 * 2 >= uint64_t(simds) * 3 ? kQ4Half24 : kQ4Half22;
+  }
+  // The largest tile that leaves every SIMD two and a half waves.  2 x 1: also from two waves on (90 x 4096 x 11008 in blocks of 128 as 2064 waves
+  // of 2 x 1 37 us, as 4128 of 1 x 1 42), but rows that a pair of tiles pads do not count: up to four waves of 1 x 1 per SIMD fit it at
+  // once, and 2 x 1 pays from there on (us, 1 x 1 / 2 x 1, waves of 1 x 1 in brackets: blocks of 128, 40 x 4096 x 16384 [3072] 23.5 / 28.7, 70 x
+  // 8192 x 11008 [3440] 63 / 67, 128 x 2048 x 8192 [4096] 15.9 / 16.9, 128 x 4096 x 8192 [4096] 28.6 / 27.8, 96 x 4096 x 11008 [4128] 38.9 / 33.2;
+  // one scale per column, 40 x 4096 x 16384 23.5 / 25.4, 128 x 2048 x 8192 13.1 / 13.5, 96 x 4096 x 11008 28.6 / 27.9).  Blocks of 256: 2 x 1 is
+  // level from two waves of it per SIMD on (40 x 4096 x 16384 20.9 / 21.0, 70 x 4096 x 11008 29.9 / 29.6, 100 x 4096 x 8192 25.1 / 19.8).
+  if (int22 >= 2560) return kQ4Int22;
+  return (upb == 8 ? int21 >= 2048 : int11 > 4096) ? kQ4Int21 : kQ4Int11;
+}
+
+}  // namespace vkt

@@ -38,6 +38,7 @@
 
 #include "common.h"
 #include "kernels.h"
+#include "plans.h"
 
 namespace vkt {
 namespace {
@@ -1582,19 +1583,15 @@ int launch_matrix(const Q4CParams& p, uint32_t phase_and_flags, uint32_t groupwi
   // one-row-tile kernel, whose four waves split K.  Phase values 1 | 2 with bit 4 (16) set keep the one-row-tile
   // kernel, with bit 5 (32) force the wave-per-tile kernels (tests, tuning; flag bits 6-7 choose among those).
   const bool rows_kernel = ((uint64_t((p.m + 15) / 16) * M.tiles >= (M.upb ? 2048u : 2560u) && !(flags & 16)) || (flags & 32));
-  // Blocks of 32 and 64, many tiles: the products in float16 (qmm4m_half), 2 x 4 or 2 x 2 tiles per wave, against a workspace that
-  // holds the rows' values, in pieces of rows that fit it.  Fewer waves than four for every five SIMDs of 2 x 2: the integer kernel, a
-  // wave per tile (us at blocks of 32, waves of 2 x 2 in brackets: 128 x 11008 x 4096 [512] integers 59, float16 67; 64 x 4096 x
-  // 11008 [688] 30, 30; 256 x 4096 x 4096 [1024] 36.5, 34; 128 x 4096 x 11008 [1376] 50, 43.5; 64 x 4096 x 28672 [1792] 61, 45).
-  // 2 x 4 from three waves for two SIMDs on (128 x 4096 x 11008 [688 of 2 x 4] 48.5 against 43.5; 64 x 4096 x 28672 [896] 49.5, 45;
-  // 100 x 4096 x 27777 in blocks of 64 [1738] 67, 80; 512 x 4096 x 11008 [2752] 108, 110).
+  // Blocks of 32 and 64, many tiles: the products in float16 (qmm4m_half), against a workspace that holds the rows' values, in
+  // pieces of rows that fit it (none where it does not hold 64 rows).
   const uint64_t row_bytes = uint64_t(M.quads) * 256;
-  const uint64_t row_pairs = (uint64_t(p.m) + 31) / 32, simds = uint64_t(mc.compute_units) * 4;
   uint32_t piece = uint32_t((mc.workspace_bytes / row_bytes < 16384 ? mc.workspace_bytes / row_bytes : 16384) & ~63ull);
   const uint32_t asked = (flags & 32) ? (flags >> 6) & 3u : 0;
-  const bool eight = asked ? asked == 3 : row_pairs * ((M.tiles + 3) / 4) * 2 >= simds * 3;
-  const bool halves = (M.upb == 1 || M.upb == 2) && rows_kernel && piece >= 64 &&
-                      (asked ? asked >= 2 : row_pairs * ((M.tiles + 1) / 2) * 5 >= simds * 4);
+  const bool half_blocks = M.upb == 1 || M.upb == 2;
+  const uint32_t simds = uint32_t(mc.compute_units) * 4;
+  const Q4Form form = asked ? Q4Form(half_blocks && asked >= 2 ? asked + 2 : half_blocks ? 1 : asked) : q4_rows_form(p.m, M.tiles, M.quads, M.upb, simds);
+  const bool halves = rows_kernel && piece >= 64 && (form == kQ4Half22 || form == kQ4Half24), eight = form == kQ4Half24;
   if (halves && phase != 0) {
     const uint32_t pieces = (p.m + piece - 1) / piece;
     piece = ((p.m + pieces - 1) / pieces + 63) & ~63u;  // (of about equal size)
@@ -1620,11 +1617,8 @@ int launch_matrix(const Q4CParams& p, uint32_t phase_and_flags, uint32_t groupwi
     for (uint32_t m0 = 0; rows_kernel && m0 < p.m; m0 += 16 * 1024) {
       const uint32_t rows = p.m - m0 < 16 * 1024 ? p.m - m0 : 16 * 1024;
       uint32_t shape = (flags >> 6) & 3u;
-      // (the largest wave tile that leaves every SIMD two and a half waves, two for 2 x 1: 90 x 11008 x 4096 in blocks of 128 as 2064 waves of
-      //  2 x 1 takes 37 us, as 4128 of 1 x 1 42)
-      if (M.upb == 1 || M.upb == 2) shape = 1;  // (the float16 form has more tiles per wave)
-      else if (shape == 0)
-        shape = uint64_t((rows + 31) / 32) * ((M.tiles + 1) / 2) >= 2560 ? 3 : uint64_t((rows + 31) / 32) * M.tiles >= 2048 ? 2 : 1;
+      if (half_blocks) shape = 1;  // (the float16 form has more tiles per wave)
+      else if (shape == 0) shape = q4_rows_form(rows, M.tiles, M.quads, M.upb, simds);
       const int rc = shape == 3 ? launch_rows<T, 2, 2>(p, M, m0, rows, stream)
                    : shape == 2 ? launch_rows<T, 2, 1>(p, M, m0, rows, stream)
                                 : launch_rows<T, 1, 1>(p, M, m0, rows, stream);
