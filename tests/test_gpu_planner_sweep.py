@@ -54,6 +54,9 @@ def _q4_shapes():
     # row tiles x column tiles on both sides of 2048 / 2560 (a wave per tile from there), and of the wave-tile sizes
     out += [(512, 128, 1024, 32, True), (512, 128, 1008, 32, False), (640, 128, 1024, 32, True), (640, 128, 1008, 32, False), (640, 96, 1024, 96, False), (1280, 64, 1024, 64, True), (2560, 256, 1030, 128, False),
             (650, 96, 1024, 96, True), (1290, 64, 2048, 64, False)]
+    # either side of the lines between the wave tiles of integers and float16 (blocks of 32 and 64: padded rows, four waves per SIMD)
+    out += [(48, 64, 16384, 32, True), (64, 64, 16384, 32, False), (64, 64, 16384, 64, True), (65, 64, 16384, 64, False), (48, 128, 16384, 128, False),
+            (65, 128, 16384, 128, True), (48, 256, 16384, 256, True)]
     return out
 
 

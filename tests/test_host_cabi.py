@@ -251,3 +251,15 @@ def test_q4_wave_tiles_count_real_rows(bs):
     for m, k, n in [(96, 4096, 11008), (90, 4096, 11008), (70, 4096, 16384), (150, 4096, 8192)]:
         assert _q4_form(m, k, n, bs or k) == "2x1", (m, k, n)
     assert _q4_form(300, 4096, 11008, bs or k) == "2x2" and _q4_form(64, 4096, 11008, bs or k) == "1x1"
+
+
+def test_q4_float16_form_where_it_pays():
+    """4-bit products in blocks of 32 and 64: the float16 form takes 32 rows per wave and a longer first pass, so few rows stay on integers;
+    blocks of 64, whose integer form is the faster one, longer."""
+    for m, k, n, bs in [(40, 4096, 16384, 64), (64, 2048, 16384, 64), (70, 2048, 11008, 64), (128, 4096, 8192, 64), (256, 4096, 4096, 64),
+                        (48, 2048, 16384, 32), (70, 1024, 11008, 32), (64, 4096, 8192, 32)]:
+        assert _q4_form(m, k, n, bs) == "1x1", (m, k, n, bs)
+    for m, k, n, bs in [(96, 4096, 11008, 64), (100, 2048, 11008, 64), (33, 4096, 28672, 64), (48, 4096, 16384, 32), (17, 4096, 28672, 32),
+                        (200, 4096, 4096, 32), (100, 2048, 8192, 32)]:
+        assert _q4_form(m, k, n, bs) == "half 2x2", (m, k, n, bs)
+    assert _q4_form(2048, 4096, 11008, 32) == "half 2x4" and _q4_form(2048, 11008, 4096, 64) == "half 2x4"

@@ -16,12 +16,19 @@ constexpr Q4Form q4_rows_form(uint32_t m, uint32_t tiles, uint32_t quads, uint32
   const uint64_t int11 = rows16 * tiles, int21 = rows32 * tiles, int22 = rows32 * ((uint64_t(tiles) + 1) / 2);  // waves of each
   const uint64_t half22 = int22, half24 = rows32 * ((uint64_t(tiles) + 3) / 4);
   if (upb == 1 || upb == 2) {
-    (void)quads;
-    // Fewer waves of 2 x 2 than four for every five SIMDs: the integer kernel (us at blocks of 32, waves of 2 x 2 in brackets: 128 x 11008
-    // x 4096 [512] integers 59, float16 67; 64 x 4096 x 11008 [688] 30, 30; 256 x 4096 x 4096 [1024] 36.5, 34; 128 x 4096 x 11008
-    // [1376] 50, 43.5; 64 x 4096 x 28672 [1792] 61, 45).  2 x 4 from three waves for two SIMDs on (128 x 4096 x 11008 [688 of 2 x 4] 48.5 against
-    // 43.5; 64 x 4096 x 28672 [896] 49.5, 45; 100 x 4096 x 27777 in blocks of 64 [1738] 67, 80; 512 x 4096 x 11008 [2752] 108, 110).
-    const bool halves = half22 * 5 >= uint64_t(simds) * 4;
+    // The integer kernel, a wave per tile, where there are few: a wave of it takes 16 rows and a float16 one 32, the integer form of blocks
+    // of 64 is twice as fast as that of 32, and the float16 form writes twice the bytes per row first (~4 us more before it is ahead).
+    // Blocks of 64: up to four integer waves per SIMD, what fits one at once (us, integers / float16, waves of 1 x 1 in brackets: 40 x 4096 x 16384
+    // [3072] 24.9 / 32.3, 70 x 2048 x 11008 [3440] 18.2 / 20.4, 128 x 4096 x 8192 [4096] 30.0 / 32.4, 96 x 4096 x 11008 [4128] 40.5 / 34.9, 100 x
+    // 4096 x 11008 [4816] 44.2 / 38.2).  Blocks of 32: fewer waves of 2 x 2 than four for every five SIMDs (waves of 2 x 2 in brackets: 128 x
+    // 11008 x 4096 [512] 53 / 62, 64 x 4096 x 11008 [688] 28 / 26, 180 x 4096 x 4096 [768] 27.0 / 28.0, 200 x 4096 x 4096 [896] 31.8 / 28.4, 128 x
+    // 4096 x 11008 [1376] 51 / 37), and up to 2048 values of k, where the first pass weighs most, also rows of which more than a seventh is
+    // padding up to pairs of tiles (48 x 2048 x 16384 16.0 / 16.8, 70 x 2048 x 11008 19.8 / 21.1; 48 x 4096 x 16384 28.1 / 25.7, 100 x 2048 x 8192 18.6 /
+    // 17.6).
+    const bool halves = upb == 2 ? int11 > 4ull * simds
+                                 : half22 * 5 >= uint64_t(simds) * 4 && (quads > 16 || int11 > 4ull * simds || int11 * 2 >= half22 * 7);
+    // 2 x 4 from three waves for two SIMDs on (128 x 4096 x 11008 [688 of 2 x 4] 48.5 against 43.5; 64 x 4096 x 28672 [896] 49.5, 45; 100 x 4096 x
+    // 27777 in blocks of 64 [1738] 67, 80; 512 x 4096 x 11008 [2752] 108, 110).
     return !halves ? kQ4Int11 : half24 * 2 >= uint64_t(simds) * 3 ? kQ4Half24 : kQ4Half22;
   }
   // The largest tile that leaves every SIMD two and a half waves.  2 x 1: also from two waves on (90 x 4096 x 11008 in blocks of 128 as 2064 waves
