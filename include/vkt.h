@@ -87,15 +87,16 @@ void vkt_event_destroy(void* event);
 /* vkt_dispatch for callers that cannot allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid it).  No counterpart in the reference.  Same arguments, same kernels, same results; the
  * difference is where the kernels' own workspace lives (the partial sums of a product that is split over
- * workgroups, e.g. "qmm8_bf16" at 64 rows): here it is a fixed array of VKT_STATIC_SCRATCH_BYTES in the library's
+ * workgroups, e.g. "qmm8_bf16" at 64 rows, and the float16 rows of "qmm4c_*" with many rows in blocks of 32 and 64): here it is a fixed array of VKT_STATIC_SCRATCH_BYTES in the library's
  * code object, one per device, held until the process ends, and the call makes no hipMalloc / hipFree (vkt_dispatch
  * takes its workspace from the pool at its first call and grows a second region for many-row int8 products).
  *   - The runtime must be running: call any other function (e.g. vkt_device_info) once at start-up.
  *   - A product whose planned split needs more workspace than the array holds returns -1 with a message that
- *     names both sizes; it is never re-planned with fewer slices.  Many-row int8 products do not widen their
+ *     names both sizes; it is never re-planned with fewer slices.  4-bit products take their rows in as many pieces as
+ *     the array needs.  Many-row int8 products do not widen their
  *     weights here: they run on the row-block kernels.
  *   - Calls are queued on the runtime's one in-order stream like every other dispatch, so two calls never overlap on
- *     the device; the array keeps the last call's partial sums, and every kernel writes what it later reads (nothing
+ *     the device; the array keeps what the last call left in it, and every kernel writes what it later reads (nothing
  *     has to start at zero). */
 #define VKT_STATIC_SCRATCH_BYTES (16u << 20)
 int vkt_dispatch_static(const char* name, const uint32_t* spec, size_t nspec, const uint8_t* push, size_t npush,
@@ -163,11 +164,14 @@ typedef struct Q4PackParams {
  * side-car of that LAYOUT.  PHASE 0 writes the quantised activations into q
  * (vkt_qmm4c_q_bytes; the arrangement differs per layout) and rows; PHASE 1 is the
  * product; PHASE 2 does both: with LAYOUT 0 in one launch per 4 rows where the rows can
- * be quantised from registers (k a multiple of 8, at most 16384), otherwise as PHASE 0
- * then 1.  Results are bit-identical to qmm4.  With LAYOUT 1, bits 4-7 of PHASE override the choice
+ * be quantised from registers (k a multiple of 8, at most 16384; q and rows are then not
+ * touched), otherwise as PHASE 0 then 1: it leaves in q and rows what PHASE 0 does.  Bit 8 of a PHASE 2 with LAYOUT 1 says
+ * that q is not read afterwards: what it holds then is unspecified (blocks of 32 and 64 with many rows multiply from the
+ * runtime's workspace, and writing the rows to q as well is a pass more).  Results are bit-identical to qmm4.  With LAYOUT 1,
+ * bits 4-7 of PHASE override the choice
  * between the product kernels, which give the same bits (tests, tuning): 16 keeps the kernel whose four waves
  * split K, 32 forces those whose waves each walk all of K (| 64, 128, 192: 1, 2, 4 tiles of 16 x 16 per wave; blocks of 32 and 64:
- * 1, 4, 8, the latter two against the runtime's workspace, to which PHASE 2 then writes the activations instead of to q).
+ * 1, 4, 8, the latter two from the workspace).
  * With LAYOUT 0, PHASE 2 with 1, 2 or 3 in bits 8-9 fixes the column tiles per workgroup (same bits). */
 typedef struct Q4CParams {
   uint64_t inp, q, rows, compact, out;

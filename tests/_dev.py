@@ -75,9 +75,10 @@ class CompactWeights:
         dp.free()
 
 
-def q4_compact(x, odt, cw, fused=True, flags=0):
+def q4_compact(x, odt, cw, fused=True, flags=0, static=False, want_q=False):
     """_dyn_quant_matmul_4bit through the streaming path ("qmm4c_*"): one fused launch
-    (PHASE 2), or row quantisation (PHASE 0) then the product (PHASE 1).  flags (matrix-core layout): 16 keeps the
+    (PHASE 2), or row quantisation (PHASE 0) then the product (PHASE 1).  static: through vkt_dispatch_static; want_q: also the
+    bytes that q and rows hold afterwards.  flags (matrix-core layout): 16 keeps the
     one-row-tile kernel, 32 forces the wave-per-tile kernel (| 64: one tile per wave, | 128: two, | 192: four)."""
     x = np.ascontiguousarray(x)
     m, n, k, bs = x.shape[0], cw.n, cw.k, cw.bs
@@ -90,11 +91,14 @@ def q4_compact(x, odt, cw, fused=True, flags=0):
     g = int(bs != k)
     name = "qmm4c_" + abi.SUFFIX[odt]
     if m and n and fused:
-        abi.dispatch(name, [2 | flags, g, cw.layout], p, ((n + 31) // 32, (m + 7) // 8))
+        abi.dispatch(name, [2 | flags, g, cw.layout], p, ((n + 31) // 32, (m + 7) // 8), static=static)
     elif m and n:
-        abi.dispatch(name, [0, g, cw.layout], p, (m,))
-        abi.dispatch(name, [1 | flags, g, cw.layout], p, ((n + 31) // 32, (m + 7) // 8))
-    return do.to_numpy(_NP[odt], (m, n))
+        abi.dispatch(name, [0, g, cw.layout], p, (m,), static=static)
+        abi.dispatch(name, [1 | flags, g, cw.layout], p, ((n + 31) // 32, (m + 7) // 8), static=static)
+    out = do.to_numpy(_NP[odt], (m, n))
+    if want_q:
+        return out, dq.to_numpy(np.uint8, (abi.lib().vkt_qmm4c_q_bytes(m, k),)), dr.to_numpy(np.uint32, (m, 2))
+    return out
 
 
 def scaled_mm(a, fmt_a, bt, fmt_b, sa, sb, rowwise, bias=None, bias_dtype=oracle.F32, scale_result=None,

@@ -128,6 +128,37 @@ def test_q4_float16_products(m, k, n, bs, flags, bias):
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), fused
 
 
+@pytest.mark.parametrize("m,k,n,bs,flags", [(64, 96, 145, 32, 32 | 128), (47, 2112, 33, 64, 32 | 192), (33, 1000, 17, 1000, 0), (80, 64, 28672, 32, 0),
+                                            (40, 128, 16, 128, 16)])
+def test_q4_phase_2_is_phase_0_then_1(m, k, n, bs, flags):
+    """PHASE 2 with the matrix-core layout leaves in q and rows what PHASE 0 does, also where its product does not read q (a second product
+    of the same rows is PHASE 1 alone); with bit 8 only the result counts."""
+    import _dev
+    w, sc, bvec = int4_weights(n, k, bs, bias=True)
+    x = int4_rows(m, k, torch.float32)
+    packed = torch._dyn_quant_pack_4bit_weight(w, sc, bvec, bs, k, n).numpy()
+    cm = _dev.CompactWeights(packed, bs, k, n, layout=1)
+    two, q2, rows2 = _dev.q4_compact(bits(x), oracle.F32, cm, fused=True, flags=flags, want_q=True)
+    one, q1, rows1 = _dev.q4_compact(bits(x), oracle.F32, cm, fused=False, flags=flags, want_q=True)
+    rows, quads = (m + 15) // 16 * 16, (k + 2047) // 2048 * 16  # (rows past m in the last row tile of q are nobody's)
+    q1, q2 = (q[: rows * quads * 128].reshape(-1, quads, 2, 4, 16, 16).transpose(0, 4, 1, 2, 3, 5).reshape(rows, -1)[:m] for q in (q1, q2))
+    assert np.array_equal(q1, q2) and np.array_equal(rows1, rows2) and np.array_equal(one, two)
+    assert np.array_equal(_dev.q4_compact(bits(x), oracle.F32, cm, flags=flags | 256), one)
+
+
+def test_q4_float16_products_on_the_fixed_workspace():
+    """vkt_dispatch_static: three pieces of rows where the pool's workspace takes two."""
+    import _dev
+    m, k, n, bs = 1030, 16384, 20, 32
+    w, sc, bvec = int4_weights(n, k, bs, bias=True)
+    x = int4_rows(m, k, torch.float32)
+    packed = torch._dyn_quant_pack_4bit_weight(w, sc, bvec, bs, k, n).numpy()
+    cm = _dev.CompactWeights(packed, bs, k, n, layout=1)
+    want = _dev.q4_compact(bits(x), oracle.F32, cm, flags=16)
+    for fused in (True, False):
+        assert np.array_equal(_dev.q4_compact(bits(x), oracle.F32, cm, fused=fused, flags=32 | 192, static=True), want), fused
+
+
 @pytest.mark.parametrize("m,k,n,bs", [(33, 2304, 145, 256), (47, 6400, 40, 256), (65, 6400, 33, 128), (33, 6176, 49, 6176)])
 @pytest.mark.parametrize("flags", [32 | 64, 32 | 128, 32 | 192])
 def test_q4_several_tiles_per_wave(m, k, n, bs, flags):

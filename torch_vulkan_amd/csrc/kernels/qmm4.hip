@@ -720,9 +720,9 @@ __device__ __forceinline__ uint64_t halves_offset(uint32_t m, uint32_t g, uint32
 
 // Phase 0 for the matrix layout, one workgroup per row, from row m0 on.  FAST: k is a multiple of 8, at most
 // 2048 * kFusedGroups, rows 16-byte aligned: the row is read once, into registers.  HALVES: the values go to `dst` as
-// qmm4m_half's operand, row m0 first, instead of to p.q.
+// qmm4m_half's operand, row m0 first, and to p.q only where `keep` says that the caller reads them there.
 template <class T, bool FAST, bool HALVES>
-__global__ __launch_bounds__(256) void qmm4m_rowquant(Q4CParams p, uint32_t groupwise, uint32_t quads, uint64_t dst, uint32_t m0) {
+__global__ __launch_bounds__(256) void qmm4m_rowquant(Q4CParams p, uint32_t groupwise, uint32_t quads, uint64_t dst, uint32_t m0, uint32_t keep) {
   constexpr uint64_t item = sizeof(typename T::storage);
   const uint32_t m = m0 + blockIdx.x, tid = threadIdx.x;
   const uint64_t row = p.inp + uint64_t(m) * p.k * item;
@@ -737,6 +737,7 @@ __global__ __launch_bounds__(256) void qmm4m_rowquant(Q4CParams p, uint32_t grou
   };
   auto put = [&](uint32_t g, int (&q)[8]) {
     if constexpr (HALVES) {
+      if (keep) stg<U2>(p.q + operand_offset(m, g, quads), operand_bytes(q));
 #pragma unroll
       for (int e = 0; e < 8; ++e) q[e] -= rq.izp;
       stg<U4>(dst + halves_offset(blockIdx.x, g, quads), operand_halves(q));
@@ -1560,7 +1561,8 @@ int launch_qmm4c_pack(const Q4PackParams& p, uint32_t layout, const Machine&, hi
 template <class T>
 int launch_matrix(const Q4CParams& p, uint32_t phase_and_flags, uint32_t groupwise, const Machine& mc, hipStream_t stream, std::string* err) {
   constexpr uint32_t item = sizeof(typename T::storage);
-  const uint32_t phase = phase_and_flags & 15u, flags = phase_and_flags & ~15u;
+  const uint32_t phase = phase_and_flags & 15u, flags = phase_and_flags & 0xf0u;
+  const uint32_t keep = phase_and_flags & 256u ? 0u : 1u;  // (whether PHASE 2 leaves the quantised rows in p.q)
   MatrixLayout M;
   if (!matrix_layout(p.n, p.k, p.bs, &M)) {
     *err = "qmm4c: this shape has no compact form (groupwise block sizes: 32, 64, 128, 256)";
@@ -1600,8 +1602,8 @@ int launch_matrix(const Q4CParams& p, uint32_t phase_and_flags, uint32_t groupwi
       const uint64_t at = mc.workspace;
       const uint32_t threads = (rows + 15) / 16 * 16 * M.quads * 16;  // (below the workspace's bytes / 16)
       if (phase == 1) hipLaunchKernelGGL(qmm4m_expand, dim3(threads / 256), dim3(256), 0, stream, p, at, m0, rows, M.quads);
-      else if (fast) hipLaunchKernelGGL((qmm4m_rowquant<T, true, true>), dim3(rows), dim3(256), 0, stream, p, groupwise, M.quads, at, m0);
-      else hipLaunchKernelGGL((qmm4m_rowquant<T, false, true>), dim3(rows), dim3(256), 0, stream, p, groupwise, M.quads, at, m0);
+      else if (fast) hipLaunchKernelGGL((qmm4m_rowquant<T, true, true>), dim3(rows), dim3(256), 0, stream, p, groupwise, M.quads, at, m0, keep);
+      else hipLaunchKernelGGL((qmm4m_rowquant<T, false, true>), dim3(rows), dim3(256), 0, stream, p, groupwise, M.quads, at, m0, keep);
       if (M.upb == 1 && eight) launch_half<T, 1, 2, 4>(p, M, at, m0, rows, stream);
       else if (M.upb == 1) launch_half<T, 1, 2, 2>(p, M, at, m0, rows, stream);
       else if (eight) launch_half<T, 2, 2, 4>(p, M, at, m0, rows, stream);
@@ -1610,8 +1612,8 @@ int launch_matrix(const Q4CParams& p, uint32_t phase_and_flags, uint32_t groupwi
     return 0;
   }
   if (phase == 0 || phase == 2) {
-    if (fast) hipLaunchKernelGGL((qmm4m_rowquant<T, true, false>), dim3(p.m), dim3(256), 0, stream, p, groupwise, M.quads, 0ull, 0u);
-    else hipLaunchKernelGGL((qmm4m_rowquant<T, false, false>), dim3(p.m), dim3(256), 0, stream, p, groupwise, M.quads, 0ull, 0u);
+    if (fast) hipLaunchKernelGGL((qmm4m_rowquant<T, true, false>), dim3(p.m), dim3(256), 0, stream, p, groupwise, M.quads, 0ull, 0u, 1u);
+    else hipLaunchKernelGGL((qmm4m_rowquant<T, false, false>), dim3(p.m), dim3(256), 0, stream, p, groupwise, M.quads, 0ull, 0u, 1u);
   }
   if (phase == 1 || phase == 2) {
     for (uint32_t m0 = 0; rows_kernel && m0 < p.m; m0 += 16 * 1024) {
@@ -1657,8 +1659,9 @@ int launch_qmm4c(const Q4CParams& p, int dtype, uint32_t phase, uint32_t groupwi
       *err = "qmm4c: GROUPWISE must be 1 exactly when bs != k";
       return -1;
     }
-    if (!p.inp || !p.out || (phase & 15u) > 2 || (phase & ~255u)) {
-      *err = (phase & 15u) > 2 || (phase & ~255u) ? "qmm4c: PHASE must be 0, 1 or 2" : "qmm4c: null or unaligned tensor address";
+    const bool bad_phase = (phase & 15u) > 2 || (phase & ~((phase & 15u) == 2 ? 511u : 255u));
+    if (!p.inp || !p.out || bad_phase) {
+      *err = bad_phase ? "qmm4c: PHASE must be 0, 1 or 2" : "qmm4c: null or unaligned tensor address";
       return -1;
     }
     const int rc = dtype == VKT_F32 ? launch_matrix<f32_t>(p, phase, groupwise, mc, stream, err)

@@ -267,7 +267,8 @@ at::Tensor dyn_quant_matmul_4bit(const at::Tensor& inp, const at::Tensor& packed
       Q4CParams p{};
       fill_piece(p, first, rows);
       p.q = gpu_address_out(q), p.rows = gpu_address_out(row_params), p.compact = gpu_address(compact);
-      dispatch("qmm4c" + family, {2u, groupwise, layout}, p, 1);  // phase 2: row quantisation + product
+      // phase 2: row quantisation + product (bit 8, matrix-core layout: the quantised rows are not read afterwards)
+      dispatch("qmm4c" + family, {layout == 1u ? 2u | 256u : 2u, groupwise, layout}, p, 1);
     });
     return output;
   }
