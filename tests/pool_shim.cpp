@@ -103,4 +103,7 @@ uint32_t shim_q4_rows_form(uint32_t m, uint32_t tiles, uint32_t quads, uint32_t 
   return vkt::q4_rows_form(m, tiles, quads, upb, simds);
 }
 
+// whether 256 x 128 tiles take less than 256 x 256 ones (kernels/plans.h)
+int shim_narrow_tiles_float8_wide(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return vkt::narrow_tiles_float8_wide(m, n, k, cus) ? 1 : 0; }
+
 }  // extern "C"

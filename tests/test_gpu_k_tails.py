@@ -73,6 +73,12 @@ def test_float8(k, variant, out):
     run_case(300, k, 264, FLOAT8[0], FLOAT8[1], out, True, torch.float32, None if out.itemsize > 1 else 2.0, variant=variant, seed=k)
 
 
+@pytest.mark.parametrize("m,k,n,out", [(3300, 144, 4900, torch.float32), (3300, 208, 4904, torch.float16)])
+def test_float8_widened_planned_tiles(m, k, n, out):
+    """Planned: 260 tiles of 256 x 256 would take two rounds, the 256 x 128 ones take two shorter ones."""
+    run_case(m, k, n, FLOAT8[0], FLOAT8[1], out, True, torch.float32, seed=n)
+
+
 @pytest.mark.parametrize("out", [torch.bfloat16, torch.float32, torch.float16, torch.float8_e4m3fn])
 def test_float8_last_slice_shorter_than_a_step(out):
     """Planned: 16 slices of 9 steps, the last of them 64 bytes."""

@@ -263,3 +263,15 @@ def test_q4_float16_form_where_it_pays():
                         (200, 4096, 4096, 32), (100, 2048, 8192, 32)]:
         assert _q4_form(m, k, n, bs) == "half 2x2", (m, k, n, bs)
     assert _q4_form(2048, 4096, 11008, 32) == "half 2x4" and _q4_form(2048, 11008, 4096, 64) == "half 2x4"
+
+
+def test_narrow_tiles_where_their_rounds_are_shorter():
+    """Float8 products with float32 and float16 outputs whose k ends inside a step: a few more wide tiles than compute units take two
+    rounds, where narrow ones take two or three of little more than half the length."""
+    L = ctypes.CDLL(os.path.join(os.path.dirname(abi.LIB_PATH), "libvkt_hosttest.so"))
+    L.shim_narrow_tiles_float8_wide.argtypes = [ctypes.c_uint32] * 4
+    for m, k, n in [(3265, 736, 4944), (6435, 1216, 2593), (4949, 3536, 3433), (3307, 6160, 5107), (4333, 624, 8928), (2609, 272, 6496)]:
+        assert L.shim_narrow_tiles_float8_wide(m, n, k, 256), (m, k, n)
+        assert not L.shim_narrow_tiles_float8_wide(m, n, (k + 127) // 128 * 128, 256), (m, k, n)  # (whole steps: as ever)
+    for m, k, n in [(4096, 4112, 4096), (2048, 4112, 16384), (5000, 3600, 5000), (8192, 144, 8192), (6439, 2880, 8599)]:
+        assert not L.shim_narrow_tiles_float8_wide(m, n, k, 256), (m, k, n)

@@ -41,4 +41,19 @@ constexpr Q4Form q4_rows_form(uint32_t m, uint32_t tiles, uint32_t quads, uint32
   return (upb == 8 ? int21 >= 2048 : int11 > 4096) ? kQ4Int21 : kQ4Int11;
 }
 
+// ---- The tile kernel with 256 x 256 or 256 x 128 outputs per workgroup, one workgroup per compute unit: whether the narrow
+// tiles take less, where a round of them costs `cost` hundredths of a round of the wide ones.  Both are built for a k that ends inside
+// a step (of 128 bytes), the narrow ones staged through registers.
+constexpr bool narrow_tiles_pay(uint32_t m, uint32_t n, uint64_t batches, uint32_t cus, uint32_t cost) {
+  const uint64_t rows = (uint64_t(m) + 255) / 256;
+  const uint64_t wide = rows * ((uint64_t(n) + 255) / 256) * batches, narrow = rows * ((uint64_t(n) + 127) / 128) * batches;
+  return (narrow + cus - 1) / cus * cost < (wide + cus - 1) / cus * 100;
+}
+// Float8 operands widened to bfloat16 (float32 and float16 outputs).  Rounds of wide / narrow tiles in brackets, us: 3265 x 736 x 4944 [2, 2]
+// 76 / 47, 6435 x 1216 x 2593 [2, 3] 129 / 110, 4949 x 3536 x 3433 [2, 3] 229 / 207, 3307 x 6160 x 5107 [2, 3] 344 / 314, 4333 x 624 x 8928 [3, 5] 110 /
+// 104, 3572 x 416 x 14808 [4, 7] 129 / 126, 6439 x 2880 x 8599 [4, 7] 408 / 425, 4096 x 4112 x 4096 [1, 2] 133 / 157, 8192 x 144 x 8192 [4, 8] 113 / 115.
+constexpr bool narrow_tiles_float8_wide(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) {
+  return k % 128 != 0 && narrow_tiles_pay(m, n, 1, cus, k <= 1024 ? 56 : 59);
+}
+
 }  // namespace vkt
