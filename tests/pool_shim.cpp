@@ -105,5 +105,13 @@ uint32_t shim_q4_rows_form(uint32_t m, uint32_t tiles, uint32_t quads, uint32_t 
 
 // whether 256 x 128 tiles take less than 256 x 256 ones (kernels/plans.h)
 int shim_narrow_tiles_float8_wide(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return vkt::narrow_tiles_float8_wide(m, n, k, cus) ? 1 : 0; }
+int shim_narrow_tiles_16bit(uint32_t m, uint32_t n, uint64_t batches, uint32_t k_bytes, uint32_t cus) {
+  return vkt::narrow_tiles_16bit(m, n, batches, k_bytes, cus) ? 1 : 0;
+}
+// whether 16-bit operands run on the stream kernel (kernels/plans.h)
+int shim_stream_pays_16bit(uint32_t m, uint32_t n, uint64_t batches, uint32_t k, uint32_t cus, int int8) {
+  return vkt::stream_pays_16bit(m, n, batches, k, cus, int8 != 0) ? 1 : 0;
+}
+uint32_t shim_stream_columns(uint32_t m, uint32_t n, uint64_t batches, uint32_t cus) { return vkt::mma_stream_tiles(m, n, batches, cus).columns; }
 
 }  // extern "C"

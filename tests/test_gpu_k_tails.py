@@ -73,6 +73,18 @@ def test_float8(k, variant, out):
     run_case(300, k, 264, FLOAT8[0], FLOAT8[1], out, True, torch.float32, None if out.itemsize > 1 else 2.0, variant=variant, seed=k)
 
 
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("m,k,n", [(3300, 72, 4901), (3300, 72, 4098)])
+def test_planned_tiles_off_the_stream_kernel(dtype, m, k, n):
+    """An odd n: 256 x 128 tiles where 260 of 256 x 256 would take two rounds, and 256 x 256 ones where they take one."""
+    import _dev
+    a, w = (torch.randn(m, k, generator=gen(34)) * 0.5).to(dtype), (torch.randn(n, k, generator=gen(35)) * 0.5).to(dtype)
+    want, mag = (a.double() @ w.double().T).numpy(), (a.double().abs() @ w.double().abs().T).numpy()
+    got = unbits(_dev.gemm16(bits(a), bits(w).T, ODT[dtype]), dtype).double().numpy()
+    # eps * |want| + 2^-20 * mag, the oracle's bound, around sums in 64 bits; below 2^-14 float16's values lie eps * 2^-14 apart
+    assert (np.abs(got - want) <= torch.finfo(dtype).eps * np.maximum(np.abs(want), 2.0**-14) + 2.0**-20 * mag).all()
+
+
 @pytest.mark.parametrize("m,k,n,out", [(3300, 144, 4900, torch.float32), (3300, 208, 4904, torch.float16)])
 def test_float8_widened_planned_tiles(m, k, n, out):
     """Planned: 260 tiles of 256 x 256 would take two rounds, the 256 x 128 ones take two shorter ones."""
@@ -99,7 +111,7 @@ def test_last_slice_shorter_than_a_step(dtype, layout):
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=str)
-@pytest.mark.parametrize("m,k,n", [(1500, 208, 6000), (400, 80, 8264)])
+@pytest.mark.parametrize("m,k,n", [(1500, 208, 6000), (400, 80, 8264), (3300, 80, 4901)])
 def test_int8_many_rows(dtype, m, k, n):
     import _dev
     a = torch.randn(m, k, generator=gen(29)).to(dtype)

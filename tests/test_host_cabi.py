@@ -275,3 +275,29 @@ def test_narrow_tiles_where_their_rounds_are_shorter():
         assert not L.shim_narrow_tiles_float8_wide(m, n, (k + 127) // 128 * 128, 256), (m, k, n)  # (whole steps: as ever)
     for m, k, n in [(4096, 4112, 4096), (2048, 4112, 16384), (5000, 3600, 5000), (8192, 144, 8192), (6439, 2880, 8599)]:
         assert not L.shim_narrow_tiles_float8_wide(m, n, k, 256), (m, k, n)
+    # 16-bit operands that the stream kernel does not serve: the same with a higher price of a narrow round
+    L.shim_narrow_tiles_16bit.argtypes = [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint64, ctypes.c_uint32, ctypes.c_uint32]
+    for m, k, n in [(3686, 304, 5427), (6799, 3824, 2397), (1652, 984, 12457), (2100, 304, 8195)]:
+        assert L.shim_narrow_tiles_16bit(m, n, 1, 2 * k, 256) and not L.shim_narrow_tiles_16bit(m, n, 1, (2 * k + 127) // 128 * 128, 256)
+    for m, k, n in [(4096, 4104, 14337), (7526, 440, 10851), (4096, 4104, 4095), (1024, 200, 14337)]:
+        assert not L.shim_narrow_tiles_16bit(m, n, 1, 2 * k, 256), (m, k, n)
+
+
+def test_stream_kernel_where_it_pays():
+    """16-bit operands and int8 weights with few tiles: the stream kernel's tiles of 256 rows where their rounds are shorter than the 128 x 128
+    tiles' one round, not where padded rows and a short k make them longer."""
+    L = ctypes.CDLL(os.path.join(os.path.dirname(abi.LIB_PATH), "libvkt_hosttest.so"))
+    L.shim_stream_pays_16bit.argtypes = [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint64, ctypes.c_uint32, ctypes.c_uint32, ctypes.c_int]
+    L.shim_stream_columns.argtypes = [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint64, ctypes.c_uint32]
+    pays = lambda m, k, n, int8=0, batches=1: bool(L.shim_stream_pays_16bit(m, n, batches, k, 256, int8))  # noqa: E731
+    for m, k, n in [(581, 128, 12800), (353, 256, 17960), (640, 1024, 11520), (275, 128, 18976), (512, 4096, 8192), (1024, 4096, 4096)]:
+        assert not pays(m, k, n), (m, k, n)
+    for m, k, n in [(300, 4096, 11008), (1500, 8192, 3072), (516, 2048, 12944), (581, 4096, 12800), (700, 136, 8192), (2048, 4096, 4096), (259, 256, 13064)]:
+        assert pays(m, k, n), (m, k, n)
+    for m, k, n in [(1024, 256, 4096), (1024, 4096, 4096), (271, 256, 18432), (372, 1024, 16896), (336, 2048, 18192), (300, 256, 11008), (513, 256, 6656)]:
+        assert not pays(m, k, n, 1), (m, k, n)
+    for m, k, n in [(1024, 8192, 4096), (300, 4096, 11008), (1030, 256, 4096), (1537, 5120, 13824), (1152, 256, 7040), (520, 512, 8192)]:
+        assert pays(m, k, n, 1), (m, k, n)
+    assert not pays(100, 512, 1000, batches=36) and pays(512, 128, 512, batches=40)
+    assert [L.shim_stream_columns(m, n, 1, 256) for m, n in [(1024, 8192), (1537, 13824), (1024, 14336), (4096, 28672)]] == [128, 192, 256, 256]
+    assert [L.shim_stream_columns(m, n, 1, 256) for m, n in [(2000, 10240), (700, 22016)]] == [192, 192]

@@ -19,6 +19,7 @@
 #include "mma_tile.h"
 #include "mma_skinny.h"
 #include "mma_slices.h"
+#include "plans.h"
 
 namespace vkt {
 namespace {
@@ -297,7 +298,7 @@ int launch_tiles(const GemmParams& p, uint32_t use_cin, uint32_t batch, uint32_t
       }
     }
   }
-  // variant 0: planned; 1: 128x128 tiles; 2: 256x128; 3: 256x256 with direct loads; 4: 128x128 with direct loads;
+  // variant 0: planned; 1: 128x128 tiles; 2: 256x128 (planned for a k that ends inside a step); 3: 256x256 with direct loads; 4: 128x128 with direct loads;
   // 5: 256x256 with direct loads over 8 waves; 6: the stream kernel (mma_stream.h; else 3)
   // (k-major operands run on the direct forms only)
   uint32_t small = 3;  // what the stream kernel's products run on where it does not serve
@@ -310,11 +311,10 @@ int launch_tiles(const GemmParams& p, uint32_t use_cin, uint32_t batch, uint32_t
     //  with k-contiguous operands the 8-wave form reads 1.5x the LDS bytes and is 3-5 % slower)
     variant = large ? (TRA && TRB ? 5 : 3) : (TRA || TRB ? 4 : 1);
     // both operands contiguous along k (x @ w.T): the stream kernel where it serves (8192^3: 0.94-1.00 -> 0.89 ms), with the columns per
-    // tile that suit the shape also below that line, from more 128 x 128 tiles than compute units on (us, 128 x 128 tiles / stream: 258
-    // tiles of 300 x 11008 x 4096 72 / 57, 288 of 1500 x 3072 x 8192 137 / 105, 512 of 2048 x 4096 x 4096 84 / 69; up to 256 tiles they are
-    // level: 512 x 8192 x 4096 56.1 / 55.5, 512 x 5120 x 4096 52.3 / 53.7)
-    const bool more = uint64_t((p.m + 127) / 128) * ((p.n + 127) / 128) * batch > uint64_t(mc.compute_units);
-    if (!TRA && !TRB && (variant == 3 || more)) small = variant, variant = 6;
+    // tile that suit the shape also below that line
+    const bool more = stream_pays_16bit(p.m, p.n, batch, p.k, uint32_t(mc.compute_units), false);
+    if (!TRA && !TRB && (variant == 3 || more))
+      small = variant == 3 && narrow_tiles_16bit(p.m, p.n, batch, g.k, uint32_t(mc.compute_units)) ? 2 : variant, variant = 6;
   }
   const bool stream_ok = g.k > BK && p.n % 8 == 0 && p.c_sm % 8 == 0 && p.c_sb % 8 == 0 && p.c % 16 == 0 &&
                          mma_stream_strides_ok(g.lda, g.ldb);
@@ -467,11 +467,12 @@ int launch_q8_gemm_t(const Q8Params& p, const Machine& mc, hipStream_t stream, s
   Q8GemmProblem<T> g;
   g.a = p.a, g.b = mc.scratch, g.m = p.m, g.n = p.n, g.k = p.k * 2, g.lda = uint32_t(p.a_sm) * 2, g.ldb = p.k * 2;
   g.batches = 1, g.a_batch = 0, g.b_batch = 0, g.c = p.c, g.scales = p.scales;
-  // (the stream kernel throughout: there are as many 128 x 128 tiles as compute units, and it is level there, 1024 x 4096 x 4096 69.2 against
-  //  68.0 us, and ahead from there on; see the 16-bit product)
-  if (g.k > BK && p.n % 8 == 0 && p.c % 16 == 0 && p.scales % 16 == 0 && mma_stream_strides_ok(g.lda, g.ldb))
-    return launch_mma_stream<0, 0, MATH>(g, 0, mc.compute_units, stream, err, "qmm8");
   const bool large = uint64_t((p.m + 255) / 256) * ((p.n + 255) / 256) * 8 >= uint64_t(mc.compute_units) * 5;  // (as for the 16-bit product)
+  if ((large || stream_pays_16bit(p.m, p.n, 1, p.k, uint32_t(mc.compute_units), true)) && g.k > BK && p.n % 8 == 0 && p.c % 16 == 0 && p.scales % 16 == 0 &&
+      mma_stream_strides_ok(g.lda, g.ldb))
+    return launch_mma_stream<0, 0, MATH>(g, 0, mc.compute_units, stream, err, "qmm8");
+  if (large && narrow_tiles_16bit(p.m, p.n, 1, g.k, uint32_t(mc.compute_units)))
+    return launch_mma_tile<2, 2, 8, 4, 0, 0, true, false, MATH>(g, mc.compute_units, stream, err, "qmm8");
   if (large) return launch_mma_tile<2, 2, 8, 8, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "qmm8");
   return launch_mma_tile<2, 2, 4, 4, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "qmm8");
 }

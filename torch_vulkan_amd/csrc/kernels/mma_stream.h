@@ -1,7 +1,7 @@
 // The matrix-core kernel for large products with 16-bit outputs (float8 operands for _scaled_mm, 16-bit operands for
 // the matrix product and the many-row int8 product): 256 x 256 tiles of A [m, k] x B [n, k]^T (rows of k contiguous
 // bytes, as in mma_tile.h) on 8 waves of 64 x 128, K in steps of 128 bytes through two LDS stages of 64 KiB.  (Or 256 x 192 and 256 x
-// 128 tiles, waves of 64 x 96 and 64 x 64: mma_stream_columns.)
+// 128 tiles, waves of 64 x 96 and 64 x 64: mma_stream_tiles, plans.h.)
 // It differs from mma_tile in how a workgroup's time is laid out, after measuring where mma_tile's goes (one wave's
 // clock read at four points of every step): the matrix cores were busy 58-66 % of the cycles; the rest was the wave
 // issuing address arithmetic for its LDS-direct loads (380 cycles a step) and all eight waves starting every step
@@ -38,6 +38,7 @@
 
 #include "limits.h"
 #include "mma_tile.h"
+#include "plans.h"
 
 namespace vkt {
 namespace {
@@ -409,27 +410,10 @@ int launch_mma_stream_one(const P& p, int compute_units, hipStream_t stream, std
   return 0;
 }
 
-// Columns per tile: 256, or 192 or 128 where they take fewer or fuller rounds of a tile per compute unit.  A round costs about 100,
-// 81 and 64 parts of the same step (4096 x 14336 x 4096 in bfloat16, full rounds: 106, 86 and 64 us each; 4096 x 28672 x 8192 in float8: 102,
-// 83 and 66), and fewer columns read more bytes per product, so a tie goes to the wider tile.  us, 256 / 192 / 128 (rounds): float8 1024 x
-// 8192 x 8192 88 / 77 / 64 (1, 1, 1); 2000 x 10240 x 8192 184 / 155 / 176 (2, 2, 3); 700 x 22016 x 4096 95 / 80 / 90 (2, 2, 3); 4096 x 28672
-// x 8192 712 / 828 / 923 (7, 10, 14); bfloat16 1537 x 13824 x 5120 252 / 218 / 235 (2, 2, 3); 1024 x 14336 x 4096 107 / 149 / 121 (1, 2, 2).
-inline uint32_t mma_stream_columns(uint32_t m, uint32_t n, uint32_t batches, uint32_t cus) {
-  const uint32_t columns[3] = {256, 192, 128}, cost[3] = {100, 81, 64};
-  uint32_t best = 0;
-  uint64_t best_cost = 0;
-  for (int i = 0; i < 3; ++i) {
-    const uint64_t tiles = uint64_t((m + 255) / 256) * ((n + columns[i] - 1) / columns[i]) * batches;
-    const uint64_t c = (tiles + cus - 1) / cus * cost[i];
-    if (best == 0 || c < best_cost) best = columns[i], best_cost = c;
-  }
-  return best;
-}
-
 // forced: 1, 2, 3 for 256, 192, 128 columns per tile (tests, tuning), 0: planned.
 template <int FA, int FB, int MATH, class P>
 int launch_mma_stream(const P& p, uint32_t forced, int compute_units, hipStream_t stream, std::string* err, const char* who) {
-  const uint32_t columns = forced ? 320 - 64 * forced : mma_stream_columns(p.m, p.n, p.batches, uint32_t(compute_units));
+  const uint32_t columns = forced ? 320 - 64 * forced : mma_stream_tiles(p.m, p.n, p.batches, uint32_t(compute_units)).columns;
   const bool tail = p.k % BK != 0;
 #define VKT_STREAM(BN)                                                                          \
   (tail ? launch_mma_stream_one<FA, FB, MATH, BN, true>(p, compute_units, stream, err, who) \

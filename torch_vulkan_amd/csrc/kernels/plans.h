@@ -55,5 +55,52 @@ constexpr bool narrow_tiles_pay(uint32_t m, uint32_t n, uint64_t batches, uint32
 constexpr bool narrow_tiles_float8_wide(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) {
   return k % 128 != 0 && narrow_tiles_pay(m, n, 1, cus, k <= 1024 ? 56 : 59);
 }
+// 16-bit operands (the matrix product and the many-row int8 product) where the stream kernel does not serve, from five eighths of a wide tile
+// per compute unit on.  us, wide / narrow, rounds in brackets: x @ w.T 3686 x 304 x 5427 [2, 3] 59 / 55, 6799 x 3824 x 2397 [2, 3] 244 / 237, 1652 x
+// 984 x 12457 [2, 3] 97.6 / 95.6, 4096 x 4104 x 14337 [4, 8] 564 / 720, 7526 x 440 x 10851 [6, 10] 196 / 202; int8 weights 2100 x 304 x 8195 [2, 3] 59 / 56,
+// 6799 x 304 x 2397 [2, 3] 55.6 / 53.7.
+constexpr bool narrow_tiles_16bit(uint32_t m, uint32_t n, uint64_t batches, uint32_t k_bytes, uint32_t cus) {
+  return k_bytes % 128 != 0 && narrow_tiles_pay(m, n, batches, cus, 65);
+}
+
+// ---- The stream kernel (mma_stream.h): columns per tile of 256 rows.  256, or 192 or 128 where they take fewer or fuller rounds of a tile per
+// compute unit.  A round costs about 100, 81 and 64 parts of the same step (4096 x 14336 x 4096 in bfloat16, full rounds: 106, 86 and 64 us each; 4096
+// x 28672 x 8192 in float8: 102, 83 and 66), and fewer columns read more bytes per product, so a tie goes to the wider tile.  us, 256 / 192 /
+// 128 (rounds): float8 1024 x 8192 x 8192 88 / 77 / 64 (1, 1, 1); 2000 x 10240 x 8192 184 / 155 / 176 (2, 2, 3); 700 x 22016 x 4096 95 / 80 /
+// 90 (2, 2, 3); 4096 x 28672 x 8192 712 / 828 / 923 (7, 10, 14); bfloat16 1537 x 13824 x 5120 252 / 218 / 235 (2, 2, 3); 1024 x 14336 x 4096 107 /
+// 149 / 121 (1, 2, 2).
+struct StreamTiles {
+  uint32_t columns;
+  uint64_t cost;
+};
+constexpr StreamTiles mma_stream_tiles(uint32_t m, uint32_t n, uint64_t batches, uint32_t cus) {
+  const uint32_t columns[3] = {256, 192, 128}, cost[3] = {100, 81, 64};
+  StreamTiles best = {0, 0};
+  for (int i = 0; i < 3; ++i) {
+    const uint64_t tiles = (uint64_t(m) + 255) / 256 * ((uint64_t(n) + columns[i] - 1) / columns[i]) * batches;
+    const uint64_t c = (tiles + cus - 1) / cus * cost[i];
+    if (best.columns == 0 || c < best.cost) best = StreamTiles{columns[i], c};
+  }
+  return best;
+}
+// Whether 16-bit operands that have fewer than five eighths of a 256 x 256 tile per compute unit run on it instead of on 128 x 128 tiles, of which two
+// fit a compute unit: from more of those than compute units on (us, 128 x 128 / stream: 258 tiles of 300 x 4096 x 11008 72 / 57, 288 of 1500 x 8192 x 3072
+// 137 / 105, 512 of 2048 x 4096 x 4096 84 / 69; up to 256 tiles they are level: 512 x 4096 x 8192 56.1 / 55.5, 512 x 4096 x 5120 52.3 / 53.7).
+// While the 128 x 128 tiles fit the machine at once (512), the stream kernel takes 192 columns only where its rows are padded to 256, and a
+// round of that is no shorter than theirs: of one or two tiles down, and of three with a short k, they stay (581 x 128 x 12800 10.1 /
+// 12.0, 353 x 256 x 17960 12.1 / 12.7, 640 x 1024 x 11520 25.8 / 26.1; but 516 x 2048 x 12944 44.3 / 43.0, 581 x 4096 x 12800 83.5 / 78.9; int8 weights 271
+// x 256 x 18432 18.5 / 21.1, 372 x 1024 x 16896 39.5 / 42.6, 336 x 2048 x 18192 60.6 / 62.9).
+// int8: the many-row int8 product, whose 128 x 128 tiles are loaded into LDS directly: they also stay where they are one per compute unit (1024 x
+// 256 x 4096 11.3 / 12.6, x 4096 x 64.4 / 65.2, x 8192 x 115.4 / 113.5), and with padded rows up to 256 values of k (300 x 256 x 11008 13.4 / 14.5, 513 x
+// 256 x 6656 12.4 / 12.9; 520 x 512 x 8192 20.2 / 20.1; 1030 x 256 x 4096 13.7 / 12.4).
+constexpr bool stream_pays_16bit(uint32_t m, uint32_t n, uint64_t batches, uint32_t k, uint32_t cus, bool int8) {
+  const uint64_t rows128 = (uint64_t(m) + 127) / 128, rows256 = (uint64_t(m) + 255) / 256, tiles128 = rows128 * ((uint64_t(n) + 127) / 128) * batches;
+  if (tiles128 < cus || (tiles128 == cus && (!int8 || k <= 4096))) return false;
+  if (tiles128 > 2ull * cus) return true;
+  const StreamTiles tiles = mma_stream_tiles(m, n, batches, cus);
+  if (tiles.cost >= 100) return false;  // (batches of up to 128 rows: half of every tile would be padding)
+  if (tiles.columns != 128 && (rows256 <= 2 || (rows256 == 3 && k < 2048))) return false;
+  return !(int8 && k <= 256 && rows128 % 2 && rows256 <= 3);
+}
 
 }  // namespace vkt
