@@ -113,5 +113,6 @@ int shim_stream_pays_16bit(uint32_t m, uint32_t n, uint64_t batches, uint32_t k,
   return vkt::stream_pays_16bit(m, n, batches, k, cus, int8 != 0) ? 1 : 0;
 }
 uint32_t shim_stream_columns(uint32_t m, uint32_t n, uint64_t batches, uint32_t cus) { return vkt::mma_stream_tiles(m, n, batches, cus).columns; }
+int shim_stream_pays_float8(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return vkt::stream_pays_float8(m, n, k, cus) ? 1 : 0; }
 
 }  // extern "C"

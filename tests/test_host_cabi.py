@@ -301,3 +301,9 @@ def test_stream_kernel_where_it_pays():
     assert not pays(100, 512, 1000, batches=36) and pays(512, 128, 512, batches=40)
     assert [L.shim_stream_columns(m, n, 1, 256) for m, n in [(1024, 8192), (1537, 13824), (1024, 14336), (4096, 28672)]] == [128, 192, 256, 256]
     assert [L.shim_stream_columns(m, n, 1, 256) for m, n in [(2000, 10240), (700, 22016)]] == [192, 192]
+    # float8: from half a tile per compute unit on; long rows that begin inside a 128-byte line only where the rows are padded
+    L.shim_stream_pays_float8.argtypes = [ctypes.c_uint32] * 4
+    for m, k, n in [(512, 8192, 5120), (512, 8192, 8192), (256, 1104, 15712), (841, 4112, 3712), (640, 4112, 4096), (143, 8208, 13696), (384, 8224, 6400), (896, 8208, 4608), (308, 8224, 10368)]:
+        assert L.shim_stream_pays_float8(m, n, k, 256), (m, k, n)
+    for m, k, n in [(512, 8192, 4096), (256, 8272, 12800), (768, 6224, 4736), (222, 8224, 14912), (198, 6176, 16000), (700, 4128, 4096), (512, 8224, 4608)]:
+        assert not L.shim_stream_pays_float8(m, n, k, 256), (m, k, n)

@@ -415,17 +415,15 @@ int launch_formats(const F8Params& p, uint32_t variant, const Machine& mc, hipSt
     variant = 0;
   }
   // (The exact path: 256 x 256 tiles from one per compute unit on (256 x 128 where k ends inside a step and their rounds are the
-  //  shorter ones), else 128 x 128: 2048 x 4096 x 4096: 94 us on 128 x 128 tiles against 116; 1024 x 8192 x 8192: 164 against 200.  The float8 path: the stream kernel from half a 128 x 128 tile per compute unit on, with the columns
-  //  per tile that suit the shape (us, 128 x 128 tiles / stream: 160 tiles of 512 x 5120 x 8192 61 / 54, 256 of 512 x 8192 x 8192 66 / 56, 258 of
-  //  300 x 11008 x 4096 49 / 33, 288 of 1500 x 3072 x 8192 84 / 56); with fewer tiles the smaller ones leave less of the machine idle.  Where
-  //  it does not serve: 256 x 256 tiles from one per four units on, else 128 x 128.)
+  //  shorter ones), else 128 x 128: 2048 x 4096 x 4096: 94 us on 128 x 128 tiles against 116; 1024 x 8192 x 8192: 164 against 200.  The float8 path: the stream kernel
+  //  where it pays (stream_pays_float8), with the columns per tile that suit the shape; where it does not serve: 256 x 256 tiles from one per
+  //  four units on, else 128 x 128.)
   const uint64_t tiles256 = uint64_t((p.m + 255) / 256) * ((p.n + 255) / 256), cus = uint64_t(compute_units);
-  const uint64_t tiles128 = uint64_t((p.m + 127) / 128) * ((p.n + 127) / 128);
   bool small = false;  // what the stream kernel's products run on where it does not serve
   bool narrow = false;
   if (variant == 0 && (p.out_dtype == VKT_F32 || p.out_dtype == VKT_F16))
     variant = big && tiles256 >= cus ? 6 : 7, narrow = narrow_tiles_float8_wide(p.m, p.n, p.k, uint32_t(cus));
-  else if (variant == 0) variant = 2 * tiles128 > cus ? 11 : 1, small = !(big && 4 * tiles256 > cus);
+  else if (variant == 0) variant = stream_pays_float8(p.m, p.n, p.k, uint32_t(cus)) ? 11 : 1, small = !(big && 4 * tiles256 > cus);
   const uint32_t columns = (variant & ~0x300u) == 11 ? variant >> 8 : 0;  // (bits 8-9: columns per tile, mma_stream.h)
   if (columns) variant = 11;
   if ((variant & 0xff) == 14) return launch_sliced<FA, FB>(p, (variant >> 8) & 31u, mc, stream, err);

@@ -103,4 +103,18 @@ constexpr bool stream_pays_16bit(uint32_t m, uint32_t n, uint64_t batches, uint3
   return !(int8 && k <= 256 && rows128 % 2 && rows256 <= 3);
 }
 
+// The same for float8 operands (bfloat16 and float8 outputs): from half a 128 x 128 tile per compute unit on (us, 128 x 128 / stream: 160 tiles of 512 x
+// 8192 x 5120 61 / 54, 256 of 512 x 8192 x 8192 66 / 56, 258 of 300 x 4096 x 11008 49 / 33, 288 of 1500 x 8192 x 3072 84 / 56; with fewer tiles the smaller
+// ones leave less of the machine idle).  Rows that begin inside a 128-byte line cost a workgroup a line more per row and step: with a long k and
+// little padding in its 256 rows half as many workgroups that each bring in half as much again are the slower ones, while 128 x 128 tiles are one per
+// compute unit at most and 256 x 256 ones fewer than a quarter (256 x 8272 x 12800 68 / 77, 768 x 6224 x 4736 54 / 59, 222 x 8224 x 14912 68 / 72,
+// 512 x 8224 x 4608 67 / 70, 700 x 4128 x 4096 37.0 / 38.5, 911 x 6160 x 2304 53.1 / 54.5, 198 x 6176 x 16000 52.6 / 54.2; 256 x 1104 x 15712 16.9 / 14.7,
+// 192 x 2080 x 16000 24.9 / 23.0, 217 x 3088 x 15744 33.0 / 33.1, 640 x 4112 x 4096 39.1 / 36.8, 143 x 8208 x 13696 66.4 / 63.7, 384 x 8224 x 6400 66.6 / 61.8).
+constexpr bool stream_pays_float8(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) {
+  const uint64_t rows256 = (uint64_t(m) + 255) / 256, tiles256 = rows256 * ((uint64_t(n) + 255) / 256);
+  const uint64_t rows128 = (uint64_t(m) + 127) / 128, tiles128 = rows128 * ((uint64_t(n) + 127) / 128);
+  if (2 * tiles128 <= cus) return false;
+  return !(k % 128 != 0 && k >= 4096 && tiles128 <= cus && 4 * tiles256 <= cus && rows128 % 2 == 0 && uint64_t(m) * 4 >= rows256 * 256 * 3);
+}
+
 }  // namespace vkt
