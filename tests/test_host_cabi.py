@@ -307,3 +307,23 @@ def test_stream_kernel_where_it_pays():
         assert L.shim_stream_pays_float8(m, n, k, 256), (m, k, n)
     for m, k, n in [(512, 8192, 4096), (256, 8272, 12800), (768, 6224, 4736), (222, 8224, 14912), (198, 6176, 16000), (700, 4128, 4096), (512, 8224, 4608)]:
         assert not L.shim_stream_pays_float8(m, n, k, 256), (m, k, n)
+
+
+def test_tile_slices_where_they_pay():
+    """Slices of K of the tile kernel: two that do not divide the steps only where what they save outweighs the partial sums' passes; the partial
+    sums fit the budget and the tiles two workgroups per compute unit."""
+    L = ctypes.CDLL(os.path.join(os.path.dirname(abi.LIB_PATH), "libvkt_hosttest.so"))
+    L.shim_tile_slices.argtypes = [ctypes.c_uint32] * 4 + [ctypes.c_uint64, ctypes.c_int, ctypes.c_int]
+    slices = lambda m, k_bytes, n, float8=0, widened=0: L.shim_tile_slices(m, n, k_bytes, 256, 16 << 20, float8, widened)  # noqa: E731
+    for m, k, n in [(236, 1088, 7424), (432, 1344, 3968), (105, 1032, 10608), (640, 1416, 2200), (384, 1344, 4992), (210, 1216, 5528)]:
+        assert slices(m, 2 * k, n) == 1, (m, k, n)
+    for m, k, n in [(160, 1032, 3200), (128, 1848, 11616), (186, 1216, 4760), (124, 2240, 8944), (128, 1024, 3000)]:
+        assert slices(m, 2 * k, n) == 2, (m, k, n)
+    assert slices(459, 2128, 3984, 1) == 1 and slices(262, 2176, 4480, 1) == 2 and slices(128, 2048, 4000, 1) == 2
+    assert slices(1000, 2064, 2000, 1, 1) == 1 and slices(80, 3456, 1424, 1, 1) == 1 and slices(80, 3456, 1424, 1) == 2 and slices(106, 3088, 2960, 1, 1) == 2
+    assert slices(450, 2 * 4464, 1408) == 4 and slices(100, 17344, 520, 1) == 16 and slices(170, 32000, 2069) == 8
+    for k in range(1024, 40000, 208):
+        for m, n in [(65, 512), (130, 3000), (1000, 2000)]:
+            s = slices(m, k, n)
+            assert 1 <= s <= 16 and s * m * n * 4 <= 16 << 20 and s * ((m + 127) // 128) * ((n + 127) // 128) <= 512
+            assert s == 1 or (k + 127) // 128 >= 8 * s

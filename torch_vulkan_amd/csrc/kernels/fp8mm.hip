@@ -384,7 +384,7 @@ int launch_formats(const F8Params& p, uint32_t variant, const Machine& mc, hipSt
     // over workgroups (mma_slices.h; variant 14 asks for it, bits 8-12: slices)
     if (variant == 0 && p.m > 64) {
       const uint64_t budget = mc.workspace_bytes < VKT_STATIC_SCRATCH_BYTES ? mc.workspace_bytes : VKT_STATIC_SCRATCH_BYTES;
-      const uint32_t slices = tile_slices(p.m, p.n, p.k, uint32_t(mc.compute_units), budget);
+      const uint32_t slices = tile_slices(p.m, p.n, p.k, uint32_t(mc.compute_units), budget, true, p.out_dtype == VKT_F32 || p.out_dtype == VKT_F16);
       if (slices >= 2 && uint64_t((p.m + 127) / 128) * ((p.n + 127) / 128) * 2 <= uint64_t(mc.compute_units)) return launch_sliced<FA, FB>(p, slices, mc, stream, err);
     }
     // 65 to 256 rows against few tiles: the few-row kernel over blocks of 64 rows, where that many passes over the

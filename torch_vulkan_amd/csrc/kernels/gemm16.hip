@@ -257,7 +257,7 @@ int launch_tiles(const GemmParams& p, uint32_t use_cin, uint32_t batch, uint32_t
     if ((variant == 0 || (variant & 0xff) == 10) && batch == 1) {
       const bool asked = (variant & 0xff) == 10;
       const uint64_t budget = mc.workspace_bytes < VKT_STATIC_SCRATCH_BYTES ? mc.workspace_bytes : VKT_STATIC_SCRATCH_BYTES;
-      const uint32_t slices = asked ? (variant >> 8) & 31u : (p.m > 64 ? tile_slices(p.m, p.n, g.k, uint32_t(mc.compute_units), budget) : 1);
+      const uint32_t slices = asked ? (variant >> 8) & 31u : (p.m > 64 ? tile_slices(p.m, p.n, g.k, uint32_t(mc.compute_units), budget, false, false) : 1);
       if (asked && (slices < 2 || slices > (g.k + BK - 1) / BK || uint64_t(slices) * p.m * p.n * 4 > mc.workspace_bytes)) {
         *err = "gemmcm: " + std::to_string(slices) + " slices of K are fewer than 2 or more than its steps of 64 values, or their partial sums do not fit the workspace";
         return -1;

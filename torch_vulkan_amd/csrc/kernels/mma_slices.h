@@ -2,10 +2,10 @@
 // few for the machine: a workgroup of the tile kernel walks all of K, so 128 x 128 tiles of a 128 x 8192 product keep
 // 64 of 256 compute units busy for the whole launch.
 //
-// The tile kernel already runs batches of products; slice s of K is batch s of a product whose operands begin
-// s * (k / slices) bytes into their rows (both operands are rows of k) and whose "outputs" are float32 partial sums in
-// the workspace, [slice][m][n]: SliceProblem is that product (weights stored [k, n]: a slice begins k / slices rows
-// down; the last slice ends where k does).  A second launch adds the slices up in slice order (the result does not depend on timing) and runs the real
+// The tile kernel already runs batches of products; slice s of K is batch s of a product whose operands begin s * per steps of
+// 128 bytes into their rows (both operands are rows of k; per = ceil(steps / slices)) and whose "outputs" are float32 partial sums in
+// the workspace, [slice][m][n]: SliceProblem is that product (weights stored [k, n]: a slice begins s * per * 64 rows
+// down; the last slice ends where k does, and may be as short as 16 bytes).  How many slices: tile_slices, plans.h.  A second launch adds the slices up in slice order (the result does not depend on timing) and runs the real
 // problem's epilogue on 4 consecutive columns of a row, the unit every problem's store<DT>() takes.
 #pragma once
 #include <string>
@@ -14,6 +14,7 @@
 #include "kernels.h"
 #include "limits.h"
 #include "mma_tile.h"
+#include "plans.h"
 
 namespace vkt {
 namespace {
@@ -81,19 +82,6 @@ __global__ __launch_bounds__(256) void mma_slices_finish(Problem p, uint32_t sli
   const auto whole = p.whole();
   const auto cs = p.columns(0, col, whole);
   p.for_output_type(col + 3 < p.n, whole, [&](auto dt) { p.template store<decltype(dt)::value>(0, row, col, sum, cs, whole); });
-}
-
-// How many slices of K serve a product of m rows whose operands are rows of k bytes: a power of two that
-// leaves a slice 1024 bytes and more, brings the 128 x 128 tiles up to two workgroups per compute
-// unit at most, and whose partial sums fit `budget` bytes.  1: the product is not split.  (The slices need not divide
-// the steps: fp8, 111 x 4672 x 11904 and its way back 114 -> 70 us for the two, which went unsplit, or to the few-row
-// kernels, while they had to.)
-inline uint32_t tile_slices(uint32_t m, uint32_t n, uint32_t k_bytes, uint32_t cus, uint64_t budget) {
-  const uint32_t steps = (k_bytes + BK - 1) / BK;
-  const uint64_t tiles = uint64_t((m + 127) / 128) * ((n + 127) / 128);
-  uint32_t s = 1;
-  while (s < 16 && steps / (2 * s) >= 8 && tiles * (2 * s) <= 2ull * cus && uint64_t(2 * s) * m * n * 4 <= budget) s *= 2;
-  return k_slices(steps, s).slices;  // (no empty slice)
 }
 
 // Launches the 128 x 128 tile kernel of the given arithmetic over `slices` slices of K and the second launch.
