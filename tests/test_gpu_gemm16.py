@@ -19,6 +19,11 @@ def close(got, want, mag, dtype):
     assert (np.abs(gf - wf) <= tol).all(), float(np.max(np.abs(gf - wf) - tol))
 
 
+def wider(x):
+    """The bits of a tensor as a view of rows that go on with NaN."""
+    return bits(torch.cat([x, torch.full(x.shape[:-1] + (64,), float("nan"), dtype=x.dtype)], -1))[..., : x.shape[-1]]
+
+
 def col_major(x):
     """The same values with the last two dims stored column by column."""
     return np.ascontiguousarray(np.swapaxes(x, -1, -2)).swapaxes(-1, -2)
@@ -126,7 +131,8 @@ def test_gemm16_few_rows_k_slices(dtype, m, k, n, nt, slices):
 @pytest.mark.parametrize("dtype", DTYPES, ids=str)
 @pytest.mark.parametrize("variant", [0, 9, 9 | 2 << 12, 9 | 3 << 12, 9 | 8 << 12])
 @pytest.mark.parametrize("m,k,n", [(1, 512, 64), (7, 1088, 200), (16, 2048, 1000), (17, 576, 72), (33, 1536, 4104), (64, 2048, 1032), (50, 4096, 520),
-                                   (8, 512, 14344)])  # (one slice, many columns, a short last workgroup)
+                                   (8, 512, 14344),  # (one slice, many columns, a short last workgroup)
+                                   (5, 520, 264), (40, 1032, 200), (64, 2056, 1000)])  # (k ends inside a chunk of 64)
 def test_gemm16_few_rows_weights_in_rows_of_n(dtype, variant, m, k, n):
     """Up to 64 rows against weights stored [k, n] (x @ w) run on the few-row kernel that reads the weights through the
     transposing LDS read: planned and asked for (variant 9), with K in slices over workgroups (slices that do not
@@ -163,7 +169,8 @@ def test_gemm16_few_rows_weights_in_rows_of_n_infinities(dtype):
 @pytest.mark.parametrize("batch,m,k,n,layout,variant", [
     (6, 1, 128, 520, "nt", 0), (5, 8, 128, 200, "nt", 0), (9, 16, 256, 72, "nt", 0),          # rows of k too short to share: a wave per 64 columns
     (3, 16, 2048, 264, "nt", 0), (4, 33, 1024, 130, "nt", 0), (2, 64, 4096, 520, "nt", 7 | 2 << 8 | 4 << 12), (3, 5, 8192, 100, "nt", 0),
-    (7, 1, 1024, 128, "nn", 0), (3, 8, 4096, 128, "nn", 0), (2, 40, 576, 200, "nn", 0), (3, 16, 2048, 72, "nn", 9 | 3 << 12)])
+    (7, 1, 1024, 128, "nn", 0), (3, 8, 4096, 128, "nn", 0), (2, 40, 576, 200, "nn", 0), (3, 16, 2048, 72, "nn", 9 | 3 << 12),
+    (3, 8, 1032, 128, "nn", 0), (2, 33, 2056, 72, "nn", 9 | 3 << 12)])
 def test_gemm16_batched_few_rows(dtype, batch, m, k, n, layout, variant):
     """A batch of few-row products (attention at decode: q @ k.T with rows of k of one head's length, p @ v with the
     values in rows of n) runs on the few-row kernels, a workgroup per batch, column group and slice of K: batch strides
@@ -213,7 +220,8 @@ def test_gemm16_tile_kernel_k_slices_weights_in_rows_of_n(dtype, m, k, n, varian
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=str)
-@pytest.mark.parametrize("batch,m,k,n,layout", [(1, 96, 4104, 520, "nt"), (1, 130, 4096, 264, "nn"), (1, 256, 8200, 72, "nt"), (2, 100, 2048, 128, "nn"), (3, 65, 2048, 200, "nt")])
+@pytest.mark.parametrize("batch,m,k,n,layout", [(1, 96, 4104, 520, "nt"), (1, 130, 4096, 264, "nn"), (1, 256, 8200, 72, "nt"), (2, 100, 2048, 128, "nn"), (3, 65, 2048, 200, "nt"),
+                                              (2, 130, 2056, 72, "nn")])
 def test_gemm16_row_blocks_on_few_row_kernels(dtype, batch, m, k, n, layout):
     """65 to 256 rows against few columns (few tiles for the tile kernels, whose workgroups each walk all of K) run as
     passes of the few-row kernels over blocks of 64 rows: a short last block, both weight layouts, batches, an addend
@@ -265,6 +273,18 @@ def test_gemm16_stream_kernel(dtype):
         if m * n <= 1 << 20:
             want, mag = oracle.gemm16(a, w.transpose(0, 2, 1), ODT[dtype], cin=bias, alpha=2.0, beta=0.5, want_mag=True)
             close(got[6], want, mag, dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("batch,m,k,n,columns", [(3, 300, 200, 392, 2), (3, 300, 200, 392, 3), (70, 260, 128, 136, 3), (40, 257, 136, 520, 0), (150, 200, 72, 264, 2)])
+def test_gemm16_stream_kernel_batches(dtype, batch, m, k, n, columns):
+    """Batches on the stream kernel's tiles of 192 and 128 columns (planned where they have enough tiles), streams that run from one batch into
+    the next at a k that ends inside a step: bit for bit the tile kernel's outputs."""
+    import _dev
+    a = wider((torch.randn(batch, m, k, generator=gen(113)) * 0.5).to(dtype))
+    w = wider((torch.randn(batch, n, k, generator=gen(114)) * 0.5).to(dtype))
+    got = [_dev.gemm16(a, w.transpose(0, 2, 1), ODT[dtype], variant=v) for v in (6 | columns << 8 if columns else 0, 3)]
+    assert np.array_equal(got[0], got[1])
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=str)

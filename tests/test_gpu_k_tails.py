@@ -8,7 +8,7 @@ import torch
 import oracle
 from _util import ODT, bits, gen, unbits
 from test_gpu_fp8mm import FLOAT8, run_case
-from test_gpu_gemm16 import close, col_major
+from test_gpu_gemm16 import close, col_major, wider
 
 pytestmark = pytest.mark.gpu
 DTYPES = [torch.bfloat16, torch.float16]
@@ -40,6 +40,18 @@ def test_rows_of_k_in_wider_rows(dtype, variant, k):
     close(_dev.gemm16(wide(a), wide(w).T, ODT[dtype], variant=variant), want, mag, dtype)
     if variant != 6:
         close(_dev.gemm16(wide(a), np.ascontiguousarray(w.T), ODT[dtype], variant=variant), want, mag, dtype)
+        close(_dev.gemm16(col_major(a[:296]), wide(w).T, ODT[dtype], variant=variant), want[:296], mag[:296], dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("batch,m,k,n,variant", [(1, 5, 520, 264, 0), (1, 40, 1032, 200, 9 | 3 << 12), (1, 64, 2056, 1000, 9), (3, 8, 1032, 128, 0),
+                                                 (2, 130, 2056, 72, 0)])  # (the last: blocks of 64 rows)
+def test_few_rows_against_weights_in_rows_of_n(dtype, batch, m, k, n, variant):
+    """x @ w on the few-row kernel at k that ends inside a chunk of 64, both operands' rows going on with NaN."""
+    import _dev
+    a, w = wider((torch.randn(batch, m, k, generator=gen(36)) * 0.5).to(dtype)), wider((torch.randn(batch, k, n, generator=gen(37)) * 0.5).to(dtype))
+    want, mag = oracle.gemm16(a, w, ODT[dtype], want_mag=True)
+    close(_dev.gemm16(a, w, ODT[dtype], variant=variant), want, mag, dtype)
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=str)
@@ -103,11 +115,10 @@ def test_last_slice_shorter_than_a_step(dtype, layout):
     """The same for 16-bit operands, whose rows go on with NaN."""
     import _dev
     m, k, n = 100, 8672, 264
-    a = bits((torch.randn(m, k, generator=gen(32)) * 0.5).to(dtype))
-    w = bits((torch.randn(n, k, generator=gen(33)) * 0.5).to(dtype))
+    a, w = (wider((torch.randn(rows, k, generator=gen(32 + rows)) * 0.5).to(dtype)) for rows in (m, n))
     want, mag = oracle.gemm16(a, w.T, ODT[dtype], want_mag=True)
-    wide = lambda x: np.concatenate([x, np.full((x.shape[0], 64), 0x7FC1 if dtype == torch.bfloat16 else 0x7E01, np.uint16)], 1)[:, :x.shape[1]]  # noqa: E731
-    close(_dev.gemm16(wide(a), wide(w).T if layout == "nt" else wide(np.ascontiguousarray(w.T)), ODT[dtype]), want, mag, dtype)
+    b = w.T if layout == "nt" else wider(torch.from_numpy(np.ascontiguousarray(w.T).view(np.int16)).view(dtype))
+    close(_dev.gemm16(a, b, ODT[dtype]), want, mag, dtype)
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=str)
