@@ -200,7 +200,9 @@ __global__ __launch_bounds__(512) void mma_stream(P p, uint32_t tiles_m, uint32_
   // What the epilogue costs is the time its stores take to drain (every workgroup stores its tile at about the same
   // time, with the matrix cores idle).  Stores that write 32 or 64 bytes of each of their rows take as long, in any
   // order tried, but put 1.5 times the output's bytes on the way to memory (counted: 201 MiB for the 128 MiB of
-  // 8192 x 8192 bfloat16 outputs); with whole lines the count is the output's size.  Non-temporal stores are 1.5 times
+  // 8192 x 8192 bfloat16 outputs); with whole lines (tiles of 256 and 128 columns) the count is the output's size.  With 192 columns a wave's 96
+  // are a block and a half of two: the third block goes out in halves of a line, and the second wave's pair straddles two lines, so of the
+  // three lines of a row one is written whole (counted: 1.16 times the output's bytes for 1537 x 13824, 1.05 for 1537 x 5120).  Non-temporal stores are 1.5 times
   // slower, and waiting after every few stores, or starting the workgroups a few microseconds apart, only costs.
   auto epilogue = [&](const Tile& t) {
     const uint32_t wm0 = t.m0 + wm * (TM2 * 32), wn0 = t.n0 + wn * (TN2 * 32);

@@ -1068,29 +1068,20 @@ __global__ __launch_bounds__(256) void qmm4m_rows(Q4CParams p, MatrixLayout L, u
       const Set& cur = kInPlace ? sets[i] : taken;
       constexpr int mask = UPB ? UPB - 1 : 0;
       if constexpr (UPB == 1) {
+        static_assert(RT * CT == 1, "blocks of 32 with several tiles per wave: qmm4m_half");
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          long b[CT];
+          const uint32_t v = cur.w[0][j];
+          const long b = long(uint64_t(v & 0x0f0f0f0fu) | uint64_t((v >> 4) & 0x0f0f0f0fu) << 32);
+          const U4& qq = j < 2 ? cur.q0[0] : cur.q1[0];
+          const long a = long(uint64_t(qq[(j & 1) * 2]) | uint64_t(qq[(j & 1) * 2 + 1]) << 32);
+          V4I x = unit_const[0];
+          x = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, x, 0, 0, 0);
+          x = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, minus8, x, 0, 0, 0);
+          x = __builtin_amdgcn_mfma_i32_16x16x32_i8(nz_a[0], b, x, 0, 0, 0);
+          x = __builtin_amdgcn_mfma_i32_16x16x32_i8(nz_b[0], b, x, 0, 0, 0);
 #pragma unroll
-          for (int c = 0; c < CT; ++c) {
-            const uint32_t v = cur.w[c][j];
-            b[c] = long(uint64_t(v & 0x0f0f0f0fu) | uint64_t((v >> 4) & 0x0f0f0f0fu) << 32);
-          }
-#pragma unroll
-          for (int t = 0; t < RT; ++t) {
-            const U4& qq = j < 2 ? cur.q0[t] : cur.q1[t];
-            const long a = long(uint64_t(qq[(j & 1) * 2]) | uint64_t(qq[(j & 1) * 2 + 1]) << 32);
-#pragma unroll
-            for (int c = 0; c < CT; ++c) {
-              V4I x = unit_const[t];
-              x = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b[c], x, 0, 0, 0);
-              x = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, minus8, x, 0, 0, 0);
-              x = __builtin_amdgcn_mfma_i32_16x16x32_i8(nz_a[t], b[c], x, 0, 0, 0);
-              x = __builtin_amdgcn_mfma_i32_16x16x32_i8(nz_b[t], b[c], x, 0, 0, 0);
-#pragma unroll
-              for (int r = 0; r < 4; ++r) acc[t][c][r] = acc[t][c][r] + float(x[r]) * cur.s[c][j];  // in block order
-            }
-          }
+          for (int r = 0; r < 4; ++r) acc[0][0][r] = acc[0][0][r] + float(x[r]) * cur.s[0][j];  // in block order
         }
       } else {
         // Blocks of two units and more: two units, 64 values of k, per matrix-core instruction (the full-rate form).  The sums of
@@ -1213,8 +1204,8 @@ __global__ __launch_bounds__(256) void qmm4m_expand(Q4CParams p, uint64_t dst, u
 // order: at most 64 x 255 x (1039 + 79) / 2 = 9.1e6.  That bounds the blocks to 64 values; longer ones stay on the integer form.
 // What bounds it: vector-unit issue.  Block-by-block float32 sums cost a product and an addition per output and block (8 instructions
 // per unit and tile), the nibbles 5 per unit and column tile, which RT row tiles share.  The integer
-// form (qmm4m_rows) takes 15 and four half-rate products.  2048 x 4096 x 11008, blocks of 32, kernel alone: 527 -> 318 us, 80 % of
-// the vector units' issue at the 2.05 GHz that the card holds in it.  2 x 4 tiles per wave (196 registers: two waves per SIMD) against
+// form (qmm4m_rows) takes 15 and four half-rate products.  2048 x 4096 x 11008, blocks of 32, kernel alone: 527 -> 318 us; vector instructions
+// issue in 84 % of its cycles (counted).  2 x 4 tiles per wave (196 registers: two waves per SIMD) against
 // 2 x 2 and 4 x 2, whole call: 325, 360, 346 us.
 template <class T, int UPB, int RT, int CT>
 __global__ __launch_bounds__(256, 2) void qmm4m_half(Q4CParams p, MatrixLayout L, uint64_t halves, uint32_t m0, uint32_t rows) {
@@ -1224,7 +1215,7 @@ __global__ __launch_bounds__(256, 2) void qmm4m_half(Q4CParams p, MatrixLayout L
   const uint32_t col = lane & 15, kg = lane >> 4;
   // Workgroups to operand panels: workgroup i runs on XCD i % 8, each with an L2 of its own, so an XCD takes a contiguous eighth
   // of an order that walks down kPanel row groups before it moves on to the next column group.  (In the plain order an XCD's 64
-  // workgroups touch 43 column groups: a third of the reads hit L2, 2 GB came from beyond it, 352 us instead of 325.)
+  // workgroups touch 43 column groups: 352 us instead of 325.)
   constexpr uint32_t kPanel = 8;
   const uint32_t col_groups = (L.tiles + 4 * CT - 1) / (4 * CT), row_groups = (rows + 16 * RT - 1) / (16 * RT);
   const uint32_t total = col_groups * row_groups, per = (total + 7) / 8, at = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
