@@ -253,6 +253,13 @@ def test_q4_wave_tiles_count_real_rows(bs):
     assert _q4_form(300, 4096, 11008, bs or k) == "2x2" and _q4_form(64, 4096, 11008, bs or k) == "1x1"
 
 
+def test_q4_wave_tiles_of_blocks_of_256():
+    """Blocks of 256: two row tiles per wave from two waves of them per SIMD on, 2 x 2 where a SIMD has no room for all of those."""
+    for (m, k, n), form in {(64, 4096, 11008): "1x1", (40, 4096, 16384): "2x1", (128, 4096, 8192): "2x1", (150, 4096, 11008): "2x1",
+                            (167, 4608, 12264): "2x2", (200, 4096, 11008): "2x2", (512, 4096, 11008): "2x2"}.items():
+        assert _q4_form(m, k, n, 256) == form, (m, k, n)
+
+
 def test_q4_float16_form_where_it_pays():
     """4-bit products in blocks of 32 and 64: the float16 form takes 32 rows per wave and a longer first pass, so few rows stay on integers;
     blocks of 64, whose integer form is the faster one, longer."""

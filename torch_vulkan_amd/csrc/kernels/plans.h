@@ -38,8 +38,10 @@ constexpr Q4Form q4_rows_form(uint32_t m, uint32_t tiles, uint32_t quads, uint32
   // once, and 2 x 1 pays from there on (us, 1 x 1 / 2 x 1, waves of 1 x 1 in brackets: blocks of 128, 40 x 4096 x 16384 [3072] 23.5 / 28.7, 70 x
   // 8192 x 11008 [3440] 63 / 67, 128 x 2048 x 8192 [4096] 15.9 / 16.9, 128 x 4096 x 8192 [4096] 28.6 / 27.8, 96 x 4096 x 11008 [4128] 38.9 / 33.2;
   // one scale per column, 40 x 4096 x 16384 23.5 / 25.4, 128 x 2048 x 8192 13.1 / 13.5, 96 x 4096 x 11008 28.6 / 27.9).  Blocks of 256: 2 x 1 is
-  // level from two waves of it per SIMD on (40 x 4096 x 16384 20.9 / 21.0, 70 x 4096 x 11008 29.9 / 29.6, 100 x 4096 x 8192 25.1 / 19.8).
-  if (int22 >= 2560) return kQ4Int22;
+  // level from two waves of it per SIMD on (40 x 4096 x 16384 20.9 / 21.0, 70 x 4096 x 11008 29.9 / 29.6, 100 x 4096 x 8192 25.1 / 19.8), and a SIMD has
+  // room for four of its waves: 2 x 2 from more on (2 x 1 / 2 x 2, waves of 2 x 1 in brackets: 180 x 4096 x 11008 [4128] 51.3 / 48.6, 167 x 4608 x 12264
+  // [4602] 73 / 60, 200 x 4096 x 11008 [4816] 53.2 / 49.1).
+  if (int22 >= 2560 || (upb == 8 && int21 > 4096)) return kQ4Int22;
   return (upb == 8 ? int21 >= 2048 : int11 > 4096) ? kQ4Int21 : kQ4Int11;
 }
 
