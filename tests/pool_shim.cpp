@@ -114,6 +114,7 @@ int shim_stream_pays_16bit(uint32_t m, uint32_t n, uint64_t batches, uint32_t k,
 }
 uint32_t shim_stream_columns(uint32_t m, uint32_t n, uint64_t batches, uint32_t cus) { return vkt::mma_stream_tiles(m, n, batches, cus).columns; }
 int shim_stream_pays_float8(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return vkt::stream_pays_float8(m, n, k, cus) ? 1 : 0; }
+int shim_staged_tiles_int8(uint32_t m, uint32_t n, uint32_t k_bytes, uint32_t cus) { return vkt::staged_tiles_int8(m, n, k_bytes, cus) ? 1 : 0; }
 
 // the slices of K of the tile kernel (kernels/plans.h)
 uint32_t shim_tile_slices(uint32_t m, uint32_t n, uint32_t k_bytes, uint32_t cus, uint64_t budget, int float8, int widened) {

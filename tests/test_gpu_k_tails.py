@@ -122,7 +122,7 @@ def test_last_slice_shorter_than_a_step(dtype, layout):
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=str)
-@pytest.mark.parametrize("m,k,n", [(1500, 208, 6000), (400, 80, 8264), (3300, 80, 4901)])
+@pytest.mark.parametrize("m,k,n", [(1500, 208, 6000), (400, 80, 8264), (3300, 80, 4901), (512, 336, 8188)])
 def test_int8_many_rows(dtype, m, k, n):
     import _dev
     a = torch.randn(m, k, generator=gen(29)).to(dtype)

@@ -334,3 +334,13 @@ def test_tile_slices_where_they_pay():
             s = slices(m, k, n)
             assert 1 <= s <= 16 and s * m * n * 4 <= 16 << 20 and s * ((m + 127) // 128) * ((n + 127) // 128) <= 512
             assert s == 1 or (k + 127) // 128 >= 8 * s
+
+
+def test_int8_tiles_staged_where_the_last_round_is_thin():
+    """Many-row int8 products on 128 x 128 tiles at k inside a step: staged through registers where a compute unit's last tile is alone on it."""
+    L = ctypes.CDLL(os.path.join(os.path.dirname(abi.LIB_PATH), "libvkt_hosttest.so"))
+    L.shim_staged_tiles_int8.argtypes = [ctypes.c_uint32] * 4
+    for m, k, n in [(512, 2064, 8188), (1792, 2096, 4730), (2176, 6160, 4198), (2533, 7184, 3428)]:
+        assert L.shim_staged_tiles_int8(m, n, 2 * k, 256) and not L.shim_staged_tiles_int8(m, n, (2 * k + 127) // 128 * 128, 256), (m, k, n)
+    for m, k, n in [(604, 6160, 7645), (808, 7184, 6140), (1603, 1040, 4395)]:
+        assert not L.shim_staged_tiles_int8(m, n, 2 * k, 256), (m, k, n)

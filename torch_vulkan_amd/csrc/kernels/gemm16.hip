@@ -474,6 +474,7 @@ int launch_q8_gemm_t(const Q8Params& p, const Machine& mc, hipStream_t stream, s
   if (large && narrow_tiles_16bit(p.m, p.n, 1, g.k, uint32_t(mc.compute_units)))
     return launch_mma_tile<2, 2, 8, 4, 0, 0, true, false, MATH>(g, mc.compute_units, stream, err, "qmm8");
   if (large) return launch_mma_tile<2, 2, 8, 8, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "qmm8");
+  if (staged_tiles_int8(p.m, p.n, g.k, uint32_t(mc.compute_units))) return launch_mma_tile<2, 2, 4, 4, 0, 0, true, false, MATH>(g, mc.compute_units, stream, err, "qmm8");
   return launch_mma_tile<2, 2, 4, 4, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "qmm8");
 }
 

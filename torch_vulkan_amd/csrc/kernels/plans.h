@@ -67,6 +67,15 @@ constexpr bool narrow_tiles_16bit(uint32_t m, uint32_t n, uint64_t batches, uint
   return k_bytes % 128 != 0 && narrow_tiles_pay(m, n, batches, cus, 65);
 }
 
+// The many-row int8 product on 128 x 128 tiles, k inside a step: loaded into LDS directly, or staged through registers, two steps ahead, where the
+// last round (of two tiles per compute unit) leaves a unit one workgroup, which waits for its own direct loads (us, direct / staged, tiles in brackets: 512 x
+// 2064 x 8188 [256] 55.0 / 49.0, 1792 x 2096 x 4730 [518] 92.0 / 88.5, 2176 x 6160 x 4198 [561] 234 / 215, 2048 x 8240 x 4850 [608] 289 / 279; 604 x 6160 x
+// 7645 [300] 125 / 138, 808 x 7184 x 6140 [336] 134 / 154, 1603 x 1040 x 4395 [455] 39.1 / 39.6).
+constexpr bool staged_tiles_int8(uint32_t m, uint32_t n, uint32_t k_bytes, uint32_t cus) {
+  const uint64_t tiles128 = (uint64_t(m) + 127) / 128 * ((uint64_t(n) + 127) / 128);
+  return k_bytes % 128 != 0 && tiles128 != 0 && (tiles128 - 1) % (2ull * cus) < cus;
+}
+
 // ---- The stream kernel (mma_stream.h): columns per tile of 256 rows.  256, or 192 or 128 where they take fewer or fuller rounds of a tile per
 // compute unit.  A round costs about 100, 81 and 64 parts of the same step (4096 x 14336 x 4096 in bfloat16, full rounds: 106, 86 and 64 us each; 4096
 // x 28672 x 8192 in float8: 102, 83 and 66), and fewer columns read more bytes per product, so a tie goes to the wider tile.  us, 256 / 192 /
