@@ -317,8 +317,8 @@ def test_stream_kernel_where_it_pays():
 
 
 def test_tile_slices_where_they_pay():
-    """Slices of K of the tile kernel: two that do not divide the steps only where what they save outweighs the partial sums' passes; the partial
-    sums fit the budget and the tiles two workgroups per compute unit."""
+    """Slices of K of the tile kernel: a count that does not divide the steps only where what it saves outweighs the partial sums' passes, which
+    are slower where n is no multiple of 4; the partial sums fit the budget and the tiles two workgroups per compute unit."""
     L = ctypes.CDLL(os.path.join(os.path.dirname(abi.LIB_PATH), "libvkt_hosttest.so"))
     L.shim_tile_slices.argtypes = [ctypes.c_uint32] * 4 + [ctypes.c_uint64, ctypes.c_int, ctypes.c_int]
     slices = lambda m, k_bytes, n, float8=0, widened=0: L.shim_tile_slices(m, n, k_bytes, 256, 16 << 20, float8, widened)  # noqa: E731
@@ -328,6 +328,7 @@ def test_tile_slices_where_they_pay():
         assert slices(m, 2 * k, n) == 2, (m, k, n)
     assert slices(459, 2128, 3984, 1) == 1 and slices(262, 2176, 4480, 1) == 2 and slices(128, 2048, 4000, 1) == 2
     assert slices(1000, 2064, 2000, 1, 1) == 1 and slices(80, 3456, 1424, 1, 1) == 1 and slices(80, 3456, 1424, 1) == 2 and slices(106, 3088, 2960, 1, 1) == 2
+    assert slices(196, 2 * 2176, 4569) == 2 and slices(196, 2 * 2176, 4572) == 4
     assert slices(450, 2 * 4464, 1408) == 4 and slices(100, 17344, 520, 1) == 16 and slices(170, 32000, 2069) == 8
     for k in range(1024, 40000, 208):
         for m, n in [(65, 512), (130, 3000), (1000, 2000)]:

@@ -134,25 +134,29 @@ constexpr bool stream_pays_float8(uint32_t m, uint32_t n, uint32_t k, uint32_t c
 // most a power of two that leaves the slices' average 1024 bytes and more, brings the tiles up to two workgroups per compute unit at most,
 // and whose partial sums fit `budget` bytes; slices of whole steps of 128 bytes, the last one shorter (down to one step) where they do
 // not divide.  1: the product is not split.
-// Two slices that do not divide the steps, against no slices (those that do were measured against what came before them): they save half of the
-// steps, 0.87 us each for 16-bit values and 1.3 for float8 (rows that begin inside a line among them), and cost a launch and two passes over the partial
-// sums, 3.5 us and 0.6 per MB (us, none / two slices, steps and MB in brackets: x @ w.T 236 x 1088 x 7424 [17, 14] 15.9 / 19.4, 432 x 1344 x 3968 [21, 14]
-// 18.3 / 21.1, 105 x 1032 x 10608 [17, 9] 16.9 / 18.7, 640 x 1416 x 2200 [23, 11] 20.2 / 21.3, 160 x 1032 x 3200 [17, 4] 16.4 / 13.9, 128 x 1848 x 11616 [29,
-// 12] 29.2 / 23.6; x @ w 384 x 1344 x 4992 [21, 15] 18.0 / 21.5, 186 x 1216 x 4760 [19, 7] 16.9 / 15.5; float8 459 x 2128 x 3984 [17, 15] 21.5 / 22.8, 262 x 2176 x
-// 4480 [17, 9] 20.1 / 18.1, 1000 x 2064 x 2000 [17, 16] with float32 outputs 25.4 / 26.5).  Four and more saved time wherever they were tried.
+// Counts that divide the steps are taken as they are (they were measured against what came before them).  One that does not is weighed against the
+// largest that does: it saves steps, 0.87 us each for 16-bit values and 1.3 for float8 (rows that begin inside a line among them), and costs, from no slices
+// on, a launch, 3.5 us, and two passes over its partial sums, 0.6 us per MB, 1.4 where n is no multiple of 4 and they move one by one (us, without / with,
+// slices, steps and MB in brackets: x @ w.T 236 x 1088 x 7424 [1, 2, 17, 14] 15.9 / 19.4, 432 x 1344 x 3968 [1, 2, 21, 14] 18.3 / 21.1, 105 x 1032 x 10608 [1,
+// 2, 17, 9] 16.9 / 18.7, 640 x 1416 x 2200 [1, 2, 23, 11] 20.2 / 21.3, 196 x 2176 x 4569 [2, 4, 34, 14] 26.0 / 29.1, 160 x 1032 x 3200 [1, 2, 17, 4] 16.4 / 13.9, 128 x
+// 1848 x 11616 [1, 2, 29, 12] 29.2 / 23.6, 170 x 16000 x 2069 [2, 8, 250, 11] 90 / 47; x @ w 384 x 1344 x 4992 [1, 2, 21, 15] 18.0 / 21.5, 186 x 1216 x 4760 [1, 2, 19, 7]
+// 16.9 / 15.5; float8 459 x 2128 x 3984 [1, 2, 17, 15] 21.5 / 22.8, 262 x 2176 x 4480 [1, 2, 17, 9] 20.1 / 18.1, 1000 x 2064 x 2000 [1, 2, 17, 16] with float32
+// outputs 25.4 / 26.5).
 // widened: float8 operands widened to bfloat16.  Up to 80 rows of those take the few-row kernel's second pass, of 16 rows, instead of two
 // uneven slices (80 x 3456 x 1424 16.8 / 19.9, 79 x 3712 x 3480 19.1 / 21.2; 106 x 3088 x 2960 20.2 / 20.1).
 constexpr uint32_t tile_slices(uint32_t m, uint32_t n, uint32_t k_bytes, uint32_t cus, uint64_t budget, bool float8, bool widened) {
   const uint32_t steps = k_bytes / 128 + (k_bytes % 128 != 0);
   const uint64_t tiles = (uint64_t(m) + 127) / 128 * ((uint64_t(n) + 127) / 128), plane = uint64_t(m) * n * 4;
-  uint32_t s = 1;
-  while (s < 16 && steps / (2 * s) >= 8 && tiles * (2 * s) <= 2ull * cus && 2 * s * plane <= budget) s *= 2;
-  const KSlices cut = k_slices(steps, s);  // (no empty slice)
-  if (s == 2 && (k_bytes % 128 != 0 || steps % 2 != 0)) {
-    const uint64_t saved_ns = uint64_t(steps - cut.chunks_per_slice) * (float8 ? 1300 : 870);
-    if (saved_ns * 10000 < 35000000 + 2 * plane * 6 || (widened && m <= 80)) return 1;  // (0.6 ns per 1000 bytes)
-  }
-  return cut.slices;
+  uint32_t most = 1;
+  while (most < 16 && steps / (2 * most) >= 8 && tiles * (2 * most) <= 2ull * cus && 2 * most * plane <= budget) most *= 2;
+  uint32_t best = 1;
+  while (k_bytes % 128 == 0 && best < most && steps % (2 * best) == 0) best *= 2;
+  // (in units of 0.1 ns: a step, the launch, 0.6 or 1.4 us per MB)
+  const uint64_t step = float8 ? 13000 : 8700, per_kb = n % 4 == 0 ? 6 : 14;
+  auto time = [&](uint32_t s) { return (steps + s - 1) / s * step + (s > 1 ? 35000 + s * plane * per_kb / 1000 : 0); };
+  for (uint32_t s = 2 * best; s <= most; s *= 2)
+    if (time(s) < time(best) && !(widened && m <= 80 && s == 2)) best = s;
+  return k_slices(steps, best).slices;  // (no empty slice)
 }
 
 }  // namespace vkt
