@@ -281,7 +281,8 @@ typedef struct MinMaxParams {
 /* "fp8mm", spec {}: out = cast((f32(A)*sa) @ (f32(B)*sb) + bias) [* 1/scale_result]
  * (quant.cpp:279-300 fused into one kernel).  A: fp8 [m,k] row-major (lda bytes);
  * B: fp8, column-major, i.e. [n,k] rows ldb bytes apart.  104 bytes.  An optional entry overrides the launcher's
- * choice of kernel (tests, tuning; 0 or absent: planned): 1-9 tile shapes, 11 the stream kernel, 12 the few-row kernel
+ * choice of kernel (tests, tuning; 0 or absent: planned): 1-9 tile shapes, 11 the stream kernel (bits 8-9: 1, 2, 3 for 256,
+ * 192, 128 columns per tile), 12 the few-row kernel
  * (up to 64 rows; bits 8-11: 16s of columns per workgroup, bits 12-16: slices of K over workgroups), 13 the vector-unit
  * kernel (up to 4 rows), 14 the 128 x 128 tile kernel with K in slices over workgroups (bits 8-12: slices, at most
  * k's steps of 128 bytes), 255 one thread per output. */
