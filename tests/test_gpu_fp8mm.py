@@ -324,6 +324,26 @@ def test_scaled_mm_stream_kernel_columns(m, k, n, columns):
         assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("columns", [1, 2, 3])
+@pytest.mark.parametrize("m,k,n", [(1, 16, 1), (257, 128, 7), (300, 144, 261), (130, 400, 387), (255, 256, 130)])
+def test_scaled_mm_stream_kernel_any_columns(m, k, n, columns):
+    """Any number of columns, one step of k and a part of one: the tile kernel's bits, and the oracle's values."""
+    import _dev
+    a = torch.randn(m, k, generator=gen(1101)).to(FLOAT8[0])
+    bt = torch.randn(n, k, generator=gen(1102)).to(FLOAT8[0])
+    sa = torch.empty(m, 1).uniform_(0.5, 2, generator=gen(1103)).numpy()
+    sb = torch.empty(1, n).uniform_(0.5, 2, generator=gen(1104)).numpy()
+    bias = torch.randn(n, generator=gen(1105)).numpy()
+    for odt in (oracle.BF16, oracle.E4M3):
+        kw = dict(bias=bias, bias_dtype=oracle.F32, out_dtype=odt)
+        got, tile = (_dev.scaled_mm(bits(a), oracle.E4M3, bits(bt), oracle.E4M3, sa, sb, True, variant=v, **kw) for v in (11 | columns << 8, 1))
+        assert np.array_equal(got, tile)
+    want, mag = oracle.scaled_mm(bits(a), oracle.E4M3, bits(bt), oracle.E4M3, sa, sb, True, bias, oracle.F32, None, oracle.BF16, want_mag=True)
+    want = oracle.to_f32(want, oracle.BF16).astype(np.float64)
+    got = _dev.scaled_mm(bits(a), oracle.E4M3, bits(bt), oracle.E4M3, sa, sb, True, bias=bias, bias_dtype=oracle.F32, out_dtype=oracle.BF16, variant=11 | columns << 8)
+    assert (np.abs(oracle.to_f32(got, oracle.BF16) - want) <= ref_tol(want, mag, oracle.BF16) + HW_WINDOW * mag).all()
+
+
 def test_scaled_mm_stream_kernel_nan_and_inf():
     """NaN and infinities through the stream kernel's epilogue, whose bfloat16 conversion looks at its values one by one
     only where a wave has seen a NaN: NaN operands (both e4m3fn codes), e5m2 infinities of both signs (inf - inf and

@@ -288,6 +288,43 @@ def test_gemm16_stream_kernel_batches(dtype, batch, m, k, n, columns):
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("columns", [0, 1, 2, 3])  # planned, 256, 192 (k-major second operand: 128), 128 per tile
+@pytest.mark.parametrize("layout", ["nt", "nn", "tn", "tt"])
+@pytest.mark.parametrize("m,k,n", [(8, 8, 8), (264, 64, 136), (248, 72, 520), (520, 200, 264), (256, 392, 1032)])
+def test_gemm16_stream_kernel_layouts(dtype, columns, layout, m, k, n):
+    """Operands in rows of k and k-major ones on the stream kernel: one step of k and a part of one, edges of tiles, beta and a bias; bit for
+    bit the tile kernel's outputs.  Rows go on with NaN."""
+    import _dev
+    a = (torch.randn(2, m, k, generator=gen(130)) * 0.5).to(dtype)
+    b = (torch.randn(2, k, n, generator=gen(131)) * 0.5).to(dtype)
+    want, mag = oracle.gemm16(bits(a), bits(b), ODT[dtype], want_mag=True)
+    x = wider(a) if layout[0] == "n" else wider(a.transpose(1, 2).contiguous()).transpose(0, 2, 1)
+    y = wider(b) if layout[1] == "n" else wider(b.transpose(1, 2).contiguous()).transpose(0, 2, 1)
+    got = _dev.gemm16(x, y, ODT[dtype], variant=6 | columns << 8)
+    close(got, want, mag, dtype)
+    assert np.array_equal(got, _dev.gemm16(x, y, ODT[dtype], variant=4))
+    bias = bits(torch.randn(n, generator=gen(132)).to(dtype))
+    want, mag = oracle.gemm16(bits(a), bits(b), ODT[dtype], cin=bias, alpha=2.0, beta=0.5, want_mag=True)
+    close(_dev.gemm16(x, y, ODT[dtype], cin=bias, alpha=2.0, beta=0.5, variant=6 | columns << 8), want, mag, dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("columns", [1, 2, 3])
+@pytest.mark.parametrize("batch,m,k,n", [(1, 1, 8, 1), (1, 257, 136, 7), (2, 300, 72, 261), (1, 64, 200, 387), (2, 255, 64, 130)])
+def test_gemm16_stream_kernel_any_columns(dtype, columns, batch, m, k, n):
+    """Any number of columns: 8 outputs of a row that begin at any even address, and fewer than 8 at a row's end."""
+    import _dev
+    a = wider((torch.randn(batch, m, k, generator=gen(133)) * 0.5).to(dtype))
+    w = wider((torch.randn(batch, n, k, generator=gen(134)) * 0.5).to(dtype))
+    bias = bits(torch.randn(n, generator=gen(135)).to(dtype))
+    kw = dict(cin=bias, alpha=2.0, beta=0.5)
+    want, mag = oracle.gemm16(a, w.transpose(0, 2, 1), ODT[dtype], want_mag=True, **kw)
+    got = _dev.gemm16(a, w.transpose(0, 2, 1), ODT[dtype], variant=6 | columns << 8, **kw)
+    close(got, want, mag, dtype)
+    assert np.array_equal(got, _dev.gemm16(a, w.transpose(0, 2, 1), ODT[dtype], variant=4, **kw))
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
 def test_gemm16_stream_kernel_nan_and_inf(dtype):
     """NaN and infinities through the stream kernel's epilogue (its bfloat16 conversion looks at its values one by one
     only where a wave has seen a NaN): a NaN operand of either sign, infinities of both signs in one column (inf - inf)

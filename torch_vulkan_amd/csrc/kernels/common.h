@@ -36,6 +36,23 @@ __device__ __forceinline__ void stg(uint64_t addr, X v) {
   *reinterpret_cast<VKT_GLOBAL X*>(addr) = v;
 }
 
+// 16 bytes at an address that is a multiple of 2 (the memory pipeline takes any; the compiler has to be told).
+struct __attribute__((packed, aligned(2))) U4Unaligned {
+  U4 v;
+};
+__device__ __forceinline__ void stg_unaligned(uint64_t addr, const U4& v) { reinterpret_cast<VKT_GLOBAL U4Unaligned*>(addr)->v = v; }
+
+// 8 16-bit outputs of a row of n columns, from column `col` < n on, those past the last column left out, at any address.
+__device__ __forceinline__ void store8_ragged(uint64_t addr, uint32_t col, uint32_t n, const uint32_t (&w)[4]) {
+  if (col + 8 <= n) {
+    stg_unaligned(addr, U4{w[0], w[1], w[2], w[3]});
+  } else {
+#pragma unroll
+    for (uint32_t e = 0; e < 8; ++e)
+      if (col + e < n) stg<uint16_t>(addr + 2 * e, uint16_t(w[e / 2] >> (16 * (e & 1))));
+  }
+}
+
 // A store of data that this kernel does not read again (a streamed output): non-temporal.
 template <class X>
 __device__ __forceinline__ void stg_stream(uint64_t addr, X v) {
@@ -49,6 +66,12 @@ template <int OFF>
 __device__ __forceinline__ void load_to_lds(uint32_t offset, uint64_t base, uint32_t lds_at) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3" ::"v"(offset), "s"(base), "s"(lds_at), "i"(OFF)
                : "memory");
+}
+
+// The same with a 64-bit address per lane.
+template <int OFF>
+__device__ __forceinline__ void load_to_lds_at(uint64_t address, uint32_t lds_at) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off offset:%2" ::"v"(address), "s"(lds_at), "i"(OFF) : "memory");
 }
 
 __device__ __forceinline__ float bits_f32(uint32_t u) { return __builtin_bit_cast(float, u); }

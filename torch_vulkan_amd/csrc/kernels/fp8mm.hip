@@ -123,11 +123,6 @@ struct F8Problem : F8Params {
         if (col + r < n) store_out(*this, index + r, v[r]);
     }
   }
-  // the epilogue that stores straight from the accumulators: bfloat16 outputs, 16-byte aligned rows
-  static constexpr bool kRegisterEpilogue = true;
-  __device__ __forceinline__ bool register_epilogue(const Whole&) const {
-    return out_dtype == VKT_BF16 && (ldo & 7u) == 0 && (out & 15u) == 0;
-  }
   __device__ __forceinline__ float row_scale(uint32_t row, const Whole& w) const {
     return rowwise ? ldg<float>(scale_a + 4ull * row) : w.sa_all;
   }
@@ -141,9 +136,6 @@ struct F8Problem : F8Params {
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) b[r] = bias ? load_any_f32(bias, col + r, bias_dtype) : -0.0f;  // (adding -0.0f changes nothing, a zero's sign included)
-  }
-  __device__ __forceinline__ void store_bf16x8(uint32_t, uint32_t row, uint32_t col, const U4& v) const {
-    stg<U4>(out + (uint64_t(row) * ldo + col) * 2, v);
   }
   // the stream kernel's epilogue (bfloat16 or float8 outputs)
   struct Rows {
@@ -159,6 +151,27 @@ struct F8Problem : F8Params {
     return c;
   }
   __device__ __forceinline__ bool narrow(const Whole&) const { return out_dtype != VKT_BF16; }
+  __device__ __forceinline__ bool ragged(const Whole&) const { return ((n | ldo | (out_dtype == VKT_BF16 ? uint32_t(out) / 2 | (uint32_t(out) & 1u) : uint32_t(out))) & 7u) != 0; }
+  __device__ __forceinline__ Columns4 columns4_ragged(uint32_t, uint32_t col, const Whole& w) const {
+    Columns4 c;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const uint32_t nn = col + r < n ? col + r : n - 1;
+      c.scale[r] = rowwise ? ldg<float>(scale_b + 4ull * nn) : w.sb_all;
+      c.bias[r] = bias ? load_any_f32(bias, nn, bias_dtype) : -0.0f;
+    }
+    return c;
+  }
+  __device__ __forceinline__ void store_ragged(uint32_t, uint32_t row, uint32_t col, const uint32_t (&w)[4], const Whole& whole) const {
+    const uint64_t index = uint64_t(row) * ldo + col;
+    if (!narrow(whole)) {
+      store8_ragged(out + index * 2, col, n, w);
+    } else {
+#pragma unroll
+      for (uint32_t e = 0; e < 8; ++e)
+        if (col + e < n) stg<uint8_t>(out + index + e, uint8_t(w[e / 4] >> (8 * (e & 3))));
+    }
+  }
   __device__ __forceinline__ void finish4(uint32_t, uint32_t, uint32_t, const float (&t)[4], const Rows& r, const Columns4& c, const Whole&,
                                           float (&v)[4]) const {
 #pragma unroll
@@ -338,25 +351,25 @@ int launch_sliced(const F8Params& p0, uint32_t slices, const Machine& mc, hipStr
     *err = "fp8mm: " + std::to_string(slices) + " slices of K are fewer than 2 or more than its steps of 128 bytes, or their partial sums do not fit the workspace";
     return -1;
   }
-  if (p0.out_dtype == VKT_F32 || p0.out_dtype == VKT_F16) return launch_tile_slices<FA, FB, true, kMathFp8Wide>(p, slices, mc, stream, err, "fp8mm");
-  return launch_tile_slices<FA, FB, false, kMathFp8>(p, slices, mc, stream, err, "fp8mm");
+  if (p0.out_dtype == VKT_F32 || p0.out_dtype == VKT_F16) return launch_tile_slices<FA, FB, kMathFp8Wide>(p, slices, mc, stream, err, "fp8mm");
+  return launch_tile_slices<FA, FB, kMathFp8>(p, slices, mc, stream, err, "fp8mm");
 }
 
-template <int WAVES_M, int WAVES_N, int TM, int TN, int FA, int FB, bool MF32 = false, bool DIRECT = false, bool WIDE = false>
+template <int WAVES_M, int WAVES_N, int TM, int TN, int FA, int FB, bool DIRECT = false, bool WIDE = false>
 int launch_tile(const F8Params& p, int compute_units, hipStream_t stream, std::string* err) {
   F8Problem problem;
   static_cast<F8Params&>(problem) = p;
-  return launch_mma_tile<WAVES_M, WAVES_N, TM, TN, FA, FB, MF32, DIRECT, WIDE ? kMathFp8Wide : kMathFp8>(
+  return launch_mma_tile<WAVES_M, WAVES_N, TM, TN, FA, FB, DIRECT, WIDE ? kMathFp8Wide : kMathFp8>(
       problem, compute_units, stream, err, "fp8mm");
 }
 
-// The stream kernel, where it serves the problem (bfloat16 or float8 output in aligned rows); -2: it does not.
+// The stream kernel, where it serves the problem (bfloat16 or float8 output, row strides that its offsets hold); -2: it does not.
 template <int FA, int FB>
 int launch_stream(const F8Params& p, uint32_t columns, int compute_units, hipStream_t stream, std::string* err) {
   F8Problem problem;
   static_cast<F8Params&>(problem) = p;
   const bool float8_out = p.out_dtype == VKT_E4M3 || p.out_dtype == VKT_E5M2;
-  if (!(p.out_dtype == VKT_BF16 || float8_out) || p.ldo % 8 || p.out % (float8_out ? 8 : 16) || !mma_stream_serves(problem)) return -2;
+  if (!(p.out_dtype == VKT_BF16 || float8_out) || !mma_stream_strides_ok(p.lda, p.ldb)) return -2;
   return launch_mma_stream<FA, FB, kMathFp8>(problem, columns, compute_units, stream, err, "fp8mm");
 }
 
@@ -364,12 +377,9 @@ template <int FA, int FB>
 int launch_formats(const F8Params& p, uint32_t variant, const Machine& mc, hipStream_t stream, std::string* err) {
   const int compute_units = mc.compute_units;
   // variant 0: planned.  Explicit variants run the MFMA kernel whatever the output dtype
-  // (tests, tuning): 1: 128x128 tiles (4 waves of 64x64, 16x16x128 MFMA); 2: 256x256 (4 waves of
-  // 128x128, 16x16x128); 3: 256x128; 4: 256x256 with the 32x32x64 MFMA (measured ~10 % faster
-  // than 16x16x128 at equal work); 5: as 4 with global-to-LDS direct loads; 8: as 5 with 8 waves of 64x128 instead of 4 of 128x128 (two waves per SIMD cover each
-  // other's waits: 8192^3 2.34-2.42 -> 2.56-2.59 PFLOP/s; what they get where the stream kernel does not serve).  11: the stream kernel of
-  // mma_stream.h where it serves the problem (large bfloat16 and float8 outputs get it), else 8.  255: the one-thread-per-output kernel.
-  // 6 / 7: the exact path (float8 widened to bfloat16 in registers, 32x32x16 bfloat16 MFMA) on
+  // (tests, tuning): 1 (and 2 to 5 and 8, once names of other tiles): 128x128 tiles (4 waves of 64x64); 11: the stream kernel of
+  // mma_stream.h where it serves the problem (large bfloat16 and float8 outputs get it), else 1.  255: the one-thread-per-output kernel.
+  // 6 (and 9) / 7: the exact path (float8 widened to bfloat16 in registers, 32x32x16 bfloat16 MFMA) on
   // 256x256 / 128x128 tiles: what float32 and float16 outputs get.
   const bool big = uint64_t(p.m) * p.n >= (1ull << 20);
   if (variant == 0 || variant == 13) {  // 13: the vector-unit kernel for one and two rows where it serves (what they get), else as planned
@@ -416,35 +426,32 @@ int launch_formats(const F8Params& p, uint32_t variant, const Machine& mc, hipSt
   }
   // (The exact path: 256 x 256 tiles from one per compute unit on (256 x 128 where k ends inside a step and their rounds are the
   //  shorter ones), else 128 x 128: 2048 x 4096 x 4096: 94 us on 128 x 128 tiles against 116; 1024 x 8192 x 8192: 164 against 200.  The float8 path: the stream kernel
-  //  where it pays (stream_pays_float8), with the columns per tile that suit the shape; where it does not serve: 256 x 256 tiles from one per
-  //  four units on, else 128 x 128.)
+  //  where it pays (stream_pays_float8), with the columns per tile that suit the shape, else 128 x 128.)
   const uint64_t tiles256 = uint64_t((p.m + 255) / 256) * ((p.n + 255) / 256), cus = uint64_t(compute_units);
-  bool small = false;  // what the stream kernel's products run on where it does not serve
   bool narrow = false;
   if (variant == 0 && (p.out_dtype == VKT_F32 || p.out_dtype == VKT_F16))
     variant = big && tiles256 >= cus ? 6 : 7, narrow = narrow_tiles_float8_wide(p.m, p.n, p.k, uint32_t(cus));
-  else if (variant == 0) variant = stream_pays_float8(p.m, p.n, p.k, uint32_t(cus)) ? 11 : 1, small = !(big && 4 * tiles256 > cus);
+  else if (variant == 0) variant = stream_pays_float8(p.m, p.n, p.k, uint32_t(cus)) ? 11 : 1;
   const uint32_t columns = (variant & ~0x300u) == 11 ? variant >> 8 : 0;  // (bits 8-9: columns per tile, mma_stream.h)
   if (columns) variant = 11;
   if ((variant & 0xff) == 14) return launch_sliced<FA, FB>(p, (variant >> 8) & 31u, mc, stream, err);
   switch (variant) {
     case 6:
-      if (narrow) return launch_tile<2, 2, 8, 4, FA, FB, true, false, true>(p, compute_units, stream, err);
-      return launch_tile<2, 2, 8, 8, FA, FB, true, true, true>(p, compute_units, stream, err);
-    case 7: return launch_tile<2, 2, 4, 4, FA, FB, true, false, true>(p, compute_units, stream, err);
-    case 1: return launch_tile<2, 2, 4, 4, FA, FB>(p, compute_units, stream, err);
-    case 2: return launch_tile<2, 2, 8, 8, FA, FB>(p, compute_units, stream, err);
-    case 3: return launch_tile<2, 2, 8, 4, FA, FB>(p, compute_units, stream, err);
-    case 4: return launch_tile<2, 2, 8, 8, FA, FB, true>(p, compute_units, stream, err);
-    case 9: return launch_tile<4, 2, 4, 8, FA, FB, true, true, true>(p, compute_units, stream, err);  // as 6 with 8 waves of 64x128
-    case 11: {  // the stream kernel (mma_stream.h), else 8
+    case 9:
+      if (narrow) return launch_tile<2, 2, 8, 4, FA, FB, false, true>(p, compute_units, stream, err);
+      return launch_tile<2, 2, 8, 8, FA, FB, true, true>(p, compute_units, stream, err);
+    case 7: return launch_tile<2, 2, 4, 4, FA, FB, false, true>(p, compute_units, stream, err);
+    case 11: {  // the stream kernel (mma_stream.h), else 128 x 128 tiles
       const int rc = launch_stream<FA, FB>(p, columns, compute_units, stream, err);
       if (rc != -2) return rc;
-      if (small) return launch_tile<2, 2, 4, 4, FA, FB>(p, compute_units, stream, err);
     }
       [[fallthrough]];
-    case 8: return launch_tile<4, 2, 4, 8, FA, FB, true, true>(p, compute_units, stream, err);  // 256x256 tiles over 8 waves of 64x128 (two waves per SIMD), direct loads
-    case 5: return launch_tile<2, 2, 8, 8, FA, FB, true, true>(p, compute_units, stream, err);
+    case 1:
+    case 2:
+    case 3:
+    case 4:
+    case 5:
+    case 8: return launch_tile<2, 2, 4, 4, FA, FB>(p, compute_units, stream, err);
   }
   *err = "fp8mm: unknown variant " + std::to_string(variant);
   return -1;

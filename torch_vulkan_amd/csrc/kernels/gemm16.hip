@@ -29,7 +29,7 @@ __device__ __forceinline__ float slot_float(uint64_t slot) { return bits_f32(uin
 template <class T, bool TRA = false, bool TRB = false>
 struct GemmProblem {
   static constexpr bool kTransA = TRA, kTransB = TRB;
-  static constexpr bool kRegisterEpilogue = false, kSliced = false;
+  static constexpr bool kSliced = false;
   // operands as the tile kernel takes them (bytes)
   uint64_t a, b;
   uint32_t m, n, k, lda, ldb, batches;
@@ -75,9 +75,14 @@ struct GemmProblem {
     if (w.vec_ok && full) f(std::integral_constant<int, T::dtype>{});
     else f(std::integral_constant<int, -1>{});
   }
-  // the stream kernel's epilogue (C rows and batches 16-byte aligned)
+  // the stream kernel's epilogue
   struct Rows {};
   struct Columns4 {};
+  __device__ __forceinline__ bool ragged(const Whole&) const { return ((n | uint32_t(c_sm) | uint32_t(c_sb) | uint32_t(c) / 2) & 7u) != 0; }
+  __device__ __forceinline__ Columns4 columns4_ragged(uint32_t, uint32_t, const Whole&) const { return Columns4{}; }
+  __device__ __forceinline__ void store_ragged(uint32_t batch, uint32_t row, uint32_t col, const uint32_t (&w)[4], const Whole&) const {
+    store8_ragged(c + uint64_t((int64_t(batch) * c_sb + int64_t(row) * c_sm + int64_t(col)) * 2), col, n, w);
+  }
   __device__ __forceinline__ Rows rows(uint32_t, uint32_t, const Whole&) const { return Rows{}; }
   __device__ __forceinline__ Columns4 columns4(uint32_t, uint32_t, const Whole&) const { return Columns4{}; }
   __device__ __forceinline__ bool narrow(const Whole&) const { return false; }
@@ -87,7 +92,7 @@ struct GemmProblem {
     for (int r = 0; r < 4; ++r) {
       v[r] = alpha * t[r];
       if (cin != 0) {  // beta == 0 never reads Cin (it may hold NaN): then cin is 0
-        const int64_t at = int64_t(batch) * cin_sb + int64_t(row) * cin_sm + int64_t(col + r) * cin_sn;
+        const int64_t at = int64_t(batch) * cin_sb + int64_t(row) * cin_sm + int64_t(col + r < n ? col + r : n - 1) * cin_sn;
         v[r] += beta * load_f32<T>(cin + uint64_t(at * 2));
       }
     }
@@ -263,7 +268,7 @@ int launch_tiles(const GemmParams& p, uint32_t use_cin, uint32_t batch, uint32_t
         return -1;
       }
       if (asked || (slices >= 2 && uint64_t((p.m + 127) / 128) * ((p.n + 127) / 128) * 2 <= uint64_t(mc.compute_units)))
-        return launch_tile_slices<0, 0, true, MATH>(g, slices, mc, stream, err, "gemmcm");
+        return launch_tile_slices<0, 0, MATH>(g, slices, mc, stream, err, "gemmcm");
     }
   }
   if ((variant & 0xff) == 10) variant = 0;
@@ -298,38 +303,32 @@ int launch_tiles(const GemmParams& p, uint32_t use_cin, uint32_t batch, uint32_t
       }
     }
   }
-  // variant 0: planned; 1: 128x128 tiles; 2: 256x128 (planned for a k that ends inside a step); 3: 256x256 with direct loads; 4: 128x128 with direct loads;
-  // 5: 256x256 with direct loads over 8 waves; 6: the stream kernel (mma_stream.h; else 3)
-  // (k-major operands run on the direct forms only)
-  uint32_t small = 3;  // what the stream kernel's products run on where it does not serve
+  // variant 0: planned; 1: 128x128 tiles; 2: 256x128 (planned for a k that ends inside a step); 3 and 5: 256x256 with direct loads; 4: 128x128 with direct loads;
+  // 6: the stream kernel (mma_stream.h; bits 8-9: columns per tile), else, where row strides are too large for it, 3
+  // (k-major operands: 4 in the place of 3 and 5; no 1 and 2)
+  uint32_t small = TRA || TRB ? 4 : 3;  // what the stream kernel's products run on where it does not serve
   if (variant == 0) {
     // 256 x 256 tiles where they give every compute unit one, else 128 x 128
     // (from five eighths of a tile per unit on: 1024 x 4096 x 14336 is 224 tiles on 256 units, 121 us on the stream
     //  kernel against 163 on 128 x 128 tiles; 168 tiles: 142 against 152; at 128 tiles the small tiles are level or ahead)
     const bool large = uint64_t((p.m + 255) / 256) * ((p.n + 255) / 256) * batch * 8 >= uint64_t(mc.compute_units) * 5;
-    // (both operands k-major: 8 waves, whose transposing LDS reads cover each other: 8192^3 0.94 -> 1.11-1.13 PFLOP/s;
-    //  with k-contiguous operands the 8-wave form reads 1.5x the LDS bytes and is 3-5 % slower)
-    variant = large ? (TRA && TRB ? 5 : 3) : (TRA || TRB ? 4 : 1);
-    // both operands contiguous along k (x @ w.T): the stream kernel where it serves (8192^3: 0.94-1.00 -> 0.89 ms), with the columns per
-    // tile that suit the shape also below that line
-    const bool more = stream_pays_16bit(p.m, p.n, batch, p.k, uint32_t(mc.compute_units), false);
-    if (!TRA && !TRB && (variant == 3 || more))
-      small = variant == 3 && narrow_tiles_16bit(p.m, p.n, batch, g.k, uint32_t(mc.compute_units)) ? 2 : variant, variant = 6;
+    // the stream kernel, with the columns per tile that suit the shape (both operands contiguous along k, x @ w.T: also below that line)
+    const bool more = !TRA && !TRB && stream_pays_16bit(p.m, p.n, batch, p.k, uint32_t(mc.compute_units), false);
+    const uint32_t tiles128 = !TRA && !TRB && g.k % BK != 0 ? 1 : 4;  // (mma_tile.h: why k that ends inside a step is staged)
+    if (!TRA && !TRB) small = !large ? tiles128 : narrow_tiles_16bit(p.m, p.n, batch, g.k, uint32_t(mc.compute_units)) ? 2 : 3;
+    variant = large || more ? 6 : tiles128;
   }
-  const bool stream_ok = g.k > BK && p.n % 8 == 0 && p.c_sm % 8 == 0 && p.c_sb % 8 == 0 && p.c % 16 == 0 &&
-                         mma_stream_strides_ok(g.lda, g.ldb);
-  const uint32_t columns = (variant & ~0x300u) == 6 ? variant >> 8 : 0;  // (bits 8-9: columns per tile, mma_stream.h)
-  if ((variant & ~0x300u) == 6) variant = stream_ok ? 6 : small;
+  const uint32_t columns = (variant & ~0x300u) == 6 ? variant >> 8 : 0;
+  if ((variant & ~0x300u) == 6) {
+    if (mma_stream_strides_ok(g.lda, g.ldb)) return launch_mma_stream<0, 0, MATH>(g, columns, mc.compute_units, stream, err, "gemmcm");
+    variant = small;
+  }
   if constexpr (!TRA && !TRB) {
-    // 6: the stream kernel (mma_stream.h) where it serves the problem: more than 64 values of k, n a multiple of 8, C in 16-byte aligned rows
-    if (variant == 6) return launch_mma_stream<0, 0, MATH>(g, columns, mc.compute_units, stream, err, "gemmcm");
-    if (variant == 1) return launch_mma_tile<2, 2, 4, 4, 0, 0, true, false, MATH>(g, mc.compute_units, stream, err, "gemmcm");
-    if (variant == 2) return launch_mma_tile<2, 2, 8, 4, 0, 0, true, false, MATH>(g, mc.compute_units, stream, err, "gemmcm");
+    if (variant == 1) return launch_mma_tile<2, 2, 4, 4, 0, 0, false, MATH>(g, mc.compute_units, stream, err, "gemmcm");
+    if (variant == 2) return launch_mma_tile<2, 2, 8, 4, 0, 0, false, MATH>(g, mc.compute_units, stream, err, "gemmcm");
+    if (variant == 3 || variant == 5) return launch_mma_tile<2, 2, 8, 8, 0, 0, true, MATH>(g, mc.compute_units, stream, err, "gemmcm");
   }
-  if (variant == 3) return launch_mma_tile<2, 2, 8, 8, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "gemmcm");
-  if (variant == 4) return launch_mma_tile<2, 2, 4, 4, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "gemmcm");
-  // 5: 256x256 over 8 waves of 64x128 (two waves per SIMD), direct loads
-  if (variant == 5) return launch_mma_tile<4, 2, 4, 8, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "gemmcm");
+  if (variant >= 3 && variant <= 5) return launch_mma_tile<2, 2, 4, 4, 0, 0, true, MATH>(g, mc.compute_units, stream, err, "gemmcm");
   *err = "gemmcm: unknown variant " + std::to_string(variant) + " for this k and layout";
   return -1;
 }
@@ -369,7 +368,7 @@ int launch_gemm16_t(const GemmParams& p, uint32_t use_cin, uint32_t batch, uint3
 template <class T>
 struct Q8GemmProblem {
   static constexpr bool kTransA = false, kTransB = false;
-  static constexpr bool kRegisterEpilogue = false, kSliced = false;
+  static constexpr bool kSliced = false;
   uint64_t a, b;
   uint32_t m, n, k, lda, ldb, batches;
   uint64_t a_batch, b_batch;
@@ -408,11 +407,21 @@ struct Q8GemmProblem {
     if (w.vec_ok && full) f(std::integral_constant<int, T::dtype>{});
     else f(std::integral_constant<int, -1>{});
   }
-  // the stream kernel's epilogue (n a multiple of 8, C and the scales 16-byte aligned)
+  // the stream kernel's epilogue
   struct Rows {};
   struct Columns4 {
     float s[4];
   };
+  __device__ __forceinline__ bool ragged(const Whole&) const { return ((n | uint32_t(c) / 2 | uint32_t(scales) / 2) & 7u) != 0; }
+  __device__ __forceinline__ Columns4 columns4_ragged(uint32_t, uint32_t col, const Whole&) const {
+    Columns4 cs;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) cs.s[r] = load_f32<T>(scales + uint64_t(col + r < n ? col + r : n - 1) * 2);
+    return cs;
+  }
+  __device__ __forceinline__ void store_ragged(uint32_t, uint32_t row, uint32_t col, const uint32_t (&w)[4], const Whole&) const {
+    store8_ragged(c + (uint64_t(row) * n + col) * 2, col, n, w);
+  }
   __device__ __forceinline__ Rows rows(uint32_t, uint32_t, const Whole&) const { return Rows{}; }
   __device__ __forceinline__ Columns4 columns4(uint32_t, uint32_t col, const Whole&) const {
     Columns4 cs;
@@ -468,14 +477,10 @@ int launch_q8_gemm_t(const Q8Params& p, const Machine& mc, hipStream_t stream, s
   g.a = p.a, g.b = mc.scratch, g.m = p.m, g.n = p.n, g.k = p.k * 2, g.lda = uint32_t(p.a_sm) * 2, g.ldb = p.k * 2;
   g.batches = 1, g.a_batch = 0, g.b_batch = 0, g.c = p.c, g.scales = p.scales;
   const bool large = uint64_t((p.m + 255) / 256) * ((p.n + 255) / 256) * 8 >= uint64_t(mc.compute_units) * 5;  // (as for the 16-bit product)
-  if ((large || stream_pays_16bit(p.m, p.n, 1, p.k, uint32_t(mc.compute_units), true)) && g.k > BK && p.n % 8 == 0 && p.c % 16 == 0 && p.scales % 16 == 0 &&
-      mma_stream_strides_ok(g.lda, g.ldb))
+  if ((large || stream_pays_16bit(p.m, p.n, 1, p.k, uint32_t(mc.compute_units), true)) && mma_stream_strides_ok(g.lda, g.ldb))
     return launch_mma_stream<0, 0, MATH>(g, 0, mc.compute_units, stream, err, "qmm8");
-  if (large && narrow_tiles_16bit(p.m, p.n, 1, g.k, uint32_t(mc.compute_units)))
-    return launch_mma_tile<2, 2, 8, 4, 0, 0, true, false, MATH>(g, mc.compute_units, stream, err, "qmm8");
-  if (large) return launch_mma_tile<2, 2, 8, 8, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "qmm8");
-  if (staged_tiles_int8(p.m, p.n, g.k, uint32_t(mc.compute_units))) return launch_mma_tile<2, 2, 4, 4, 0, 0, true, false, MATH>(g, mc.compute_units, stream, err, "qmm8");
-  return launch_mma_tile<2, 2, 4, 4, 0, 0, true, true, MATH>(g, mc.compute_units, stream, err, "qmm8");
+  if (staged_tiles_int8(p.m, p.n, g.k, uint32_t(mc.compute_units))) return launch_mma_tile<2, 2, 4, 4, 0, 0, false, MATH>(g, mc.compute_units, stream, err, "qmm8");
+  return launch_mma_tile<2, 2, 4, 4, 0, 0, true, MATH>(g, mc.compute_units, stream, err, "qmm8");
 }
 
 }  // namespace

@@ -22,7 +22,7 @@ namespace {
 template <bool TRB>
 struct SliceProblem {
   static constexpr bool kTransA = false, kTransB = TRB;  // (TRB: the second operand stored [k, n], 16-bit values)
-  static constexpr bool kRegisterEpilogue = false, kSliced = true;
+  static constexpr bool kSliced = true;
   uint64_t a, b;
   uint32_t m, n, k, lda, ldb, batches;  // (k: bytes of one slice, a multiple of the step; batches: the slices)
   uint32_t k_all;
@@ -85,8 +85,7 @@ __global__ __launch_bounds__(256) void mma_slices_finish(Problem p, uint32_t sli
 }
 
 // Launches the 128 x 128 tile kernel of the given arithmetic over `slices` slices of K and the second launch.
-// (MF32: the 32 x 32 matrix-core tiles, which the widened and 16-bit forms are built on.)
-template <int FA, int FB, bool MF32, int MATH, class Problem>
+template <int FA, int FB, int MATH, class Problem>
 int launch_tile_slices(const Problem& p, uint32_t slices, const Machine& mc, hipStream_t stream, std::string* err, const char* name) {
   constexpr bool TRB = Problem::kTransB;  // (k-major operands run on the tile kernel's direct-load form)
   static_assert(!Problem::kTransA, "slices of K: the first operand in rows of k");
@@ -95,7 +94,11 @@ int launch_tile_slices(const Problem& p, uint32_t slices, const Machine& mc, hip
   slices = cut.slices;
   sp.a = p.a, sp.b = p.b, sp.m = p.m, sp.n = p.n, sp.k = cut.chunks_per_slice * BK, sp.k_all = p.k, sp.lda = p.lda, sp.ldb = p.ldb, sp.batches = slices;
   sp.a_batch = sp.k, sp.b_batch = TRB ? uint64_t(sp.k / 2) * p.ldb : uint64_t(sp.k), sp.partial = mc.workspace;
-  const int rc = launch_mma_tile<2, 2, 4, 4, FA, FB, MF32, TRB, MATH>(sp, mc.compute_units, stream, err, name);
+  // (16-bit operands in rows of k: loaded directly but where k ends inside a step, as without slices)
+  constexpr bool BITS16 = MATH == kMathBf16 || MATH == kMathF16;
+  int rc;
+  if (BITS16 && !TRB && p.k % BK == 0) rc = launch_mma_tile_one<2, 2, 4, 4, FA, FB, BITS16, MATH, false>(sp, mc.compute_units, stream, err, name);
+  else rc = launch_mma_tile<2, 2, 4, 4, FA, FB, TRB, MATH>(sp, mc.compute_units, stream, err, name);
   if (rc != 0) return rc;
   const uint64_t threads = uint64_t(p.m) * ((p.n + 3) / 4);
   hipLaunchKernelGGL((mma_slices_finish<Problem>), dim3(uint32_t((threads + 255) / 256)), dim3(256), 0, stream, p, slices, mc.workspace);

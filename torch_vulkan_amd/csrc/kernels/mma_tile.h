@@ -9,9 +9,6 @@
 //   columns(batch, n, whole)             per-lane constants of columns n .. n + 3
 //   store<DT>(batch, m, n, t, cols, whole)   finish and store 4 outputs of row m
 //   for_output_type(full, whole, f)      call f(integral_constant<int, DT>) for the output type
-//   kRegisterEpilogue                    the problem also offers the epilogue that stores straight from the accumulators:
-//     register_epilogue(whole)             whether this launch takes it (bfloat16 output, aligned)
-//     row_scale(m, whole), column_terms(n, whole, scale[4], bias[4])   what an output needs: acc * row_scale * scale[c] + bias[c]
 //   kTransA, kTransB                     16-bit operands only: the operand is stored k-major, i.e.
 //                                        as [k, m] (or [k, n]) rows lda (ldb) bytes apart, contiguous
 //                                        along m (n); m (n) a multiple of 8, k any number where both are
@@ -52,10 +49,6 @@ __device__ __forceinline__ V4F mfma_f8(const V8I& first, const V8I& second, cons
 }
 
 using V16F = float __attribute__((ext_vector_type(16)));
-template <int FA, int FB>
-__device__ __forceinline__ V16F mfma_f8_32(const V8I& first, const V8I& second, const V16F& acc) {
-  return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(first, second, acc, FB, FA, 0, 0, 0, 0);
-}
 
 // The exact path: float8 values widen exactly to bfloat16 (two per instruction), and the
 // bfloat16 matrix core adds its products at float32 precision (measured: within 2^-27 of
@@ -90,25 +83,39 @@ using V8H = _Float16 __attribute__((ext_vector_type(8)));
 // Half q (16 bytes) of a 32-byte fragment.
 __device__ __forceinline__ V4I half_of(const V8I& f, int q) { return V4I{f[4 * q], f[4 * q + 1], f[4 * q + 2], f[4 * q + 3]}; }
 template <int MATH>
-__device__ __forceinline__ V16F mfma_16bit(const V4I& first, const V4I& second, const V16F& acc) {
+__device__ __forceinline__ V16F mfma_16bit_32(const V4I& first, const V4I& second, const V16F& acc) {
   if constexpr (MATH == kMathBf16)
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(V8BF, first), __builtin_bit_cast(V8BF, second), acc, 0, 0, 0);
   else
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(V8H, first), __builtin_bit_cast(V8H, second), acc, 0, 0, 0);
 }
+// Two operands of 8 16-bit values per lane, 16 x 16 outputs over 32 values of k: a lane holds, of row lane % 16 of the second operand,
+// columns 4 (lane / 16) .. + 3 of the first.  (On N(0,1) operands the 16 x 16 instructions alone run at 2.06 PFLOP/s where the 32 x 32 ones reach
+// 1.78, float8 4.42 against 4.07, and both at 2.44-2.48 and 4.95 on zeros: the part holds a higher clock, having half the accumulators to read
+// and write per multiply-add.)
+template <int MATH>
+__device__ __forceinline__ V4F mfma_16bit(const V4I& first, const V4I& second, const V4F& acc) {
+  if constexpr (MATH == kMathBf16)
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(V8BF, first), __builtin_bit_cast(V8BF, second), acc, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(V8H, first), __builtin_bit_cast(V8H, second), acc, 0, 0, 0);
+}
 
-template <int WAVES_M, int WAVES_N, int TM, int TN, int FA, int FB, bool MF32, bool DIRECT, int MATH, bool TAIL, class P>
-__global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t tiles_m, uint32_t tiles_n) {
+template <int WAVES_M, int WAVES_N, int TM, int TN, int FA, int FB, bool DIRECT, int MATH, bool TAIL, class P>
+__global__ __launch_bounds__(WAVES_M* WAVES_N * 64, TM* TN <= 16 ? 2 : 1) void mma_tile(P p, uint32_t tiles_m, uint32_t tiles_n) {
   constexpr bool WIDE = MATH == kMathFp8Wide;
-  static_assert(MATH == kMathFp8 || MF32, "the widened and 16-bit forms are built on the 32x32 tiles");
+  // 32 x 32 matrix-core tiles, or 16 x 16 ones.  (16-bit operands staged through registers: 1000 x 8192 x 3000 87 us on 32 x 32, 95 on 16 x 16; the same
+  // loaded into LDS directly 85 on 16 x 16, but where k ends inside a step, rows that begin inside a 128-byte line: 1000 x 4104 x 3000 58 against 53.)
+  constexpr bool MF32 = WIDE || ((MATH == kMathBf16 || MATH == kMathF16) && !DIRECT);
   constexpr bool TRA = P::kTransA, TRB = P::kTransB;
-  static_assert(!(TRA || TRB) || (DIRECT && MF32 && (MATH == kMathBf16 || MATH == kMathF16)),
-                "k-major operands: 16-bit values, direct loads, 32x32 tiles");
+  constexpr bool BITS16 = MATH == kMathBf16 || MATH == kMathF16;
+  static_assert(!(TRA || TRB) || (DIRECT && BITS16), "k-major operands: 16-bit values, direct loads");
   constexpr int NT = WAVES_M * WAVES_N * 64;
   constexpr int BM = WAVES_M * TM * 16, BN = WAVES_N * TN * 16;
   constexpr int A_CHUNKS = BM * 8 / NT, B_CHUNKS = BN * 8 / NT;  // 16-byte chunks per thread per step
   static_assert(BM * 8 % NT == 0 && BN * 8 % NT == 0, "tile rows must divide over the threads");
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)(lds)));
   constexpr uint32_t STAGE = (BM + BN) * BK;
 
   // tile order: groups of 8 consecutive workgroups land on the 8 XCDs round-robin, so
@@ -146,7 +153,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
     // chunk that the swizzle keeps in that slot
     if constexpr (TRA) {
       // slot id of the [64 k][BM values] tile -> (k row, chunk of 8 values along m); chunks past m repeat the last one
-      const uint32_t id = tid + NT * i, row = id / (BM / 8), c = (id % (BM / 8)) ^ ((row & 3u) << 2);
+      const uint32_t id = tid + NT * i, row = id / (BM / 8), c = (id % (BM / 8)) ^ ((row & 3u) << 1 | (row & 8u));
       const uint32_t mc = m0 / 8 + c < p.m / 8 ? m0 / 8 + c : p.m / 8 - 1;
       a_src[i] = a_base + uint64_t(row) * p.lda + mc * 16;
       a_dst[i] = 0;
@@ -160,7 +167,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
 #pragma unroll
   for (int i = 0; i < B_CHUNKS; ++i) {
     if constexpr (TRB) {
-      const uint32_t id = tid + NT * i, row = id / (BN / 8), c = (id % (BN / 8)) ^ ((row & 3u) << 2);
+      const uint32_t id = tid + NT * i, row = id / (BN / 8), c = (id % (BN / 8)) ^ ((row & 3u) << 1 | (row & 8u));
       const uint32_t nc = n0 / 8 + c < p.n / 8 ? n0 / 8 + c : p.n / 8 - 1;
       b_src[i] = b_base + uint64_t(row) * p.ldb + nc * 16;
       b_dst[i] = 0;
@@ -172,9 +179,9 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
     b_dst[i] = BM * BK + tile_offset(row, c);
   }
 
-  // MF32: the wave's sub-tile as (TM/2) x (TN/2) tiles of 32x32 (V_MFMA_F32_32X32X64_F8F6F4,
-  // two per k-step along k); otherwise TM x TN tiles of 16x16 (one 16X16X128 per k-step).
-  // Both leave a lane with groups of 4 consecutive output columns of one row.
+  // The wave's sub-tile as TM x TN tiles of 16 x 16 (float8: one 16X16X128 per k-step, 16-bit: two 16X16X32), MF32 as (TM/2) x (TN/2) tiles of 32 x 32
+  // (V_MFMA_F32_32X32X16, two per half k-step, or four of widened values).  Both leave a lane with groups of 4 consecutive output columns
+  // of one row.
   constexpr int TM2 = MF32 ? TM / 2 : 1, TN2 = MF32 ? TN / 2 : 1;
   V4F acc[MF32 ? 1 : TM][MF32 ? 1 : TN];
   V16F acc32[TM2][TN2];
@@ -198,7 +205,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
   // the chunks of step s+1 from registers to LDS (first half of the step) and loads the
   // chunks of step s+2 into the same registers (second half).
   constexpr int NC = A_CHUNKS + B_CHUNKS;      // chunks per thread per step
-  constexpr int NSIDE = DIRECT ? NC : 2 * NC, NMFMA = MF32 ? TM * TN / 2 : TM * TN;  // side operations / MFMAs per step
+  constexpr int NSIDE = DIRECT ? NC : 2 * NC, NMFMA = MF32 ? TM * TN / 2 : BITS16 ? 2 * TM * TN : TM * TN;  // side operations / MFMAs per step
   V4I reg[NC];
   const V4I zero = {0, 0, 0, 0};
   const uint32_t steps = (k_bytes + BK - 1) / BK;
@@ -227,8 +234,8 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
     *reinterpret_cast<V4I*>(lds + stage * STAGE + dst) = reg[c];
   };
   auto fragment = [&](const uint8_t* tile, uint32_t row) {
-    const V4I lo = *reinterpret_cast<const V4I*>(tile + tile_offset(row, 2 * g));
-    const V4I hi = *reinterpret_cast<const V4I*>(tile + tile_offset(row, 2 * g + 1));
+    const V4I lo = *reinterpret_cast<const V4I*>(tile + tile_offset(row, g));  // (k in an order of its own, the same for both operands: mma_stream.h's)
+    const V4I hi = *reinterpret_cast<const V4I*>(tile + tile_offset(row, 4 + g));
     return V8I{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
   };
   // Side operation `op` of step s: [0,NC) write the chunks of step s+1 to LDS, [NC,2NC) load
@@ -246,7 +253,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
   auto direct_chunk = [&](int c, uint32_t step, auto partial) {
     uint64_t src = c < A_CHUNKS ? a_src[c < A_CHUNKS ? c : 0] : b_src[c < A_CHUNKS ? 0 : c - A_CHUNKS];
     const uint32_t tile_base = c < A_CHUNKS ? uint32_t(c) * NT * 16 : BM * BK + uint32_t(c - A_CHUNKS) * NT * 16;
-    uint8_t* dst = lds + (step & 1u) * STAGE + tile_base + uint32_t(wave) * 1024;
+    const uint32_t dst = lds0 + (step & 1u) * STAGE + tile_base + __builtin_amdgcn_readfirstlane(uint32_t(wave)) * 1024;
     // a step is 128 bytes along a k-contiguous row, or 64 rows of a k-major operand
     const uint64_t advance = c < A_CHUNKS ? (TRA ? uint64_t(BK / 2) * p.lda : uint64_t(BK)) : (TRB ? uint64_t(BK / 2) * p.ldb : uint64_t(BK));
     src += uint64_t(step) * advance;
@@ -256,8 +263,9 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
       const uint32_t at = (first ? TRA : TRB) ? id / ((first ? BM : BN) / 8) * 2 : ((id & 7u) ^ ((row >> 1) & 7u)) * 16;  // (k-major: rows of k of 2 bytes each)
       if (step * BK + at >= k_bytes) src = reinterpret_cast<uint64_t>(&kZeroChunk[0]);
     }
-    __builtin_amdgcn_global_load_lds(reinterpret_cast<const VKT_GLOBAL void*>(src),
-                                     (__attribute__((address_space(3))) void*)(dst), 16, 0, 0);
+    // (inline assembly, which the compiler does not know for a load into LDS: with its own form it waits for all of them before every
+    // later fragment read)
+    load_to_lds_at<0>(src, dst);
   };
   auto side = [&](int op, uint32_t s, auto steady) {
     constexpr bool kSteady = decltype(steady)::value;
@@ -290,32 +298,8 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
       // second half of k are asked for once the first MFMAs are under way
       // (row fragments are asked for two groups of MFMAs ahead: one group, 256 cycles, is
       // less than an LDS read takes while the direct loads are writing into the same LDS)
-      // The same fragment out of a k-major tile [64 k][W values]: for each half q of the fragment the 8
-      // values k = 32 kk + 16 h + 8 q .. + 7 of column `col`, by two transposing reads of 4 k each.  Lane i
-      // of a group of 16 points at row k + i / 4, values 4 (i % 4) .. + 3 of the group's 16 columns.
-      auto frag32_t = [&](const uint8_t* tile, uint32_t width, uint32_t col0, int kk) {
-        using V4S = short __attribute__((ext_vector_type(4)));
-        V8I f;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const uint32_t k = 32 * kk + 16 * h + 4 * t + (l16 >> 2);
-          const uint32_t value = col0 + 16 * ((lane >> 4) & 1) + 4 * (l16 & 3);  // first of the 4 values this lane points at
-          const uint32_t chunk = (value >> 3) ^ ((k & 3u) << 2);
-          const V4S v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (__attribute__((address_space(3))) V4S*)(tile + k * width * 2 + chunk * 16 + (value & 7u) * 2));
-          const U2 w = __builtin_bit_cast(U2, v);
-          f[2 * t] = int(w.x), f[2 * t + 1] = int(w.y);
-        }
-        return f;
-      };
-      auto row_frag = [&](int gi) {
-        if constexpr (TRA) return frag32_t(ta, BM, (wm * TM2 + gi % TM2) * 32, gi / TM2);
-        else return frag32(ta, (wm * TM2 + gi % TM2) * 32 + l32, gi / TM2);
-      };
-      auto col_frag = [&](int j, int kk) {
-        if constexpr (TRB) return frag32_t(tb, BN, (wn * TN2 + j) * 32, kk);
-        else return frag32(tb, (wn * TN2 + j) * 32 + l32, kk);
-      };
+      auto row_frag = [&](int gi) { return frag32(ta, (wm * TM2 + gi % TM2) * 32 + l32, gi / TM2); };
+      auto col_frag = [&](int j, int kk) { return frag32(tb, (wn * TN2 + j) * 32 + l32, kk); };
       // With two waves per SIMD (8 waves) the column fragments of the second half of k take the registers of the
       // first half's, each right after its last use (256 registers per wave do not hold both halves next to the
       // accumulators), and row fragments are asked for one group ahead: the other wave covers the LDS latency.
@@ -358,18 +342,77 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
 #pragma unroll
             for (int q = 0; q < 4; ++q)
               acc32[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(widen_slice<FB>(bf[kLean ? 0 : kk][j], q), af_wide[q], acc32[i][j], 0, 0, 0);
-          } else if constexpr (MATH == kMathBf16 || MATH == kMathF16) {
-            // 16-bit elements: a fragment's 32 bytes are two operands of 8 values
+          } else {  // 16-bit elements: a fragment's 32 bytes are two operands of 8 values
 #pragma unroll
-            for (int q = 0; q < 2; ++q) acc32[i][j] = mfma_16bit<MATH>(half_of(bf[kLean ? 0 : kk][j], q), half_of(af, q), acc32[i][j]);
-          } else {
-            acc32[i][j] = mfma_f8_32<FA, FB>(bf[kLean ? 0 : kk][j], af, acc32[i][j]);
+            for (int q = 0; q < 2; ++q) acc32[i][j] = mfma_16bit_32<MATH>(half_of(bf[kLean ? 0 : kk][j], q), half_of(af, q), acc32[i][j]);
           }
           if (kLean && gi == TM2 - 1) bf[0][j] = col_frag(j, 1);
         }
         __builtin_amdgcn_sched_barrier(0);
         af = next;
         next = next2;
+      }
+    } else if constexpr (BITS16) {
+      // A fragment is 16 rows x 32 values of k: row lane % 16, the 8 values of chunk 4 kk + lane / 16.  Half a step (kk) at a time: row
+      // block after row block against all column blocks.
+      auto fragment16 = [&](const uint8_t* tile, uint32_t row0, int kk) { return *reinterpret_cast<const V4I*>(tile + tile_offset(row0 + l16, 4 * kk + g)); };
+      // The same values out of a k-major tile [64 k][width values], by two transposing reads of 4 k each.  Lane i of a group of 16
+      // points at row k + i / 4, values 4 (i % 4) .. + 3 of the block's 16.  (The swizzle puts the eight rows that 32 lanes of a read touch, k % 4
+      // and k / 8 % 2, on different 32 bytes of the banks' 256.)
+      const uint32_t at_k = (l16 >> 2 | (g & 1) << 2) << 5 ^ ((l16 >> 1 & 1) << 4 | (l16 & 1) << 3);  // (the row's key on the pair of chunks that holds a block)
+      auto fragment16_k = [&](const uint8_t* tile, uint32_t width, uint32_t block, int kk) {
+        using V4S = short __attribute__((ext_vector_type(4)));
+        const uint32_t at = (8 * g + (l16 >> 2)) * (width * 2) + (at_k ^ block << 5);
+        V4I f;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const V4S v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) V4S*)(tile + at + (32 * kk + 4 * t) * (width * 2)));
+          const U2 w = __builtin_bit_cast(U2, v);
+          f[2 * t] = int(w.x), f[2 * t + 1] = int(w.y);
+        }
+        return f;
+      };
+      auto row_frag = [&](int gi) {
+        if constexpr (TRA) return fragment16_k(ta, BM, wm * TM + gi % TM, gi / TM);
+        else return fragment16(ta, (wm * TM + gi % TM) * 16, gi / TM);
+      };
+      auto col_frag = [&](int j, int kk) {
+        if constexpr (TRB) return fragment16_k(tb, BN, wn * TN + j, kk);
+        else return fragment16(tb, (wn * TN + j) * 16, kk);
+      };
+      // (column fragments: as above; row fragments are asked for AHEAD groups of matrix-core instructions ahead)
+      constexpr bool kLean = WAVES_M * WAVES_N > 4;
+      constexpr int AHEAD = 4;
+      V4I af[AHEAD], bf[kLean ? 1 : 2][TN];
+      af[0] = row_frag(0);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) bf[0][j] = col_frag(j, 0);
+#pragma unroll
+      for (int i = 1; i < AHEAD; ++i) af[i] = row_frag(i);
+#pragma unroll
+      for (int gi = 0; gi < 2 * TM; ++gi) {
+        const int kk = gi / TM, i = gi % TM;
+        if (gi == 0 && !kLean) {
+#pragma unroll
+          for (int j = 0; j < TN; ++j) bf[kLean ? 0 : 1][j] = col_frag(j, 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const int n = gi * TN + j;
+          // (DIRECT: all at the step's start, as above, one per two instructions)
+          const int lo_op = DIRECT ? ((n + 1) / 2 < NSIDE ? (n + 1) / 2 : NSIDE) : n * NSIDE / NMFMA;
+          const int hi_op = DIRECT ? ((n + 2) / 2 < NSIDE ? (n + 2) / 2 : NSIDE) : (n + 1) * NSIDE / NMFMA;
+#pragma unroll
+          for (int op = lo_op; op < hi_op; ++op) {
+            side(op, s, steady);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          acc[i][j] = mfma_16bit<MATH>(bf[kLean ? 0 : kk][j], af[gi % AHEAD], acc[i][j]);
+          if (kLean && gi == TM - 1) bf[0][j] = col_frag(j, 1);
+        }
+        if (gi + AHEAD < 2 * TM) af[gi % AHEAD] = row_frag(gi + AHEAD);
+        __builtin_amdgcn_sched_barrier(0);
       }
     } else {
       V8I bf[TN];
@@ -384,7 +427,8 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
           const int n = i * TN + j;
-          const int lo_op = n * NSIDE / NMFMA, hi_op = (n + 1) * NSIDE / NMFMA;
+          const int lo_op = DIRECT ? (n < NSIDE ? n : NSIDE) : n * NSIDE / NMFMA;  // (DIRECT: all at the step's start)
+          const int hi_op = DIRECT ? (n + 1 < NSIDE ? n + 1 : NSIDE) : (n + 1) * NSIDE / NMFMA;
 #pragma unroll
           for (int op = lo_op; op < hi_op; ++op) {
             side(op, s, steady);
@@ -428,49 +472,6 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
 
   const auto whole = p.whole();  // what the epilogue needs once per launch
   const uint32_t wm0 = m0 + wm * TM * 16, wn0 = n0 + wn * TN * 16;
-  // Epilogue from the registers (bfloat16 outputs of whole tiles): no LDS, no barrier, so nothing holds a wave back
-  // once its last matrix-core instruction has gone, and the next tile's first loads may land in LDS meanwhile.  A 32 x 32
-  // matrix-core tile leaves lane l with row l % 32 and, for q = 0..3, columns 8 q + 4 (l / 32) .. + 3: two lanes 32
-  // apart hold the two halves of 8 consecutive outputs.  v_permlane32_swap puts them together (lanes below 32 take
-  // chunk q = 0 or 2 of their row, lanes from 32 chunk 1 or 3), and every lane stores 16 bytes; a store instruction
-  // of a wave writes 32 rows x 32 consecutive bytes.
-  bool from_registers = false;
-  if constexpr (MF32 && P::kRegisterEpilogue) {
-    from_registers = p.register_epilogue(whole) && n0 + BN <= p.n;  // (the same for every wave of the workgroup)
-    if (from_registers) {
-      const uint32_t l32 = lane & 31, h = lane >> 5;
-#pragma unroll
-      for (int j = 0; j < TN2; ++j) {
-        float scale[4][4], bias[4][4];  // of this lane's columns wn0 + 32 j + 8 q + 4 h + r
-#pragma unroll
-        for (int q = 0; q < 4; ++q) p.column_terms(wn0 + 32 * j + 8 * q + 4 * h, whole, scale[q], bias[q]);
-#pragma unroll
-        for (int i = 0; i < TM2; ++i) {
-          const uint32_t m = wm0 + 32 * i + l32;
-          const float rs = p.row_scale(m < p.m ? m : p.m - 1, whole);
-          const V16F& t = acc32[i][j];
-#pragma unroll
-          for (int qp = 0; qp < 2; ++qp) {
-            uint32_t lo[2], hi[2];  // chunks 2 qp and 2 qp + 1 as two bfloat16 pairs each
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-              const int q0 = 2 * qp, q1 = 2 * qp + 1;
-              lo[e] = pack_bf16(t[4 * q0 + 2 * e] * (rs * scale[q0][2 * e]) + bias[q0][2 * e],
-                                t[4 * q0 + 2 * e + 1] * (rs * scale[q0][2 * e + 1]) + bias[q0][2 * e + 1]);
-              hi[e] = pack_bf16(t[4 * q1 + 2 * e] * (rs * scale[q1][2 * e]) + bias[q1][2 * e],
-                                t[4 * q1 + 2 * e + 1] * (rs * scale[q1][2 * e + 1]) + bias[q1][2 * e + 1]);
-            }
-            // lanes 32.. of `lo` change places with lanes ..31 of `hi`
-            const auto s0 = __builtin_amdgcn_permlane32_swap(lo[0], hi[0], false, false);
-            const auto s1 = __builtin_amdgcn_permlane32_swap(lo[1], hi[1], false, false);
-            const uint32_t n = wn0 + 32 * j + 8 * (2 * qp + h);
-            if (m < p.m) p.store_bf16x8(batch, m, n, U4{s0[0], s1[0], s0[1], s1[1]});
-          }
-        }
-      }
-    }
-  }
-  if (!from_registers) {
   // Epilogue through LDS.  A lane holds out[m = .. + l16][n = .. + 4 g + r], r = 0..3, for each of its
   // TM x TN tiles.  Each wave transposes its sub-tile through its own slice of LDS (the
   // operand buffers are dead by now), 64 columns at a time, so that the scale / bias / cast
@@ -531,20 +532,19 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void mma_tile(P p, uint32_t 
     p.for_output_type(n + 3 < p.n, whole, rows);
   }
   __syncthreads();  // the next tile's operands overwrite the LDS the epilogue has just read
-  }  // (epilogue through LDS)
   }  // (tile loop)
 }
 
 
 // Launches the tile kernel for problem p (persistent grid: as many workgroups as are resident
 // at once, in multiples of 8, one per XCD).
-template <int WAVES_M, int WAVES_N, int TM, int TN, int FA, int FB, bool MF32, bool DIRECT, int MATH, bool TAIL, class P>
+template <int WAVES_M, int WAVES_N, int TM, int TN, int FA, int FB, bool DIRECT, int MATH, bool TAIL, class P>
 int launch_mma_tile_one(const P& p, int compute_units, hipStream_t stream, std::string* err, const char* who) {
   constexpr int BM = WAVES_M * TM * 16, BN = WAVES_N * TN * 16;
   constexpr uint32_t operand_bytes = 2 * (BM + BN) * BK, epilogue_bytes = WAVES_M * WAVES_N * TM * 16 * 256;
   constexpr uint32_t lds_bytes = operand_bytes > epilogue_bytes ? operand_bytes : epilogue_bytes;
   static_assert(TN % 4 == 0, "the epilogue moves 64 columns (4 tiles) per pass");
-  auto kernel = mma_tile<WAVES_M, WAVES_N, TM, TN, FA, FB, MF32, DIRECT, MATH, TAIL, P>;
+  auto kernel = mma_tile<WAVES_M, WAVES_N, TM, TN, FA, FB, DIRECT, MATH, TAIL, P>;
   static bool configured = false;  // guarded by the runtime's stream mutex
   if (!configured) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -568,14 +568,14 @@ int launch_mma_tile_one(const P& p, int compute_units, hipStream_t stream, std::
   return 0;
 }
 
-template <int WAVES_M, int WAVES_N, int TM, int TN, int FA, int FB, bool MF32, bool DIRECT, int MATH, class P>
+template <int WAVES_M, int WAVES_N, int TM, int TN, int FA, int FB, bool DIRECT, int MATH, class P>
 int launch_mma_tile(const P& p, int compute_units, hipStream_t stream, std::string* err, const char* who) {
   if constexpr (DIRECT) {  // (the register-staged forms handle any k)
     uint32_t k = p.k;
     if constexpr (P::kSliced) k = p.k_all;
-    if (k % BK != 0) return launch_mma_tile_one<WAVES_M, WAVES_N, TM, TN, FA, FB, MF32, DIRECT, MATH, true>(p, compute_units, stream, err, who);
+    if (k % BK != 0) return launch_mma_tile_one<WAVES_M, WAVES_N, TM, TN, FA, FB, DIRECT, MATH, true>(p, compute_units, stream, err, who);
   }
-  return launch_mma_tile_one<WAVES_M, WAVES_N, TM, TN, FA, FB, MF32, DIRECT, MATH, false>(p, compute_units, stream, err, who);
+  return launch_mma_tile_one<WAVES_M, WAVES_N, TM, TN, FA, FB, DIRECT, MATH, false>(p, compute_units, stream, err, who);
 }
 
 }  // namespace

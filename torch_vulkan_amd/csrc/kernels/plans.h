@@ -86,10 +86,11 @@ struct StreamTiles {
   uint32_t columns;
   uint64_t cost;
 };
-constexpr StreamTiles mma_stream_tiles(uint32_t m, uint32_t n, uint64_t batches, uint32_t cus) {
+constexpr StreamTiles mma_stream_tiles(uint32_t m, uint32_t n, uint64_t batches, uint32_t cus, bool k_major_b = false) {
   const uint32_t columns[3] = {256, 192, 128}, cost[3] = {100, 81, 64};
   StreamTiles best = {0, 0};
   for (int i = 0; i < 3; ++i) {
+    if (k_major_b && columns[i] == 192) continue;  // (not built)
     const uint64_t tiles = (uint64_t(m) + 255) / 256 * ((uint64_t(n) + columns[i] - 1) / columns[i]) * batches;
     const uint64_t c = (tiles + cus - 1) / cus * cost[i];
     if (best.columns == 0 || c < best.cost) best = StreamTiles{columns[i], c};
