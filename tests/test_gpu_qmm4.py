@@ -146,6 +146,23 @@ def test_q4_phase_2_is_phase_0_then_1(m, k, n, bs, flags):
     assert np.array_equal(_dev.q4_compact(bits(x), oracle.F32, cm, flags=flags | 256), one)
 
 
+@pytest.mark.parametrize("m", [127, 128, 129, 272])  # (from 128 rows on a row tile's rows are quantised on one die)
+@pytest.mark.parametrize("k,bs", [(128, 32), (160, 32), (2112, 64), (2176, 128), (2304, 256), (2080, 2080), (100, 100)])
+def test_q4_rows_and_quads_that_exist(m, k, bs):
+    """Row counts around whole row tiles of 8 dies, and k whose last units are far from the padded end of the layout: the oracle's bits."""
+    import _dev
+    n = 40
+    w, sc, bvec = int4_weights(n, k, bs, bias=True)
+    x = int4_rows(m, k, torch.float32)
+    packed = torch._dyn_quant_pack_4bit_weight(w, sc, bvec, bs, k, n).numpy()
+    want = oracle.q4_matmul(bits(x), oracle.F32, packed, bs, k, n)
+    cm = _dev.CompactWeights(packed, bs, k, n, layout=1)
+    for flags in (16, 32 | 64, 32 | 128, 32 | 192):
+        for fused in (True, False):
+            got = _dev.q4_compact(bits(x), oracle.F32, cm, fused=fused, flags=flags)
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (flags, fused)
+
+
 def test_q4_float16_products_on_the_fixed_workspace():
     """vkt_dispatch_static: three pieces of rows where the pool's workspace takes two."""
     import _dev

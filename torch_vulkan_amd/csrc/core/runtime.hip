@@ -59,7 +59,9 @@ struct HipSource {
 constexpr uint64_t kStaticScratchBytes = VKT_STATIC_SCRATCH_BYTES;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
-constexpr uint64_t kWorkspaceBytes = 32ull << 20;
+// (what asks for the most of it: the float16 rows of a 4-bit product, 2 bytes a value.  In 32 MiB 2048 x 11008 values went in two pieces, whose
+// launches leave half the machine idle against 4096 columns: 374 us, 337 in one.)
+constexpr uint64_t kWorkspaceBytes = 128ull << 20;
 // The widened-weights region of many-row int8 products is capped: larger weights run on the row-block kernels.
 constexpr uint64_t kMaxWidenedBytes = 2ull << 30;
 

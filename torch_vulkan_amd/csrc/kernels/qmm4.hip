@@ -606,6 +606,7 @@ __global__ __launch_bounds__(256 * TEAMS) void qmm4c_stream(Q4CParams p, Compact
 
 struct MatrixLayout {
   uint32_t nunits, quads, tiles, upb;  // quads: groups of 4 units, padded to a multiple of 16
+  uint32_t walked;  // the quads that hold a unit, in pairs: what the kernels walk whose waves each take all of K (11008 values of k: 86 of 96; 2048 x 11008 x 4096 337 -> 309 us)
   uint64_t nib_bytes, scale_off, scale_bytes, bias_off, total;
 };
 
@@ -616,6 +617,7 @@ __host__ __device__ inline bool matrix_layout(uint32_t n, uint32_t k, uint32_t b
   if (!channelwise && k % bs != 0) return false;
   L->nunits = (k + kUnit - 1) / kUnit;
   L->quads = (L->nunits + 63) / 64 * 16;
+  L->walked = ((L->nunits + 3) / 4 + 1) & ~1u;
   L->tiles = (n + kTileCols - 1) / kTileCols;
   L->upb = channelwise ? 0 : bs / kUnit;
   // [quad][tile][lane 64] x 16 bytes: word j of a lane = 8 nibbles of unit 4 quad + j.  Quad-major:
@@ -705,8 +707,8 @@ __device__ __forceinline__ uint64_t operand_offset(uint32_t m, uint32_t g, uint3
 
 // The same 8 values less the zero point as float16, which holds -255 .. 255 exactly, for qmm4m_half: the pairs (0, 4), (1, 5),
 // (2, 6), (3, 7), in which a word of nibbles comes apart.  [row tile][unit][lane = kg * 16 + m % 16] x 16 bytes, the
-// order of qmm4m_half's lanes.  (A row's workgroup writes 16 bytes of a line; with 128 bytes of a row side by side it takes
-// 10.7 instead of 18.1 us for 2048 x 4096 values, but the product that reads them 451 instead of 331.)
+// order of qmm4m_half's lanes.  (A row's workgroup writes 16 bytes of a line (quant_row); with 128 bytes of a row side by side the product
+// that reads them takes 451 us instead of 331.)
 using V2H = _Float16 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ U4 operand_halves(const int (&a)[8]) {
   U4 r;
@@ -718,13 +720,23 @@ __device__ __forceinline__ uint64_t halves_offset(uint32_t m, uint32_t g, uint32
   return ((uint64_t(m >> 4) * (quads * 4) + (g >> 2)) * 64 + (g & 3) * 16 + (m & 15)) * 16;
 }
 
+// Which of `rows` rows a workgroup of qmm4m_rowquant takes.  The 16 rows of a row tile write 8 or 16 bytes of a line each; workgroup i
+// runs on XCD i % 8, and in that order eight L2s write parts of every line (2048 x 4096 float32 rows 18-22 us).  From 128 rows on a
+// tile's rows go to one XCD, whose L2 puts the lines together: 12.8 us.
+constexpr uint32_t kSpreadRows = 128;
+__host__ __device__ inline uint32_t quant_row(uint32_t i, uint32_t rows) {
+  return rows < kSpreadRows ? i : ((i >> 7) * 8 + (i & 7)) * 16 + (i >> 3 & 15);
+}
+inline dim3 quant_grid(uint32_t rows) { return dim3(rows < kSpreadRows ? rows : (rows + 127) / 128 * 128); }
+
 // Phase 0 for the matrix layout, one workgroup per row, from row m0 on.  FAST: k is a multiple of 8, at most
 // 2048 * kFusedGroups, rows 16-byte aligned: the row is read once, into registers.  HALVES: the values go to `dst` as
 // qmm4m_half's operand, row m0 first, and to p.q only where `keep` says that the caller reads them there.
 template <class T, bool FAST, bool HALVES>
-__global__ __launch_bounds__(256) void qmm4m_rowquant(Q4CParams p, uint32_t groupwise, uint32_t quads, uint64_t dst, uint32_t m0, uint32_t keep) {
+__global__ __launch_bounds__(256) void qmm4m_rowquant(Q4CParams p, uint32_t groupwise, uint32_t quads, uint64_t dst, uint32_t m0, uint32_t rows, uint32_t keep) {
   constexpr uint64_t item = sizeof(typename T::storage);
-  const uint32_t m = m0 + blockIdx.x, tid = threadIdx.x;
+  const uint32_t in = quant_row(blockIdx.x, rows), m = m0 + in, tid = threadIdx.x;
+  if (in >= rows) return;
   const uint64_t row = p.inp + uint64_t(m) * p.k * item;
   const uint32_t groups_all = quads * 16;
   RowQuant rq;
@@ -740,7 +752,7 @@ __global__ __launch_bounds__(256) void qmm4m_rowquant(Q4CParams p, uint32_t grou
       if (keep) stg<U2>(p.q + operand_offset(m, g, quads), operand_bytes(q));
 #pragma unroll
       for (int e = 0; e < 8; ++e) q[e] -= rq.izp;
-      stg<U4>(dst + halves_offset(blockIdx.x, g, quads), operand_halves(q));
+      stg<U4>(dst + halves_offset(in, g, quads), operand_halves(q));
     } else {
       stg<U2>(p.q + operand_offset(m, g, quads), operand_bytes(q));
     }
@@ -1019,7 +1031,7 @@ __global__ __launch_bounds__(256) void qmm4m_rows(Q4CParams p, MatrixLayout L, u
   };
   Set sets[kRowsAhead];
   auto request = [&](Set& set, uint32_t quad) {
-    quad = quad < L.quads ? quad : L.quads - 1;
+    quad = quad < L.walked ? quad : L.walked - 1;
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
       set.q0[t] = ldg<U4>(qbase[t] + uint64_t(quad) * 2048);
@@ -1035,6 +1047,8 @@ __global__ __launch_bounds__(256) void qmm4m_rows(Q4CParams p, MatrixLayout L, u
   // across the requests.  Left to itself the scheduler puts these loops' loads next to their use (the chains are short, and it aims at one
   // more wave per SIMD), five waits for memory per two quads.  us, before the shared sums / with them / with them and in place: 512 x
   // 4096 x 11008 129 / 143 / 103, 512 x 8192 x 11008 246 / 269 / 200, 96 x 4096 x 28672 60 / 64 / 49, 2048 x 4096 x 11008 489 / 451 / 379.
+  // (Blocks of 128, with the shared sums / and in place: 2048 x 4096 x 11008 411 / 386, but 300 x 4096 x 11008 77 / 83, 150 rows 42.5 / 45; one scale per
+  // column 330 / 350, 1024 x 8192 x 8192 188 / 218.)
   constexpr bool kInPlace = UPB == 8 && RT * CT > 1;
 #pragma unroll
   for (int i = 0; i < kRowsAhead; ++i) {
@@ -1056,8 +1070,8 @@ __global__ __launch_bounds__(256) void qmm4m_rows(Q4CParams p, MatrixLayout L, u
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[t][c][r] = -0.0f;
     }
-  // (quads is a multiple of 16, so of kRowsAhead, and blocks of up to 8 units start at even quads)
-  for (uint32_t quad0 = 0; quad0 < L.quads; quad0 += kRowsAhead) {
+  // (a multiple of kRowsAhead, and blocks of up to 8 units start at even quads)
+  for (uint32_t quad0 = 0; quad0 < L.walked; quad0 += kRowsAhead) {
 #pragma unroll
     for (int i = 0; i < kRowsAhead; ++i) {
       Set taken;
@@ -1162,7 +1176,7 @@ __global__ __launch_bounds__(256) void qmm4m_rows(Q4CParams p, MatrixLayout L, u
         const uint32_t m = row0 + 16 * t + kg * 4 + r;
         if (m >= p.m) continue;
         float v = acc[t][c][r];
-        if constexpr (UPB == 0) v = float(d[t][c][r] + row_sum[t][r] + nzp_r[t][r] * (col_sum[c][r] - 256 * int(L.quads * 4))) * s;
+        if constexpr (UPB == 0) v = float(d[t][c][r] + row_sum[t][r] + nzp_r[t][r] * (col_sum[c][r] - 256 * int(L.walked * 4))) * s;
         finish_store<T>(p.out + (uint64_t(m) * p.n + n) * item, v, bits_f32(ldg<uint32_t>(p.rows + 8ull * m)), p.has_bias != 0, bias);
       }
   }
@@ -1247,7 +1261,7 @@ __global__ __launch_bounds__(256, 2) void qmm4m_half(Q4CParams p, MatrixLayout L
     F4 s[CT];
   };
   auto request = [&](Set& set, uint32_t quad) {
-    quad = quad < L.quads ? quad : L.quads - 1;
+    quad = quad < L.walked ? quad : L.walked - 1;
 #pragma unroll
     for (int c = 0; c < CT; ++c) {
       set.w[c] = ldg_at<U4>(wbase[c] + quad * wstep, lane_at);
@@ -1316,7 +1330,7 @@ __global__ __launch_bounds__(256, 2) void qmm4m_half(Q4CParams p, MatrixLayout L
   };
   Set even, odd;
   request(even, 0);
-  for (uint32_t quad = 0; quad < L.quads; quad += 2) {  // (quads is a multiple of 16)
+  for (uint32_t quad = 0; quad < L.walked; quad += 2) {
     request(odd, quad + 1);
     process(even);
     request(even, quad + 2);  // (past the end the last quad again, so that the loop is straight-line code)
@@ -1593,8 +1607,8 @@ int launch_matrix(const Q4CParams& p, uint32_t phase_and_flags, uint32_t groupwi
       const uint64_t at = mc.workspace;
       const uint32_t threads = (rows + 15) / 16 * 16 * M.quads * 16;  // (below the workspace's bytes / 16)
       if (phase == 1) hipLaunchKernelGGL(qmm4m_expand, dim3(threads / 256), dim3(256), 0, stream, p, at, m0, rows, M.quads);
-      else if (fast) hipLaunchKernelGGL((qmm4m_rowquant<T, true, true>), dim3(rows), dim3(256), 0, stream, p, groupwise, M.quads, at, m0, keep);
-      else hipLaunchKernelGGL((qmm4m_rowquant<T, false, true>), dim3(rows), dim3(256), 0, stream, p, groupwise, M.quads, at, m0, keep);
+      else if (fast) hipLaunchKernelGGL((qmm4m_rowquant<T, true, true>), quant_grid(rows), dim3(256), 0, stream, p, groupwise, M.quads, at, m0, rows, keep);
+      else hipLaunchKernelGGL((qmm4m_rowquant<T, false, true>), quant_grid(rows), dim3(256), 0, stream, p, groupwise, M.quads, at, m0, rows, keep);
       if (M.upb == 1 && eight) launch_half<T, 1, 2, 4>(p, M, at, m0, rows, stream);
       else if (M.upb == 1) launch_half<T, 1, 2, 2>(p, M, at, m0, rows, stream);
       else if (eight) launch_half<T, 2, 2, 4>(p, M, at, m0, rows, stream);
@@ -1603,8 +1617,8 @@ int launch_matrix(const Q4CParams& p, uint32_t phase_and_flags, uint32_t groupwi
     return 0;
   }
   if (phase == 0 || phase == 2) {
-    if (fast) hipLaunchKernelGGL((qmm4m_rowquant<T, true, false>), dim3(p.m), dim3(256), 0, stream, p, groupwise, M.quads, 0ull, 0u, 1u);
-    else hipLaunchKernelGGL((qmm4m_rowquant<T, false, false>), dim3(p.m), dim3(256), 0, stream, p, groupwise, M.quads, 0ull, 0u, 1u);
+    if (fast) hipLaunchKernelGGL((qmm4m_rowquant<T, true, false>), quant_grid(p.m), dim3(256), 0, stream, p, groupwise, M.quads, 0ull, 0u, p.m, 1u);
+    else hipLaunchKernelGGL((qmm4m_rowquant<T, false, false>), quant_grid(p.m), dim3(256), 0, stream, p, groupwise, M.quads, 0ull, 0u, p.m, 1u);
   }
   if (phase == 1 || phase == 2) {
     for (uint32_t m0 = 0; rows_kernel && m0 < p.m; m0 += 16 * 1024) {
