@@ -77,3 +77,25 @@ def test_qmm4_planner(m, k, n, bs, bias):
         for layout in (0, 1):
             cw = _dev.CompactWeights(packed, bs, k, n, layout=layout)
             assert np.array_equal(_dev.q4_compact(bits(x), ODT[dtype], cw, fused=True), want), (layout, dtype)
+
+
+@pytest.mark.parametrize("rest", [1, 16])
+@pytest.mark.parametrize("kind,whole,k,n", [("int8", 2048, 1024, 8192), ("bf16", 2048, 1024, 8192), ("fp8", 2048, 2048, 8192)])
+def test_rows_past_the_last_tile_apart(kind, whole, k, n, rest):
+    """A few rows past whole tiles of 256 as a product of their own: the bits of the two products, and the rows' own scales."""
+    import _dev
+    m = whole + rest
+    if kind == "fp8":
+        a, w = torch.randn(m, k, generator=gen(1)).to(torch.float8_e4m3fn), torch.randn(n, k, generator=gen(2)).to(torch.float8_e4m3fn)
+        sa, sb = (torch.rand(m, 1, generator=gen(3)) + 0.5).numpy(), (torch.rand(1, n, generator=gen(4)) + 0.5).numpy()
+        run = lambda r: _dev.scaled_mm(bits(a[r]), oracle.E4M3, bits(w), oracle.E4M3, sa[r], sb, True, out_dtype=oracle.BF16)  # noqa: E731
+    elif kind == "bf16":
+        a, w = torch.randn(m, k, generator=gen(1)).bfloat16(), (torch.randn(n, k, generator=gen(2)) * 0.1).bfloat16()
+        cin = bits(torch.randn(m, n, generator=gen(5)).bfloat16())
+        run = lambda r: _dev.gemm16(bits(a[r]), bits(w).T, oracle.BF16, cin=cin[r], beta=0.5)  # noqa: E731
+    else:
+        a, w = torch.randn(m, k, generator=gen(1)).bfloat16(), torch.randint(-128, 128, (n, k), dtype=torch.int8, generator=gen(2)).numpy()
+        s = bits((torch.rand(n, generator=gen(3)) * 0.01).bfloat16())
+        run = lambda r: _dev.qmm8(bits(a[r]), oracle.BF16, w, s)  # noqa: E731
+    got = run(slice(0, m))
+    assert np.array_equal(got[:whole], run(slice(0, whole))) and np.array_equal(got[whole:], run(slice(whole, m)))

@@ -308,15 +308,29 @@ int launch_tiles(const GemmParams& p, uint32_t use_cin, uint32_t batch, uint32_t
   // (k-major operands: 4 in the place of 3 and 5; no 1 and 2)
   uint32_t small = TRA || TRB ? 4 : 3;  // what the stream kernel's products run on where it does not serve
   if (variant == 0) {
-    // 256 x 256 tiles where they give every compute unit one, else 128 x 128
-    // (from five eighths of a tile per unit on: 1024 x 4096 x 14336 is 224 tiles on 256 units, 121 us on the stream
-    //  kernel against 163 on 128 x 128 tiles; 168 tiles: 142 against 152; at 128 tiles the small tiles are level or ahead)
-    const bool large = uint64_t((p.m + 255) / 256) * ((p.n + 255) / 256) * batch * 8 >= uint64_t(mc.compute_units) * 5;
-    // the stream kernel, with the columns per tile that suit the shape (both operands contiguous along k, x @ w.T: also below that line)
-    const bool more = !TRA && !TRB && stream_pays_16bit(p.m, p.n, batch, p.k, uint32_t(mc.compute_units), false);
+    // the stream kernel where it pays, with the columns per tile that suit the shape, else 128 x 128 tiles
+    // (k-major operands, 128 x 128 tiles / stream: x @ w 1024 x 4096 x 8192 67 / 61, 1536 x 13824 x 5120 201 / 182, 1537 rows 351 / 286; x.t() @ y 1024 x
+    //  4096 x 8192 74 / 64, 1536 x 13824 x 5120 217 / 186; not where more than half of the tiles' rows would be padding, as in batches of few rows)
+    const uint32_t cus = uint32_t(mc.compute_units);
+    const bool large = uint64_t((p.m + 255) / 256) * ((p.n + 255) / 256) * batch * 8 >= uint64_t(cus) * 5;
+    const bool padded = (TRA || TRB) && uint64_t((p.m + 255) / 256) * 512 > uint64_t(p.m) * 3;
+    const bool streams = large || (!padded && stream_16bit(p.m, p.n, batch, p.k, cus, false, TRB));
     const uint32_t tiles128 = !TRA && !TRB && g.k % BK != 0 ? 1 : 4;  // (mma_tile.h: why k that ends inside a step is staged)
     if (!TRA && !TRB) small = !large ? tiles128 : narrow_tiles_16bit(p.m, p.n, batch, g.k, uint32_t(mc.compute_units)) ? 2 : 3;
-    variant = large || more ? 6 : tiles128;
+    variant = streams ? 6 : tiles128;
+    if constexpr (!TRA && !TRB) {
+      const uint32_t apart = batch == 1 ? rows_apart(p.m, p.n, g.k, uint64_t(p.n) * g.k, uint32_t(mc.compute_units)) : 0;
+      const uint32_t whole = p.m - apart;
+      if (variant == 6 && apart && stream_16bit(whole, p.n, 1, p.k, cus, false) && mma_stream_strides_ok(g.lda, g.ldb)) {
+        g.m = whole;
+        if (launch_mma_stream<0, 0, MATH>(g, 0, mc.compute_units, stream, err, "gemmcm") != 0) return -1;
+        GemmParams q = p;
+        q.m = apart;
+        q.a = p.a + uint64_t(whole) * g.lda, q.c = p.c + uint64_t(int64_t(whole) * p.c_sm * 2);
+        if (use_cin) q.cin = p.cin + uint64_t(int64_t(whole) * p.cin_sm * 2);
+        return launch_tiles<T, TRA, TRB>(q, use_cin, 1, 0, mc, stream, err);
+      }
+    }
   }
   const uint32_t columns = (variant & ~0x300u) == 6 ? variant >> 8 : 0;
   if ((variant & ~0x300u) == 6) {
@@ -476,8 +490,7 @@ int launch_q8_gemm_t(const Q8Params& p, const Machine& mc, hipStream_t stream, s
   Q8GemmProblem<T> g;
   g.a = p.a, g.b = mc.scratch, g.m = p.m, g.n = p.n, g.k = p.k * 2, g.lda = uint32_t(p.a_sm) * 2, g.ldb = p.k * 2;
   g.batches = 1, g.a_batch = 0, g.b_batch = 0, g.c = p.c, g.scales = p.scales;
-  const bool large = uint64_t((p.m + 255) / 256) * ((p.n + 255) / 256) * 8 >= uint64_t(mc.compute_units) * 5;  // (as for the 16-bit product)
-  if ((large || stream_pays_16bit(p.m, p.n, 1, p.k, uint32_t(mc.compute_units), true)) && mma_stream_strides_ok(g.lda, g.ldb))
+  if (stream_16bit(p.m, p.n, 1, p.k, uint32_t(mc.compute_units), true) && mma_stream_strides_ok(g.lda, g.ldb))
     return launch_mma_stream<0, 0, MATH>(g, 0, mc.compute_units, stream, err, "qmm8");
   if (staged_tiles_int8(p.m, p.n, g.k, uint32_t(mc.compute_units))) return launch_mma_tile<2, 2, 4, 4, 0, 0, false, MATH>(g, mc.compute_units, stream, err, "qmm8");
   return launch_mma_tile<2, 2, 4, 4, 0, 0, true, MATH>(g, mc.compute_units, stream, err, "qmm8");

@@ -107,11 +107,11 @@ constexpr StreamTiles mma_stream_tiles(uint32_t m, uint32_t n, uint64_t batches,
 // int8: the many-row int8 product, whose 128 x 128 tiles are loaded into LDS directly: they also stay where they are one per compute unit (1024 x
 // 256 x 4096 11.3 / 12.6, x 4096 x 64.4 / 65.2, x 8192 x 115.4 / 113.5), and with padded rows up to 256 values of k (300 x 256 x 11008 13.4 / 14.5, 513 x
 // 256 x 6656 12.4 / 12.9; 520 x 512 x 8192 20.2 / 20.1; 1030 x 256 x 4096 13.7 / 12.4).
-constexpr bool stream_pays_16bit(uint32_t m, uint32_t n, uint64_t batches, uint32_t k, uint32_t cus, bool int8) {
+constexpr bool stream_pays_16bit(uint32_t m, uint32_t n, uint64_t batches, uint32_t k, uint32_t cus, bool int8, bool k_major_b = false) {
   const uint64_t rows128 = (uint64_t(m) + 127) / 128, rows256 = (uint64_t(m) + 255) / 256, tiles128 = rows128 * ((uint64_t(n) + 127) / 128) * batches;
   if (tiles128 < cus || (tiles128 == cus && (!int8 || k <= 4096))) return false;
   if (tiles128 > 2ull * cus) return true;
-  const StreamTiles tiles = mma_stream_tiles(m, n, batches, cus);
+  const StreamTiles tiles = mma_stream_tiles(m, n, batches, cus, k_major_b);
   if (tiles.cost >= 100) return false;  // (batches of up to 128 rows: half of every tile would be padding)
   if (tiles.columns != 128 && (rows256 <= 2 || (rows256 == 3 && k < 2048))) return false;
   return !(int8 && k <= 256 && rows128 % 2 && rows256 <= 3);
@@ -129,6 +129,25 @@ constexpr bool stream_pays_float8(uint32_t m, uint32_t n, uint32_t k, uint32_t c
   const uint64_t rows128 = (uint64_t(m) + 127) / 128, tiles128 = rows128 * ((uint64_t(n) + 127) / 128);
   if (2 * tiles128 <= cus) return false;
   return !(k % 128 != 0 && k >= 4096 && tiles128 <= cus && 4 * tiles256 <= cus && rows128 % 2 == 0 && uint64_t(m) * 4 >= rows256 * 256 * 3);
+}
+
+// Whether 16-bit operands run on the stream kernel: from five eighths of a 256 x 256 tile per compute unit on (1024 x 4096 x 14336 is 224 tiles on 256
+// units, 121 us on it against 163 on 128 x 128 tiles; 168 tiles: 142 against 152; at 128 tiles the small tiles are level or ahead), or by the rule above.
+constexpr bool stream_16bit(uint32_t m, uint32_t n, uint64_t batches, uint32_t k, uint32_t cus, bool int8, bool k_major_b = false) {
+  return (uint64_t(m) + 255) / 256 * ((uint64_t(n) + 255) / 256) * batches * 8 >= uint64_t(cus) * 5 || stream_pays_16bit(m, n, batches, k, cus, int8, k_major_b);
+}
+
+// Rows past the last whole tile of 256, up to 16 of them, as a product of their own on the few-row kernels, which cost a launch and a pass over the
+// weights (about 6 us + bytes / 5 TB/s), where that is well below what whole tiles save (a round of 256 columns takes about 8 us + 1.4 us per step of
+// 128 bytes; 1.6: one round on fewer units also runs at a higher clock); how many, or 0.  us, as one / apart: 2050 x 8192 x 8192 int8 weights 325 / 235,
+// bfloat16 282 / 211, float8 140 / 112; int8 1537 x 13824 x 5120 236 / 221; not bfloat16 1537 x 13824 x 5120 226 / 222, float8 108 / 113.
+constexpr uint32_t rows_apart(uint32_t m, uint32_t n, uint32_t k_bytes, uint64_t weight_bytes, uint32_t cus) {
+  const uint32_t rest = m % 256;
+  if (m < 256 || rest == 0 || rest > 16) return 0;
+  // (in units of 10 ns)
+  const uint64_t round = 800 + 140ull * (k_bytes / 128 + (k_bytes % 128 != 0)), few = 600 + weight_bytes / 50000;
+  const uint64_t saved = (mma_stream_tiles(m, n, 1, cus).cost - mma_stream_tiles(m - rest, n, 1, cus).cost) * round / 100;
+  return saved * 10 > few * 16 ? rest : 0;
 }
 
 // ---- How many slices of K serve a product of m rows whose operands are rows of k bytes on the 128 x 128 tile kernel (mma_slices.h): from at
