@@ -4,8 +4,8 @@
 // host side crates/pyvk/csrc/linalg.cpp:227-255), behind its kernel names ("gemmcm_bf16",
 // "gemmcm_f16"), parameter block (GemmParams, strides in elements) and spec {USE_CIN, ..}.
 //   - operands whose rows are 16-byte aligned and contiguous along one of their two dims, C
-//     contiguous along n: the tile kernel of _scaled_mm (mma_tile.h: 256x256x64-value workgroup
-//     tiles, direct global-to-LDS loads, persistent grid) with V_MFMA_F32_32X32X16_{BF16,F16}
+//     contiguous along n: the stream and tile kernels of _scaled_mm (mma_stream.h: 256x256x64-value workgroup
+//     tiles, mma_tile.h: 128x128; direct global-to-LDS loads, persistent grid) with V_MFMA_F32_16X16X32_{BF16,F16}
 //     and an alpha / beta epilogue.  A contiguous along k and B along k (x @ W.t(), the Linear
 //     layout) takes k a multiple of 8; an operand contiguous along m or n (x @ W, x.t() @ y:
 //     what backward passes produce) is read through the transposing LDS load and takes m (n) a

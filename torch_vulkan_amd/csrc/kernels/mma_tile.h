@@ -1,5 +1,5 @@
 // The matrix-core tile kernel shared by aten::_scaled_mm (float8 operands) and the 16-bit
-// matrix product: a workgroup computes a BM x BN tile of A [m, k] x B [n, k]^T, both operands
+// matrix product where their outputs are few for mma_stream.h: a workgroup computes a BM x BN tile of A [m, k] x B [n, k]^T, both operands
 // rows of k contiguous BYTES (p.k counts bytes: float8 values, or 2 per 16-bit value),
 // K in steps of 128 bytes through double-buffered LDS.  What differs between the users is
 // the instruction that multiplies two 32-byte fragments (MATH) and the epilogue, which the

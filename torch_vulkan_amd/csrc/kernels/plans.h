@@ -77,11 +77,11 @@ constexpr bool staged_tiles_int8(uint32_t m, uint32_t n, uint32_t k_bytes, uint3
 }
 
 // ---- The stream kernel (mma_stream.h): columns per tile of 256 rows.  256, or 192 or 128 where they take fewer or fuller rounds of a tile per
-// compute unit.  A round costs about 100, 81 and 64 parts of the same step (4096 x 14336 x 4096 in bfloat16, full rounds: 106, 86 and 64 us each; 4096
-// x 28672 x 8192 in float8: 102, 83 and 66), and fewer columns read more bytes per product, so a tie goes to the wider tile.  us, 256 / 192 /
-// 128 (rounds): float8 1024 x 8192 x 8192 88 / 77 / 64 (1, 1, 1); 2000 x 10240 x 8192 184 / 155 / 176 (2, 2, 3); 700 x 22016 x 4096 95 / 80 /
-// 90 (2, 2, 3); 4096 x 28672 x 8192 712 / 828 / 923 (7, 10, 14); bfloat16 1537 x 13824 x 5120 252 / 218 / 235 (2, 2, 3); 1024 x 14336 x 4096 107 /
-// 149 / 121 (1, 2, 2).
+// compute unit.  A full round costs 100, 81 and 55 to 60 parts of the same step (4096 values of k, 4096 rows, three rounds / one: bfloat16 97 / 99, 78 / 79
+// and 53 / 59 us each, x @ w 101 and 59 / 65, float8 53 / 56, 42 / 45 and 29 / 34), a partly full one less than its share, since the part then holds a higher clock;
+// with 64 for the narrowest, which reads most bytes per product, a tie goes to the wider tile.  us, 256 / 192 / 128 (rounds): bfloat16 1537 x 5120 x
+// 13824 240 / 195 / 203 (2, 2, 3); 3000 x 2048 x 7000 99 / 88 / 88 (2, 2, 3); 2500 x 4096 x 5120 96 / 138 / 104 (1, 2, 2); 1024 x 4096 x 8192 87 / 71 / 58 (1, 1, 1);
+// float8 1537 x 13824 x 5120 136 / 117 / 151 (1, 1, 2); 512 x 4096 x 28672 54 / 79 / 59 (1, 2, 2).
 struct StreamTiles {
   uint32_t columns;
   uint64_t cost;

@@ -720,23 +720,21 @@ __device__ __forceinline__ uint64_t halves_offset(uint32_t m, uint32_t g, uint32
   return ((uint64_t(m >> 4) * (quads * 4) + (g >> 2)) * 64 + (g & 3) * 16 + (m & 15)) * 16;
 }
 
-// Which of `rows` rows a workgroup of qmm4m_rowquant takes.  The 16 rows of a row tile write 8 or 16 bytes of a line each; workgroup i
+// Which row workgroup i of qmm4m_rowquant takes.  The 16 rows of a row tile write 8 or 16 bytes of a line each; workgroup i
 // runs on XCD i % 8, and in that order eight L2s write parts of every line (2048 x 4096 float32 rows 18-22 us).  From 128 rows on a
 // tile's rows go to one XCD, whose L2 puts the lines together: 12.8 us.
 constexpr uint32_t kSpreadRows = 128;
-__host__ __device__ inline uint32_t quant_row(uint32_t i, uint32_t rows) {
-  return rows < kSpreadRows ? i : ((i >> 7) * 8 + (i & 7)) * 16 + (i >> 3 & 15);
-}
-inline dim3 quant_grid(uint32_t rows) { return dim3(rows < kSpreadRows ? rows : (rows + 127) / 128 * 128); }
+__device__ inline uint32_t quant_row(uint32_t i) { return ((i >> 7) * 8 + (i & 7)) * 16 + (i >> 3 & 15); }
 
 // Phase 0 for the matrix layout, one workgroup per row, from row m0 on.  FAST: k is a multiple of 8, at most
 // 2048 * kFusedGroups, rows 16-byte aligned: the row is read once, into registers.  HALVES: the values go to `dst` as
 // qmm4m_half's operand, row m0 first, and to p.q only where `keep` says that the caller reads them there.
-template <class T, bool FAST, bool HALVES>
+// SPREAD: from kSpreadRows rows on (quant_row).
+template <class T, bool FAST, bool HALVES, bool SPREAD>
 __global__ __launch_bounds__(256) void qmm4m_rowquant(Q4CParams p, uint32_t groupwise, uint32_t quads, uint64_t dst, uint32_t m0, uint32_t rows, uint32_t keep) {
   constexpr uint64_t item = sizeof(typename T::storage);
-  const uint32_t in = quant_row(blockIdx.x, rows), m = m0 + in, tid = threadIdx.x;
-  if (in >= rows) return;
+  const uint32_t in = SPREAD ? quant_row(blockIdx.x) : blockIdx.x, m = m0 + in, tid = threadIdx.x;
+  if (SPREAD && in >= rows) return;
   const uint64_t row = p.inp + uint64_t(m) * p.k * item;
   const uint32_t groups_all = quads * 16;
   RowQuant rq;
@@ -1563,6 +1561,16 @@ int launch_qmm4c_pack(const Q4PackParams& p, uint32_t layout, const Machine&, hi
 }
 
 // The matrix-layout form of the product: phase 0, 1 or 2 (= 0 then 1).
+template <class T, bool HALVES>
+void launch_rowquant(const Q4CParams& p, bool fast, uint32_t groupwise, uint32_t quads, uint64_t dst, uint32_t m0, uint32_t rows, uint32_t keep, hipStream_t stream) {
+  const bool spread = rows >= kSpreadRows;
+  const dim3 grid(spread ? (rows + 127) / 128 * 128 : rows);
+  if (fast && spread) hipLaunchKernelGGL((qmm4m_rowquant<T, true, HALVES, true>), grid, dim3(256), 0, stream, p, groupwise, quads, dst, m0, rows, keep);
+  else if (fast) hipLaunchKernelGGL((qmm4m_rowquant<T, true, HALVES, false>), grid, dim3(256), 0, stream, p, groupwise, quads, dst, m0, rows, keep);
+  else if (spread) hipLaunchKernelGGL((qmm4m_rowquant<T, false, HALVES, true>), grid, dim3(256), 0, stream, p, groupwise, quads, dst, m0, rows, keep);
+  else hipLaunchKernelGGL((qmm4m_rowquant<T, false, HALVES, false>), grid, dim3(256), 0, stream, p, groupwise, quads, dst, m0, rows, keep);
+}
+
 template <class T>
 int launch_matrix(const Q4CParams& p, uint32_t phase_and_flags, uint32_t groupwise, const Machine& mc, hipStream_t stream, std::string* err) {
   constexpr uint32_t item = sizeof(typename T::storage);
@@ -1607,8 +1615,7 @@ int launch_matrix(const Q4CParams& p, uint32_t phase_and_flags, uint32_t groupwi
       const uint64_t at = mc.workspace;
       const uint32_t threads = (rows + 15) / 16 * 16 * M.quads * 16;  // (below the workspace's bytes / 16)
       if (phase == 1) hipLaunchKernelGGL(qmm4m_expand, dim3(threads / 256), dim3(256), 0, stream, p, at, m0, rows, M.quads);
-      else if (fast) hipLaunchKernelGGL((qmm4m_rowquant<T, true, true>), quant_grid(rows), dim3(256), 0, stream, p, groupwise, M.quads, at, m0, rows, keep);
-      else hipLaunchKernelGGL((qmm4m_rowquant<T, false, true>), quant_grid(rows), dim3(256), 0, stream, p, groupwise, M.quads, at, m0, rows, keep);
+      else launch_rowquant<T, true>(p, fast, groupwise, M.quads, at, m0, rows, keep, stream);
       if (M.upb == 1 && eight) launch_half<T, 1, 2, 4>(p, M, at, m0, rows, stream);
       else if (M.upb == 1) launch_half<T, 1, 2, 2>(p, M, at, m0, rows, stream);
       else if (eight) launch_half<T, 2, 2, 4>(p, M, at, m0, rows, stream);
@@ -1617,8 +1624,7 @@ int launch_matrix(const Q4CParams& p, uint32_t phase_and_flags, uint32_t groupwi
     return 0;
   }
   if (phase == 0 || phase == 2) {
-    if (fast) hipLaunchKernelGGL((qmm4m_rowquant<T, true, false>), quant_grid(p.m), dim3(256), 0, stream, p, groupwise, M.quads, 0ull, 0u, p.m, 1u);
-    else hipLaunchKernelGGL((qmm4m_rowquant<T, false, false>), quant_grid(p.m), dim3(256), 0, stream, p, groupwise, M.quads, 0ull, 0u, p.m, 1u);
+    launch_rowquant<T, false>(p, fast, groupwise, M.quads, 0, 0, p.m, 1, stream);
   }
   if (phase == 1 || phase == 2) {
     for (uint32_t m0 = 0; rows_kernel && m0 < p.m; m0 += 16 * 1024) {
