@@ -4,7 +4,8 @@
 // 192 and 256 x 128 tiles, waves of 64 x 96 and 64 x 64: mma_stream_tiles, plans.h.)
 // Bound: the matrix cores' power.  On N(0,1) operands the part lowers its clock, and what counts is energy per multiply-add: 16 x 16 instructions (see
 // mfma_16bit, mma_tile.h) and loads spread over the step.  8192^3 in bfloat16, N(0,1) / zeros: 735 / 665 us, 834 with 32 x 32 instructions; without loads 602 /
-// 509, with loads that all hit the L2 699 / 568; float8 8192^3 400 -> 372.
+// 509, with loads that all hit the L2 699 / 568; float8 8192^3
+// 409 -> 385 (trace averages).
 // It differs from mma_tile in how a workgroup's time is laid out, after measuring where mma_tile's goes (one wave's
 // clock read at four points of every step): the matrix cores were busy 58-66 % of the cycles; the rest was the wave
 // issuing address arithmetic for its LDS-direct loads (380 cycles a step) and all eight waves starting every step
