@@ -163,6 +163,18 @@ def test_q4_rows_and_quads_that_exist(m, k, bs):
             assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (flags, fused)
 
 
+@pytest.mark.parametrize("m,n", [(288, 9120), (288, 12280)])  # 2565 and 3456 waves of 2 x 2
+def test_q4_blocks_of_128_planned(m, n):
+    """Planned 2 x 2 tiles, operands in place and copied first, against one tile per wave."""
+    import _dev
+    k = 256
+    w, sc, bvec = int4_weights(n, k, 128, bias=True)
+    x = int4_rows(m, k, torch.float32)
+    cm = _dev.CompactWeights(torch._dyn_quant_pack_4bit_weight(w, sc, bvec, 128, k, n).numpy(), 128, k, n, layout=1)
+    got, want = (_dev.q4_compact(bits(x), oracle.F32, cm, fused=True, flags=flags) for flags in (0, 32 | 64))
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 def test_q4_float16_products_on_the_fixed_workspace():
     """vkt_dispatch_static: three pieces of rows where the pool's workspace takes two."""
     import _dev

@@ -290,6 +290,14 @@ def test_narrow_tiles_where_their_rounds_are_shorter():
         assert not L.shim_narrow_tiles_16bit(m, n, 1, 2 * k, 256), (m, k, n)
 
 
+def test_4bit_rows_in_place():
+    """Blocks of 128 in 2 x 2 tiles: operands copied first only between three and four waves per SIMD."""
+    L = ctypes.CDLL(os.path.join(os.path.dirname(abi.LIB_PATH), "libvkt_hosttest.so"))
+    L.shim_q4_rows_in_place.argtypes = [ctypes.c_uint32] * 3
+    for m, n, want in [(300, 8704, 1), (300, 11008, 0), (330, 11008, 0), (900, 4096, 0), (1024, 4096, 0), (1025, 4096, 1), (370, 11008, 1), (2048, 11008, 1)]:
+        assert L.shim_q4_rows_in_place(m, (n + 15) // 16, 1024) == want, (m, n)
+
+
 def test_rows_past_the_last_tile_apart():
     """Up to 16 rows past whole tiles of 256 go to the few-row kernels where that saves a round's difference that pays for their launch."""
     L = ctypes.CDLL(os.path.join(os.path.dirname(abi.LIB_PATH), "libvkt_hosttest.so"))

@@ -45,6 +45,15 @@ constexpr Q4Form q4_rows_form(uint32_t m, uint32_t tiles, uint32_t quads, uint32
   return (upb == 8 ? int21 >= 2048 : int11 > 4096) ? kQ4Int21 : kQ4Int11;
 }
 
+// Blocks of 128 in 2 x 2 tiles: whether a wave's operands are requested into the registers they are used from (150 registers: three waves fit a
+// SIMD), or a step's are copied first (176: two).  Copied only where that takes two rounds of waves and the other one and a bit (us, copied / in
+// place, waves in brackets: 300 x 4096 x 8704 [2720] 70 / 52, x 11008 [3440] 77 / 83, 330 rows [3784] 78.5 / 85, 900 x 2048 x 4096 [3712] 41.5 / 44, 370 x
+// 4096 x 11008 [4128] 99 / 90, 400 rows [4472] 108 / 93, 300 x 8192 x 16384 [5120] 180 / 158, 800 x 4096 x 11008 [8600] 181 / 159, 2048 rows [22016] 415 / 389).
+constexpr bool q4_rows_in_place(uint32_t m, uint32_t tiles, uint32_t simds) {
+  const uint64_t waves = (uint64_t(m) + 31) / 32 * ((uint64_t(tiles) + 1) / 2);
+  return waves <= 3ull * simds || waves > 4ull * simds;
+}
+
 // ---- The tile kernel with 256 x 256 or 256 x 128 outputs per workgroup, one workgroup per compute unit: whether the narrow
 // tiles take less, where a round of them costs `cost` hundredths of a round of the wide ones.  Both are built for a k that ends inside
 // a step (of 128 bytes), the narrow ones staged through registers.

@@ -979,7 +979,7 @@ __global__ __launch_bounds__(256) void qmm4m_tile(Q4CParams p, MatrixLayout L, u
 // the last quad again), so that the loop body is straight-line code.
 constexpr int kRowsAhead = 2;
 
-template <class T, int UPB, int RT, int CT>
+template <class T, int UPB, int RT, int CT, bool IN_PLACE = UPB == 8 && RT * CT != 1>
 __global__ __launch_bounds__(256) void qmm4m_rows(Q4CParams p, MatrixLayout L, uint32_t m0) {
   constexpr uint64_t item = sizeof(typename T::storage);
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1041,13 +1041,13 @@ __global__ __launch_bounds__(256) void qmm4m_rows(Q4CParams p, MatrixLayout L, u
       if constexpr (UPB != 0) set.s[c] = ldg<F4>(sbase[c] + quad * sstep);
     }
   };
-  // Blocks of 256 with several tiles per wave: a quad's registers take the quad after next only once they are used up, and nothing moves
+  // IN_PLACE (blocks of 256 with several tiles per wave): a quad's registers take the quad after next only once they are used up, and nothing moves
   // across the requests.  Left to itself the scheduler puts these loops' loads next to their use (the chains are short, and it aims at one
   // more wave per SIMD), five waits for memory per two quads.  us, before the shared sums / with them / with them and in place: 512 x
   // 4096 x 11008 129 / 143 / 103, 512 x 8192 x 11008 246 / 269 / 200, 96 x 4096 x 28672 60 / 64 / 49, 2048 x 4096 x 11008 489 / 451 / 379.
-  // (Blocks of 128, with the shared sums / and in place: 2048 x 4096 x 11008 411 / 386, but 300 x 4096 x 11008 77 / 83, 150 rows 42.5 / 45; one scale per
-  // column 330 / 350, 1024 x 8192 x 8192 188 / 218.)
-  constexpr bool kInPlace = UPB == 8 && RT * CT > 1;
+  // (Blocks of 128 in 2 x 2 tiles: q4_rows_in_place, plans.h; 2 x 1 copied, 150 x 4096 x 11008 42.5 / 45; one scale per column copied, 2048 x 4096 x 11008 330
+  // / 350, 1024 x 8192 x 8192 188 / 218.)
+  constexpr bool kInPlace = IN_PLACE;
 #pragma unroll
   for (int i = 0; i < kRowsAhead; ++i) {
     request(sets[i], i);
@@ -1359,7 +1359,7 @@ void launch_half(const Q4CParams& p, const MatrixLayout& M, uint64_t halves, uin
 
 // (blocks of 32 and 64: one tile per wave only)
 template <class T, int RT, int CT>
-int launch_rows(const Q4CParams& p, const MatrixLayout& M, uint32_t m0, uint32_t rows, hipStream_t stream) {
+int launch_rows(const Q4CParams& p, const MatrixLayout& M, uint32_t m0, uint32_t rows, uint32_t simds, hipStream_t stream) {
   const dim3 grid((M.tiles + 4 * CT - 1) / (4 * CT), (rows + 16 * RT - 1) / (16 * RT));
   switch (M.upb) {
     case 0: hipLaunchKernelGGL((qmm4m_rows<T, 0, RT, CT>), grid, dim3(256), 0, stream, p, M, m0); break;
@@ -1371,7 +1371,10 @@ int launch_rows(const Q4CParams& p, const MatrixLayout& M, uint32_t m0, uint32_t
       if constexpr (RT * CT == 1) hipLaunchKernelGGL((qmm4m_rows<T, 2, 1, 1>), grid, dim3(256), 0, stream, p, M, m0);
       else return -1;
       break;
-    case 4: hipLaunchKernelGGL((qmm4m_rows<T, 4, RT, CT>), grid, dim3(256), 0, stream, p, M, m0); break;
+    case 4:
+      if (RT * CT == 4 && q4_rows_in_place(rows, M.tiles, simds)) hipLaunchKernelGGL((qmm4m_rows<T, 4, RT, CT, RT * CT == 4>), grid, dim3(256), 0, stream, p, M, m0);
+      else hipLaunchKernelGGL((qmm4m_rows<T, 4, RT, CT>), grid, dim3(256), 0, stream, p, M, m0);
+      break;
     case 8: hipLaunchKernelGGL((qmm4m_rows<T, 8, RT, CT>), grid, dim3(256), 0, stream, p, M, m0); break;
     default: return -1;
   }
@@ -1632,9 +1635,9 @@ int launch_matrix(const Q4CParams& p, uint32_t phase_and_flags, uint32_t groupwi
       uint32_t shape = (flags >> 6) & 3u;
       if (half_blocks) shape = 1;  // (the float16 form has more tiles per wave)
       else if (shape == 0) shape = q4_rows_form(rows, M.tiles, M.quads, M.upb, simds);
-      const int rc = shape == 3 ? launch_rows<T, 2, 2>(p, M, m0, rows, stream)
-                   : shape == 2 ? launch_rows<T, 2, 1>(p, M, m0, rows, stream)
-                                : launch_rows<T, 1, 1>(p, M, m0, rows, stream);
+      const int rc = shape == 3 ? launch_rows<T, 2, 2>(p, M, m0, rows, simds, stream)
+                   : shape == 2 ? launch_rows<T, 2, 1>(p, M, m0, rows, simds, stream)
+                                : launch_rows<T, 1, 1>(p, M, m0, rows, simds, stream);
       if (rc != 0) {
         *err = "qmm4c: bad layout";
         return -1;
